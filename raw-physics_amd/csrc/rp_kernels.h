@@ -102,9 +102,9 @@ struct DevWorld {
 // A settled pile of 10^5 bodies has about 4.9 items (body pairs) per body;
 // greedy colouring of its item conflict graph needs up to about 40 colours,
 // and 24 colours with 32 rounds left 60 000 of its 490 000 items to the
-// serial class (one lane: seconds per frame).
+// serial class (one item after another: seconds per frame).
 constexpr int BIG_COLOURS = 63;             // parallel colours (one 64-bit mask with the serial class)
-constexpr int BIG_SERIAL = BIG_COLOURS;     // class solved by one lane in item order
+constexpr int BIG_SERIAL = BIG_COLOURS;     // class solved one item after another, in item order
 constexpr int BIG_CLASSES = BIG_COLOURS + 1;
 constexpr int BIG_COLOUR_ROUNDS = 64;       // Jones-Plassmann rounds per frame (launches end at once when all are coloured)
 // Default: every class launched one by one over the device (a settled

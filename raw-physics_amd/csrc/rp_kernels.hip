@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "rp_device.h"
+#include "rp_pairsolve.h"
 
 namespace rp {
 
@@ -489,7 +490,7 @@ __global__ void __launch_bounds__(64) k_narrow_general(DevWorld w) {
 
 // Dependency levels of one frame's solve items (wave/scene). An item is one
 // external constraint or the contacts of one live pair (solved in order by
-// one lane). The reference's sequence is: external constraints, then the
+// two lanes, rp_pairsolve.h). The reference's sequence is: external constraints, then the
 // contacts of each pair in pair order (pbd.cpp:580-620). An item's level is
 // one above the last level of either of its non-fixed bodies, so items that
 // share a writable body keep their order and items of one level touch
@@ -630,7 +631,8 @@ __global__ void __launch_bounds__(64) k_solve(DevWorld w, double h, int iters, i
         for (int l = 0; l < Lmax; ++l) {
             int a = level_start(l), b = level_start(l + 1);
             int i0 = (l < L) ? a : 0, i1 = (l < L) ? b : 0;
-            for (int idx = i0 + lane; idx < i1; idx += LPS) solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
+            for (int idx = i0 + lane / 2; idx < i1; idx += LPS / 2)
+                solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
             __syncthreads();
         }
     }
@@ -641,7 +643,7 @@ __global__ void __launch_bounds__(64) k_solve(DevWorld w, double h, int iters, i
     for (int l = 0; l < Lmax; ++l) {
         int a = level_start(l), b = level_start(l + 1);
         int i0 = (l < L) ? a : 0, i1 = (l < L) ? b : 0;
-        for (int idx = i0 + lane; idx < i1; idx += LPS) solve_item_vel(w, order[idx], bodies[idx], h);
+        for (int idx = i0 + lane / 2; idx < i1; idx += LPS / 2) solve_item_vel(w, order[idx], bodies[idx], h);
         __syncthreads();
     }
     if (err && valid) atomicOr(&w.scene_err[s], err);

@@ -14,13 +14,14 @@
 //   solve         items (external constraints, live pairs) coloured once per
 //                 frame (Jones-Plassmann on the item conflict graph: items
 //                 sharing a non-fixed body), then solved colour by colour
-//                 with one lane per item (the first colours one launch each,
+//                 with two lanes per item (the first colours one launch each,
 //                 the small rest on one block). This replaces the reference's
 //                 sequential Gauss-Seidel order, so results differ from it
 //                 within a stated tolerance; they do not depend on thread
 //                 timing (colours and the serial class are deterministic, and
 //                 items of one colour touch disjoint writable bodies).
 #include "rp_device.h"
+#include "rp_pairsolve.h"
 
 namespace rp {
 
@@ -625,14 +626,15 @@ __global__ void __launch_bounds__(64) k_big_class(DevWorld w, BigScene b, double
     int i0 = ls[c], i1 = ls[c + 1];
     uint32_t err = 0;
     if (c == BIG_SERIAL) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (blockIdx.x == 0 && threadIdx.x < 2) {
             for (int idx = i0; idx < i1; ++idx) {
                 if (kVel) solve_item_vel(w, order[idx], bodies[idx], h);
                 else solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
             }
         }
     } else {
-        for (int idx = i0 + blockIdx.x * blockDim.x + threadIdx.x; idx < i1; idx += gridDim.x * blockDim.x) {
+        int step = (int)(gridDim.x * blockDim.x) / 2;
+        for (int idx = i0 + (int)(blockIdx.x * blockDim.x + threadIdx.x) / 2; idx < i1; idx += step) {
             if (kVel) solve_item_vel(w, order[idx], bodies[idx], h);
             else solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
         }
@@ -651,13 +653,13 @@ __global__ void __launch_bounds__(1024) k_big_tail(DevWorld w, BigScene b, doubl
     for (int c = c0; c < BIG_COLOURS; ++c) {
         int i0 = ls[c], i1 = ls[c + 1];
         if (i0 == i1) continue;  // the same for every thread
-        for (int idx = i0 + (int)threadIdx.x; idx < i1; idx += blockDim.x) {
+        for (int idx = i0 + (int)threadIdx.x / 2; idx < i1; idx += blockDim.x / 2) {
             if (kVel) solve_item_vel(w, order[idx], bodies[idx], h);
             else solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 2) {
         for (int idx = ls[BIG_SERIAL]; idx < ls[BIG_SERIAL + 1]; ++idx) {
             if (kVel) solve_item_vel(w, order[idx], bodies[idx], h);
             else solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
@@ -672,7 +674,7 @@ __global__ void k_big_velocity_update(DevWorld w, BigScene b, double h) {
 }
 
 void big_solve(const DevWorld& w, const BigScene& b, const FrameParams& fp, hipStream_t st) {
-    int gi = std::min(grid_for(b.item_cap, 64), 2048);
+    int gi = std::min(grid_for(2 * (int64_t)b.item_cap, 64), 2048);
     bool ext = w.n_ext > 0;
     if (ext) hipLaunchKernelGGL(k_big_ext_zero, dim3(grid_for(w.n_ext, 256)), dim3(256), 0, st, w, b);
     // classes 0..L-1 one launch each (the large ones), the rest on one block

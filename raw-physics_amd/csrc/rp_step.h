@@ -1338,7 +1338,6 @@ RP_HD int collider_contacts(const ColView& c1, const ColView& c2, ContactPt* out
 // XPBD base constraints (pbd_base_constraints.cpp:6-227)
 // ---------------------------------------------------------------------------
 template <class S> struct PosPrepT { V3T<S> r1, r2; M3T<S> I1, I2; };
-using PosPrep = PosPrepT<double>;
 
 template <class S>
 RP_HD void pos_prep(const BodyT<S>& e1, const BodyT<S>& e2, V3T<S> r1_lc, V3T<S> r2_lc, PosPrepT<S>& p) {
@@ -1382,26 +1381,6 @@ RP_HD void pos_apply(BodyT<S>& e1, BodyT<S>& e2, const PosPrepT<S>& p, S dl, V3T
     V3T<S> a2 = m3_mulv(p.I2, cross(p.r2, imp));
     // quaternion products use the rotation before either body is updated
     // (pbd_base_constraints.cpp:114-117); e1 and e2 are distinct bodies.
-    if (!e1.fixed) rot_update(e1, a1, true);
-    if (!e2.fixed) rot_update(e2, a2, false);
-}
-RP_HD double ang_dlambda(const M3& I1, const M3& I2, double h, double compliance, double lambda, V3 dq, uint32_t& err) {
-    double theta = len(dq);
-    if (theta <= 1e-50) return 0.0;
-    V3 n = v3(dq.x / theta, dq.y / theta, dq.z / theta);
-    double w1 = dot(n, m3_mulv(I1, n));
-    double w2 = dot(n, m3_mulv(I2, n));
-    if (w1 + w2 == 0.0) err |= ERR_ZERO_MASS;
-    double tc = compliance / (h * h);
-    return (-theta - tc * lambda) / (w1 + w2 + tc);
-}
-RP_HD void ang_apply(Body& e1, Body& e2, const M3& I1, const M3& I2, double dl, V3 dq) {
-    double theta = len(dq);
-    if (theta <= 1e-50) return;
-    V3 n = v3(dq.x / theta, dq.y / theta, dq.z / theta);
-    V3 imp = scl(-dl, n);
-    V3 a1 = m3_mulv(I1, imp);
-    V3 a2 = m3_mulv(I2, imp);
     if (!e1.fixed) rot_update(e1, a1, true);
     if (!e2.fixed) rot_update(e2, a2, false);
 }
@@ -1451,107 +1430,6 @@ RP_HD bool limit_angle(V3 n, V3 n1, V3 n2, double alpha, double beta, V3& dq) {
         return true;
     }
     return false;
-}
-
-// Joint and positional constraints (pbd.cpp:81-97, 156-173, 245-379).
-// lam[0..2] are the constraint's multipliers for this substep:
-//   positional: lambda; mutual orientation: lambda;
-//   hinge: aligned axes, position, limit; spherical: position, swing, twist.
-RP_HD void solve_external(const ExtC& c, double* lam, Body& e1, Body& e2, double h, uint32_t& err) {
-    bool bad = false;
-    switch (c.type) {
-    case 0: {  // POSITIONAL_CONSTRAINT
-        V3 dx = sub(sub(e1.x, e2.x), c.distance);
-        PosPrep p;
-        pos_prep(e1, e2, c.r1, c.r2, p);
-        double dl = pos_dlambda(e1, e2, p, h, c.compliance, lam[0], dx, err);
-        pos_apply(e1, e2, p, dl, dx);
-        lam[0] += dl;
-    } break;
-    case 2: {  // MUTUAL_ORIENTATION_CONSTRAINT
-        M3 I1 = world_tensor(e1.q, e1.Iinv), I2 = world_tensor(e2.q, e2.Iinv);
-        Q4 aux = q_mul(e1.q, q_inv(e2.q));
-        V3 dq = v3(2.0 * aux.x, 2.0 * aux.y, 2.0 * aux.z);
-        double dl = ang_dlambda(I1, I2, h, c.compliance, lam[0], dq, err);
-        ang_apply(e1, e2, I1, I2, dl, dq);
-        lam[0] += dl;
-    } break;
-    case 3: {  // HINGE_JOINT_CONSTRAINT
-        M3 I1 = world_tensor(e1.q, e1.Iinv), I2 = world_tensor(e2.q, e2.Iinv);
-        V3 a1 = q_axis(e1.q, c.axis[0], bad);
-        V3 a2 = q_axis(e2.q, c.axis[1], bad);
-        V3 dq = cross(a1, a2);
-        double dl = ang_dlambda(I1, I2, h, c.compliance, lam[0], dq, err);
-        ang_apply(e1, e2, I1, I2, dl, dq);
-        lam[0] += dl;
-        PosPrep p;
-        pos_prep(e1, e2, c.r1, c.r2, p);
-        V3 dx = sub(add(e1.x, p.r1), add(e2.x, p.r2));
-        dl = pos_dlambda(e1, e2, p, h, 0.0, lam[1], dx, err);
-        pos_apply(e1, e2, p, dl, dx);
-        lam[1] += dl;
-        if (c.limited) {
-            V3 n1 = q_axis(e1.q, c.axis[2], bad);
-            V3 n2 = q_axis(e2.q, c.axis[3], bad);
-            V3 n = q_axis(e1.q, c.axis[0], bad);
-            if (limit_angle(n, n1, n2, c.limits[0], c.limits[1], dq)) {
-                M3 J1 = world_tensor(e1.q, e1.Iinv), J2 = world_tensor(e2.q, e2.Iinv);
-                double d2 = ang_dlambda(J1, J2, h, 0.0, lam[2], dq, err);
-                ang_apply(e1, e2, J1, J2, d2, dq);
-                lam[2] += d2;
-            }
-        }
-    } break;
-    case 4: {  // SPHERICAL_JOINT_CONSTRAINT
-        const double EPSILON = 1e-50;
-        PosPrep p;
-        pos_prep(e1, e2, c.r1, c.r2, p);
-        V3 dx = sub(add(e1.x, p.r1), add(e2.x, p.r2));
-        double dl = pos_dlambda(e1, e2, p, h, 0.0, lam[0], dx, err);
-        pos_apply(e1, e2, p, dl, dx);
-        lam[0] += dl;
-        V3 n1 = q_axis(e1.q, c.axis[0], bad);
-        V3 n2 = q_axis(e2.q, c.axis[1], bad);
-        V3 n = cross(n1, n2);
-        double n_len = len(n);
-        if (n_len > EPSILON) {
-            n = v3(n.x / n_len, n.y / n_len, n.z / n_len);
-            V3 dq;
-            if (limit_angle(n, n1, n2, c.limits[0], c.limits[1], dq)) {
-                M3 I1 = world_tensor(e1.q, e1.Iinv), I2 = world_tensor(e2.q, e2.Iinv);
-                double d2 = ang_dlambda(I1, I2, h, 0.0, lam[1], dq, err);
-                ang_apply(e1, e2, I1, I2, d2, dq);
-                lam[1] += d2;
-            }
-        }
-        V3 a1 = q_axis(e1.q, c.axis[0], bad);
-        V3 b1 = q_axis(e1.q, c.axis[2], bad);
-        V3 a2 = q_axis(e2.q, c.axis[1], bad);
-        V3 b2 = q_axis(e2.q, c.axis[3], bad);
-        n = add(a1, a2);
-        n_len = len(n);
-        if (n_len > EPSILON) {
-            n = v3(n.x / n_len, n.y / n_len, n.z / n_len);
-            n1 = sub(b1, scl(dot(n, b1), n));
-            n2 = sub(b2, scl(dot(n, b2), n));
-            double n1_len = len(n1);
-            double n2_len = len(n2);
-            if (n1_len > EPSILON && n2_len > EPSILON) {
-                n1 = v3(n1.x / n1_len, n1.y / n1_len, n1.z / n1_len);
-                n2 = v3(n2.x / n2_len, n2.y / n2_len, n2.z / n2_len);
-                V3 dq;
-                if (limit_angle(n, n1, n2, c.limits[2], c.limits[3], dq)) {
-                    M3 I1 = world_tensor(e1.q, e1.Iinv), I2 = world_tensor(e2.q, e2.Iinv);
-                    double d3 = ang_dlambda(I1, I2, h, 0.0, lam[2], dq, err);
-                    ang_apply(e1, e2, I1, I2, d3, dq);
-                    lam[2] += d3;
-                }
-            }
-        }
-    } break;
-    default: bad = true; break;
-    }
-    if (bad) err |= ERR_SELECT;
 }
 
 // Velocity solve of one collision constraint (pbd.cpp:646-711)
