@@ -28,6 +28,7 @@ struct DevWorld {
     int stage_cap;                  // LDS vertices per pair: 2 x the largest hull
     int small_nv;                   // > 0: pairs of two hulls of <= small_nv vertices go to their own list
     int stage_small;                // LDS vertices per pair of that list: 2 x small_nv
+    int small_bodies;               // most bodies of a scene that is not large
     int solve_lanes;                // lanes per scene in the solve: 64, 32 or 16
     int big_launch_classes;         // large scenes: colour classes solved one launch each, the rest in one block
     // scenes

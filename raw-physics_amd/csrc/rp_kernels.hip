@@ -579,16 +579,34 @@ __global__ void __launch_bounds__(64) k_levels(DevWorld w, int collisions) {
 
 // Solve of one scene and substep: position Gauss-Seidel (pbd.cpp:615-620),
 // velocity update (pbd.cpp:623-643), velocity solve (pbd.cpp:646-711), level
-// by level over the frame's items. LPS lanes serve one scene, so a wave
-// solves 64/LPS scenes side by side (small scenes leave most of a 64-lane
-// wave idle otherwise).
-template <bool kExt, int LPS>
-__global__ void __launch_bounds__(64) k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next) {
-    constexpr int SPW = 64 / LPS;
-    int s = blockIdx.x * SPW + (int)threadIdx.x / LPS;
+// by level over the frame's items. LPS lanes serve one scene, two per item, so
+// a wave solves 64/LPS scenes side by side (small scenes leave most of a
+// 64-lane wave idle otherwise).
+//
+// kLds: the scenes' bodies are held in LDS (`cap` records per scene) from the
+// first level to the next substep's integration, and only poses and
+// velocities (the first STATE_VECS 16-byte words of a record) go back. A level
+// then costs its items' arithmetic and an LDS round trip instead of two
+// trips to L2. The items' codes are read two levels ahead and, without
+// joints, their first contacts one level ahead, both independent of the
+// bodies. What is left is the instructions of one item at a time (about 780
+// FP64 operations per contact in both sweeps): a call on a stack of 10 boxes
+// went from 3.07 to 2.81 ms, a scene of 16 bodies from 25 to 20 us per launch.
+constexpr int BODY_VECS = sizeof(Body) / sizeof(int4);
+constexpr int STATE_VECS = offsetof(Body, deact) / sizeof(int4);  // x, q, v, w, px, pq, pv, pw
+constexpr int SOLVE_LDS_LIMIT = 64 * 1024;
+static_assert(sizeof(Body) % sizeof(int4) == 0 && offsetof(Body, deact) % sizeof(int4) == 0, "copied as 16-byte words");
+
+template <bool kExt, int LPS, bool kLds>
+__global__ void __launch_bounds__(LPS > 64 ? LPS : 64) __attribute__((amdgpu_waves_per_eu(2)))
+k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next, int cap) {
+    extern __shared__ int4 rp_solve_lds[];
+    constexpr int SPB = LPS < 64 ? 64 / LPS : 1;  // scenes per block
+    constexpr int LPW = LPS < 64 ? LPS : 64;      // lanes of a wave that serve one scene
+    int s = blockIdx.x * SPB + (int)threadIdx.x / LPS;
     int lane = (int)threadIdx.x % LPS;
     bool valid = s < w.ns && !w.scene_big[s];  // large scenes: coloured solve (rp_large.hip)
-    int b0 = 0, n = 0, e0 = 0, e1x = 0, L = 0;
+    int b0 = 0, n = 0, e0 = 0, e1x = 0, L = 0, g0 = 0, np = 0;
     const int* order = nullptr;
     const int2* bodies = nullptr;
     const int* ls = nullptr;
@@ -602,21 +620,45 @@ __global__ void __launch_bounds__(64) k_solve(DevWorld w, double h, int iters, i
         bodies = w.item_bodies + ib;
         ls = w.item_lstart + ib + s;
         L = w.scene_nlevels[s];
+        g0 = w.live_prefix[s];
+        np = collisions ? w.live_count[s] : 0;
     }
-    int Lmax = L;  // levels of the wave's busiest scene: every lane joins every barrier
+    // whether some live pair of the scene has contacts (its pairs are
+    // contiguous in the live list): without, and without external
+    // constraints, there is nothing to sweep
+    int touching = 0;
+    for (int k = lane; k < np; k += LPS) touching |= w.ncontact[g0 + k];
+    Body* body = w.body + b0;
+    if constexpr (kLds) {
+        int4* own = rp_solve_lds + (size_t)((int)threadIdx.x / LPS) * cap * BODY_VECS;
+        const int4* src = (const int4*)body;
+        for (int i = lane; i < n * BODY_VECS; i += LPS) own[i] = src[i];
+        body = (Body*)own;
+    }
+    if constexpr (LPS > 64) {
+        touching = __syncthreads_or(touching);
+    } else {
+        unsigned long long m = __ballot(touching != 0);
+        if constexpr (LPS < 64) m &= ((1ull << LPS) - 1ull) << ((int)threadIdx.x & ~(LPS - 1));
+        touching = m != 0;
+    }
+    if (!touching && !(kExt && e1x > e0)) L = 0;
+    int Lmax = L;  // levels of the block's busiest scene: every lane joins every barrier
+    if constexpr (SPB > 1) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) Lmax = max(Lmax, __shfl_xor(Lmax, off));
-    // level starts ls[0..L] in the scene's lanes' registers (lane l holds
-    // ls[l]) when every scene of the wave fits, read back by lane exchange
-    // instead of a global load per level (the branch is uniform per wave)
-    bool ls_in_lanes = Lmax + 1 <= LPS;
-    int my_ls = (valid && lane <= L) ? ls[lane] : 0;
+        for (int off = 32; off > 0; off >>= 1) Lmax = max(Lmax, __shfl_xor(Lmax, off));
+    }
+    // level starts ls[0..L] in the lanes' registers (lane l of the wave's
+    // lanes of a scene holds ls[l]) when every scene of the block fits, read
+    // back by lane exchange instead of a global load per level (the branch is
+    // uniform per block)
+    bool ls_in_lanes = Lmax + 1 <= LPW;
+    int my_ls = (valid && lane % LPW <= L) ? ls[lane % LPW] : 0;
     auto level_start = [&](int l) -> int {
-        if (ls_in_lanes) return __shfl(my_ls, l, LPS);
-        return (l <= L) ? ls[l] : 0;
+        if (ls_in_lanes) return __shfl(my_ls, l, LPW);
+        return (valid && l <= L) ? ls[l] : 0;
     };
     uint32_t err = 0;
-    (void)collisions;
 
     // multipliers of the external constraints start at zero (pbd.cpp:426-462)
     if constexpr (kExt) {
@@ -627,44 +669,108 @@ __global__ void __launch_bounds__(64) k_solve(DevWorld w, double h, int iters, i
         }
     }
     __syncthreads();
-    for (int it = 0; it < iters; ++it) {
-        for (int l = 0; l < Lmax; ++l) {
-            int a = level_start(l), b = level_start(l + 1);
-            int i0 = (l < L) ? a : 0, i1 = (l < L) ? b : 0;
-            for (int idx = i0 + lane / 2; idx < i1; idx += LPS / 2)
-                solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
-            __syncthreads();
+    // One sweep over the levels. `here` is this pair's first item of level l
+    // with its contact, `next` that of level l + 1 (its code only).
+    auto sweep = [&](auto solve) {
+        int i0 = level_start(0), i1 = level_start(1), i2 = level_start(2);
+        PairItem here, next;
+        bool has = 0 < L && i0 + lane / 2 < i1, has_next = 1 < L && i1 + lane / 2 < i2;
+        if (has) {
+            load_item(here, order, bodies, i0 + lane / 2);
+            if (!kExt) load_item_contact<kExt>(here, w);
         }
-    }
+        if (has_next) load_item(next, order, bodies, i1 + lane / 2);
+        for (int l = 0; l < Lmax; ++l) {
+            int i3 = level_start(min(l + 3, L));
+            bool has_after = l + 2 < L && i2 + lane / 2 < i3;
+            PairItem after;
+            // (with joints the registers go to the joint solve)
+            if (!kExt && has_next) load_item_contact<kExt>(next, w);
+            if (has_after) load_item(after, order, bodies, i2 + lane / 2);
+            if (has) {
+                if (kExt) load_item_contact<kExt>(here, w);
+                for (int idx = i0 + lane / 2;;) {
+                    solve(here);
+                    idx += LPS / 2;
+                    if (idx >= i1) break;
+                    load_item(here, order, bodies, idx);
+                    load_item_contact<kExt>(here, w);
+                }
+            }
+            __syncthreads();
+            here = next;
+            next = after;
+            has = has_next;
+            has_next = has_after;
+            i0 = i1;
+            i1 = i2;
+            i2 = i3;
+        }
+    };
+    for (int it = 0; it < iters; ++it)
+        sweep([&](const PairItem& t) { solve_item_pos<kExt>(w, body, b0, t, h, err); });
     // velocity update
-    for (int i = lane; i < n; i += LPS) velocity_update_body(w.body[b0 + i], h);
+    for (int i = lane; i < n; i += LPS) velocity_update_body(body[i], h);
     __syncthreads();
     // velocity solve over the collision items, in the same levels
-    for (int l = 0; l < Lmax; ++l) {
-        int a = level_start(l), b = level_start(l + 1);
-        int i0 = (l < L) ? a : 0, i1 = (l < L) ? b : 0;
-        for (int idx = i0 + lane / 2; idx < i1; idx += LPS / 2) solve_item_vel(w, order[idx], bodies[idx], h);
-        __syncthreads();
-    }
+    sweep([&](const PairItem& t) { solve_item_vel(w, body, b0, t, h); });
     if (err && valid) atomicOr(&w.scene_err[s], err);
     // the next substep's integration of the scene's bodies (worlds without
     // large scenes), in place of a k_integrate launch
     if (integrate_next) {
-        __syncthreads();
-        for (int i = lane; i < n; i += LPS) integrate_body(w, b0 + i, h);
+        for (int i = lane; i < n; i += LPS) {
+            integrate(body[i], h);
+            w.model[b0 + i] = model_matrix(body[i].x, body[i].q);
+        }
         if (blockIdx.x == 0 && threadIdx.x == 0) w.counters[CNT_MANIFOLD] = 0;
+    }
+    if constexpr (kLds) {
+        __syncthreads();
+        int4* dst = (int4*)(w.body + b0);
+        const int4* src = (const int4*)body;
+        for (int i = lane; i < n * STATE_VECS; i += LPS) {
+            int b = i / STATE_VECS, k = i - b * STATE_VECS;
+            dst[b * BODY_VECS + k] = src[b * BODY_VECS + k];
+        }
     }
 }
 
+// LDS bytes of the solve's body records per block, or 0 to leave them in
+// global memory: the records may not cost the launch waves that the
+// registers (two waves per SIMD, eight per CU) would allow it to hold.
+static size_t solve_lds_bytes(const DevWorld& w, int lanes, int blocks) {
+    int scenes = std::max(1, 64 / lanes), waves = std::max(1, lanes / 64);
+    size_t bytes = (size_t)scenes * w.small_bodies * sizeof(Body);
+    if (bytes == 0 || bytes > (size_t)SOLVE_LDS_LIMIT) return 0;
+    size_t per_cu = std::min<size_t>(8 / waves, 160 * 1024 / bytes);
+    return per_cu * waves == 8 || (size_t)blocks <= 256 * per_cu ? bytes : 0;
+}
+
+template <bool kExt, int LPS>
+static void launch_solve_lanes(const DevWorld& w, const FrameParams& fp, hipStream_t st, int integrate_next) {
+    constexpr int SPB = LPS < 64 ? 64 / LPS : 1;
+    dim3 grid((w.ns + SPB - 1) / SPB), block(LPS > 64 ? LPS : 64);
+    int it = (int)fp.iters, co = fp.collisions ? 1 : 0;
+    size_t lds = solve_lds_bytes(w, LPS, (int)grid.x);
+    if (lds > 0)
+        hipLaunchKernelGGL((k_solve<kExt, LPS, true>), grid, block, lds, st, w, fp.h, it, co, integrate_next,
+                           w.small_bodies);
+    else
+        hipLaunchKernelGGL((k_solve<kExt, LPS, false>), grid, block, 0, st, w, fp.h, it, co, integrate_next, 0);
+}
+// Whole waves per scene (solve_lanes 64): scenes of more than 64 bodies have
+// levels of more items than one wave's 32 pairs of lanes, and take four waves
+// (scenes of 4 to 256 bodies, ms per frame at 64 / 128 / 256 lanes: 150
+// scenes 8.40 / 8.03 / 7.81, 600 scenes 9.94 / 9.56 / 9.46).
 template <bool kExt>
 static void launch_solve(const DevWorld& w, const FrameParams& fp, hipStream_t st, int integrate_next) {
-    int spw = 64 / w.solve_lanes;
-    dim3 grid((w.ns + spw - 1) / spw);
-    int it = (int)fp.iters, co = fp.collisions ? 1 : 0;
     switch (w.solve_lanes) {
-    case 16: hipLaunchKernelGGL((k_solve<kExt, 16>), grid, dim3(64), 0, st, w, fp.h, it, co, integrate_next); break;
-    case 32: hipLaunchKernelGGL((k_solve<kExt, 32>), grid, dim3(64), 0, st, w, fp.h, it, co, integrate_next); break;
-    default: hipLaunchKernelGGL((k_solve<kExt, 64>), grid, dim3(64), 0, st, w, fp.h, it, co, integrate_next); break;
+    case 16: launch_solve_lanes<kExt, 16>(w, fp, st, integrate_next); break;
+    case 32: launch_solve_lanes<kExt, 32>(w, fp, st, integrate_next); break;
+    default:
+        if (w.small_bodies > 64) launch_solve_lanes<kExt, 256>(w, fp, st, integrate_next);
+        else launch_solve_lanes<kExt, 64>(w, fp, st, integrate_next);
+        break;
     }
 }
 

@@ -628,15 +628,13 @@ __global__ void __launch_bounds__(64) k_big_class(DevWorld w, BigScene b, double
     if (c == BIG_SERIAL) {
         if (blockIdx.x == 0 && threadIdx.x < 2) {
             for (int idx = i0; idx < i1; ++idx) {
-                if (kVel) solve_item_vel(w, order[idx], bodies[idx], h);
-                else solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
+                solve_item_at<kExt, kVel>(w, order, bodies, idx, h, err);
             }
         }
     } else {
         int step = (int)(gridDim.x * blockDim.x) / 2;
         for (int idx = i0 + (int)(blockIdx.x * blockDim.x + threadIdx.x) / 2; idx < i1; idx += step) {
-            if (kVel) solve_item_vel(w, order[idx], bodies[idx], h);
-            else solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
+            solve_item_at<kExt, kVel>(w, order, bodies, idx, h, err);
         }
     }
     if (err) atomicOr(&w.scene_err[b.s], err);
@@ -654,15 +652,13 @@ __global__ void __launch_bounds__(1024) k_big_tail(DevWorld w, BigScene b, doubl
         int i0 = ls[c], i1 = ls[c + 1];
         if (i0 == i1) continue;  // the same for every thread
         for (int idx = i0 + (int)threadIdx.x / 2; idx < i1; idx += blockDim.x / 2) {
-            if (kVel) solve_item_vel(w, order[idx], bodies[idx], h);
-            else solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
+            solve_item_at<kExt, kVel>(w, order, bodies, idx, h, err);
         }
         __syncthreads();
     }
     if (threadIdx.x < 2) {
         for (int idx = ls[BIG_SERIAL]; idx < ls[BIG_SERIAL + 1]; ++idx) {
-            if (kVel) solve_item_vel(w, order[idx], bodies[idx], h);
-            else solve_item_pos<kExt>(w, order[idx], bodies[idx], h, err);
+            solve_item_at<kExt, kVel>(w, order, bodies, idx, h, err);
         }
     }
     if (err) atomicOr(&w.scene_err[b.s], err);

@@ -73,28 +73,6 @@ __device__ __forceinline__ void half_apply(HalfPos& e, V3 r, const M3& I, double
 }
 __device__ __forceinline__ double abs_mass(const HalfPos& e) { return second_lane() ? -e.im : e.im; }
 
-// One positional correction dx between the bodies' points at r, with the
-// world inverse inertia I (pos_dlambda, pos_apply); returns delta lambda.
-__device__ __forceinline__ double pair_position(HalfPos& e, V3 r, const M3& I, double h, double compliance, double lambda,
-                                                V3 dx, uint32_t& err) {
-    double c = len(dx);
-    if (c <= 1e-50) return 0.0;
-    V3 n = v3(dx.x / c, dx.y / c, dx.z / c);
-    double dl = pair_dlambda(half_mass(abs_mass(e), r, I, n), c, compliance / (h * h), lambda, err);
-    half_apply(e, r, I, dl, n);
-    return dl;
-}
-// One angular correction dq (ang_dlambda, ang_apply).
-__device__ __forceinline__ double pair_angular(HalfPos& e, const M3& I, double h, double compliance, double lambda, V3 dq,
-                                               uint32_t& err) {
-    double theta = len(dq);
-    if (theta <= 1e-50) return 0.0;
-    V3 n = v3(dq.x / theta, dq.y / theta, dq.z / theta);
-    double dl = pair_dlambda(dot(n, m3_mulv(I, n)), theta, compliance / (h * h), lambda, err);
-    half_rotate(e, m3_mulv(I, scl(-dl, n)));
-    return dl;
-}
-
 // collision_constraint_solve (pbd.cpp:107-154). `I` is the world inverse
 // inertia at e.q when `fresh`: it is computed once per change of the rotation
 // (the second preparation's value serves the item's next contact unless
@@ -140,78 +118,84 @@ __device__ __forceinline__ void pair_collision(V3 r_lc, V3 n, double& lambda_n, 
 // lam[0..2] are the constraint's multipliers for this substep:
 //   positional: lambda; mutual orientation: lambda;
 //   hinge: aligned axes, position, limit; spherical: position, swing, twist.
+// Every constraint is up to three corrections in a row, each positional (dx
+// between the bodies' points at r: pos_dlambda, pos_apply) or angular (dq:
+// ang_dlambda, ang_apply), so one copy of that code runs in a loop: written
+// out per constraint type it is 130 KB of instructions, which do not fit the
+// instruction cache, and a lone wave that misses it waits for every line.
 __device__ __forceinline__ void pair_external(const ExtC& c, double* lam, HalfPos& e, double h, uint32_t& err) {
     const double EPSILON = 1e-50;
     bool bad = false;
     const bool second = second_lane();
-    double l0 = lam[0], l1 = lam[1], l2 = lam[2];
-    V3 r_lc = second ? c.r2 : c.r1;
-    int ax_a = second ? c.axis[1] : c.axis[0], ax_b = second ? c.axis[3] : c.axis[2];
-    switch (c.type) {
-    case 0: {  // POSITIONAL_CONSTRAINT
-        V3 dx = sub(sub(pair_first(e.x), pair_second(e.x)), c.distance);
-        l0 += pair_position(e, q_rot(e.q, r_lc), world_tensor(e.q, e.Iinv), h, c.compliance, l0, dx, err);
-    } break;
-    case 2: {  // MUTUAL_ORIENTATION_CONSTRAINT
-        Q4 q1 = {pair_first(e.q.x), pair_first(e.q.y), pair_first(e.q.z), pair_first(e.q.w)};
-        Q4 q2 = {pair_second(e.q.x), pair_second(e.q.y), pair_second(e.q.z), pair_second(e.q.w)};
-        Q4 aux = q_mul(q1, q_inv(q2));
-        V3 dq = v3(2.0 * aux.x, 2.0 * aux.y, 2.0 * aux.z);
-        l0 += pair_angular(e, world_tensor(e.q, e.Iinv), h, c.compliance, l0, dq, err);
-    } break;
-    case 3: {  // HINGE_JOINT_CONSTRAINT
-        V3 a = q_axis(e.q, ax_a, bad);
-        V3 dq = cross(pair_first(a), pair_second(a));
-        l0 += pair_angular(e, world_tensor(e.q, e.Iinv), h, c.compliance, l0, dq, err);
-        V3 r = q_rot(e.q, r_lc);
-        V3 p = add(e.x, r);
-        V3 dx = sub(pair_first(p), pair_second(p));
-        l1 += pair_position(e, r, world_tensor(e.q, e.Iinv), h, 0.0, l1, dx, err);
-        if (c.limited) {
-            V3 m = q_axis(e.q, ax_b, bad);
-            V3 n = pair_first(q_axis(e.q, ax_a, bad));
-            if (limit_angle(n, pair_first(m), pair_second(m), c.limits[0], c.limits[1], dq))
-                l2 += pair_angular(e, world_tensor(e.q, e.Iinv), h, 0.0, l2, dq, err);
-        }
-    } break;
-    case 4: {  // SPHERICAL_JOINT_CONSTRAINT
-        V3 r = q_rot(e.q, r_lc);
-        V3 p = add(e.x, r);
-        V3 dx = sub(pair_first(p), pair_second(p));
-        l0 += pair_position(e, r, world_tensor(e.q, e.Iinv), h, 0.0, l0, dx, err);
-        V3 a = q_axis(e.q, ax_a, bad);
-        V3 n1 = pair_first(a), n2 = pair_second(a);
-        V3 n = cross(n1, n2);
-        double n_len = len(n);
-        V3 dq;
-        if (n_len > EPSILON) {
-            n = v3(n.x / n_len, n.y / n_len, n.z / n_len);
-            if (limit_angle(n, n1, n2, c.limits[0], c.limits[1], dq))
-                l1 += pair_angular(e, world_tensor(e.q, e.Iinv), h, 0.0, l1, dq, err);
-        }
-        a = q_axis(e.q, ax_a, bad);
-        V3 b = q_axis(e.q, ax_b, bad);
-        n = add(pair_first(a), pair_second(a));
-        n_len = len(n);
-        if (n_len > EPSILON) {
-            n = v3(n.x / n_len, n.y / n_len, n.z / n_len);
-            b = sub(b, scl(dot(n, b), n));
-            double b_len = len(b);
-            if (pair_first(b_len) > EPSILON && pair_second(b_len) > EPSILON) {
-                b = v3(b.x / b_len, b.y / b_len, b.z / b_len);
-                if (limit_angle(n, pair_first(b), pair_second(b), c.limits[2], c.limits[3], dq))
-                    l2 += pair_angular(e, world_tensor(e.q, e.Iinv), h, 0.0, l2, dq, err);
+    const V3 r_lc = second ? c.r2 : c.r1;
+    const int ax_a = second ? c.axis[1] : c.axis[0], ax_b = second ? c.axis[3] : c.axis[2];
+    const bool hinge = c.type == 3, spherical = c.type == 4;
+    if (c.type < 0 || c.type == 1 || c.type > 4) bad = true;
+    const int steps = bad ? 0 : spherical || (hinge && c.limited) ? 3 : hinge ? 2 : 1;
+    for (int step = 0; step < steps; ++step) {
+        const bool angular = hinge ? step != 1 : spherical ? step != 0 : c.type == 2;
+        const double compliance = step == 0 && !spherical ? c.compliance : 0.0;
+        bool apply = true;
+        V3 d, r = v3(0.0, 0.0, 0.0);
+        if (!angular) {
+            r = q_rot(e.q, r_lc);
+            V3 p = c.type == 0 ? e.x : add(e.x, r);
+            d = sub(pair_first(p), pair_second(p));
+            if (c.type == 0) d = sub(d, c.distance);  // POSITIONAL_CONSTRAINT
+        } else if (c.type == 2) {                      // MUTUAL_ORIENTATION_CONSTRAINT
+            Q4 q1 = {pair_first(e.q.x), pair_first(e.q.y), pair_first(e.q.z), pair_first(e.q.w)};
+            Q4 q2 = {pair_second(e.q.x), pair_second(e.q.y), pair_second(e.q.z), pair_second(e.q.w)};
+            Q4 aux = q_mul(q1, q_inv(q2));
+            d = v3(2.0 * aux.x, 2.0 * aux.y, 2.0 * aux.z);
+        } else {
+            V3 a = q_axis(e.q, ax_a, bad);
+            V3 a1 = pair_first(a), a2 = pair_second(a);
+            if (step == 0) {
+                d = cross(a1, a2);  // hinge: the aligned axes
+            } else {
+                // hinge limit: limit axes about the first body's hinge axis;
+                // swing: swing axes about their normal; twist: twist axes
+                // about the mean swing axis, with their parts along it removed
+                const bool swing = spherical && step == 1, twist = spherical && step == 2;
+                V3 n = a1, m = a;
+                if (!swing) m = q_axis(e.q, ax_b, bad);
+                if (spherical) {
+                    n = swing ? cross(a1, a2) : add(a1, a2);
+                    double n_len = len(n);
+                    apply = n_len > EPSILON;
+                    n = v3(n.x / n_len, n.y / n_len, n.z / n_len);
+                }
+                if (twist) {
+                    m = sub(m, scl(dot(n, m), n));
+                    double m_len = len(m);
+                    apply = apply & (pair_first(m_len) > EPSILON) & (pair_second(m_len) > EPSILON);
+                    m = v3(m.x / m_len, m.y / m_len, m.z / m_len);
+                }
+                int lim = twist ? 2 : 0;
+                V3 m1 = pair_first(m), m2 = pair_second(m);
+                apply = apply && limit_angle(n, m1, m2, c.limits[lim], c.limits[lim + 1], d);
             }
         }
-    } break;
-    default: bad = true; break;
+        if (!apply) continue;
+        double lambda = lam[step];
+        double dl = 0.0;
+        M3 I = world_tensor(e.q, e.Iinv);
+        double size = len(d);
+        if (!(size <= 1e-50)) {
+            V3 n = v3(d.x / size, d.y / size, d.z / size);
+            V3 u = cross(r, n);
+            u = v3(angular ? n.x : u.x, angular ? n.y : u.y, angular ? n.z : u.z);
+            double wu = dot(u, m3_mulv(I, u));
+            double w = angular ? wu : abs_mass(e) + wu;
+            dl = pair_dlambda(w, size, compliance / (h * h), lambda, err);
+            V3 imp = scl(angular ? -dl : dl, n);
+            if (!angular && !e.fixed) e.x = add(e.x, scl(e.im, imp));
+            V3 t = cross(r, imp);
+            half_rotate(e, m3_mulv(I, v3(angular ? imp.x : t.x, angular ? imp.y : t.y, angular ? imp.z : t.z)));
+        }
+        if (!second) lam[step] = lambda + dl;
     }
     if (bad) err |= ERR_SELECT;
-    if (!second) {
-        lam[0] = l0;
-        lam[1] = l1;
-        lam[2] = l2;
-    }
 }
 
 // Velocity solve of one collision constraint (pbd.cpp:646-711); I is the
@@ -256,71 +240,98 @@ __device__ __forceinline__ HalfContact load_half(const Contact& c) {
     return k;
 }
 
-// One solve item: an external constraint (item < 0, index ~item) or the
-// contacts of live pair `item` in order (pbd.cpp:381-406, 615-620), on
-// bodies bb (item_body_pair). Both lanes of a pair call it with the same
-// item. A contact is loaded while the one before it is solved.
+// One solve item on its pair of lanes: an external constraint (code < 0,
+// index ~code) or the contacts of live pair `code`, its two global bodies,
+// and the first contact, loaded ahead of the solve.
+struct PairItem {
+    int code;
+    int2 bb;
+    int nc;
+    HalfContact k;
+};
+__device__ __forceinline__ void load_item(PairItem& t, const int* order, const int2* bodies, int idx) {
+    t.code = order[idx];
+    t.bb = bodies[idx];
+}
+// The contact count and the first contact of a live pair (its slots are
+// always allocated, so both loads are issued together and what an empty
+// pair's slot holds is not used).
 template <bool kExt>
-__device__ __forceinline__ void solve_item_pos(const DevWorld& w, int item, int2 bb, double h, uint32_t& err) {
+__device__ __forceinline__ void load_item_contact(PairItem& t, const DevWorld& w) {
+    t.nc = 0;
+    if (kExt && t.code < 0) return;
+    t.nc = w.ncontact[t.code];
+    t.k = load_half(w.contacts[(size_t)t.code * MAXC]);
+}
+
+// Position solve of item t (pbd.cpp:381-406, 615-620) on the bodies at `body`
+// (indexed by global body less b0). Both lanes of a pair call it with the
+// same item. A contact is loaded while the one before it is solved.
+template <bool kExt>
+__device__ __forceinline__ void solve_item_pos(const DevWorld& w, Body* body, int b0, const PairItem& t, double h,
+                                               uint32_t& err) {
     const bool second = second_lane();
-    Body& g = w.body[second ? bb.y : bb.x];
-    int nc = 0;
-    const Contact* cs = nullptr;
-    if (!kExt || item >= 0) {
-        nc = w.ncontact[item];
-        cs = w.contacts + (size_t)item * MAXC;
-        if (nc == 0) return;
-    }
+    if (!(kExt && t.code < 0) && t.nc == 0) return;
+    Body& g = body[(second ? t.bb.y : t.bb.x) - b0];
     HalfPos e;
     e.x = g.x; e.q = g.q; e.px = g.px; e.pq = g.pq;
     e.im = second ? -g.inv_mass : g.inv_mass;
     e.Iinv = g.Iinv;
     e.mu_s = g.mu_s;
     e.fixed = g.fixed;
-    if (kExt && item < 0) {
-        pair_external(w.ext[~item], w.ext_lambda + 3 * (~item), e, h, err);
+    if (kExt && t.code < 0) {
+        pair_external(w.ext[~t.code], w.ext_lambda + 3 * (~t.code), e, h, err);
     } else {
-        HalfContact k = load_half(cs[0]);
+        HalfContact k = t.k;
+        Contact* cs = w.contacts + (size_t)t.code * MAXC;
         const double mu_s = (e.mu_s + pair_other(e.mu_s)) / 2.0f;
         M3 I;
         bool fresh = false;
-        for (int c = 0; c < nc; ++c) {
-            HalfContact next = load_half(cs[min(c + 1, nc - 1)]);
+        for (int c = 0; c < t.nc; ++c) {
+            HalfContact next = load_half(cs[min(c + 1, t.nc - 1)]);
             pair_collision(k.r, k.n, k.lambda_n, k.lambda_t, e, I, fresh, mu_s, h, err);
-            Contact& o = w.contacts[(size_t)item * MAXC + c];
-            *(second ? &o.lambda_t : &o.lambda_n) = second ? k.lambda_t : k.lambda_n;
+            *(second ? &cs[c].lambda_t : &cs[c].lambda_n) = second ? k.lambda_t : k.lambda_n;
             k = next;
         }
     }
     // an external constraint on one body twice keeps its second half, as a
     // write of the first body followed by one of the second does
-    if (!e.fixed && (second || bb.x != bb.y)) { g.x = e.x; g.q = e.q; }
+    if (!e.fixed && (second || t.bb.x != t.bb.y)) { g.x = e.x; g.q = e.q; }
 }
 
-// Velocity solve of the contacts of one item (pbd.cpp:646-711); external
-// constraints take no part.
-__device__ __forceinline__ void solve_item_vel(const DevWorld& w, int item, int2 bb, double h) {
-    if (item < 0) return;
-    int nc = w.ncontact[item];
-    if (nc == 0) return;
-    Body& g = w.body[second_lane() ? bb.y : bb.x];
+// Velocity solve of item t's contacts (pbd.cpp:646-711); external constraints
+// take no part.
+__device__ __forceinline__ void solve_item_vel(const DevWorld& w, Body* body, int b0, const PairItem& t, double h) {
+    if (t.nc == 0) return;
+    Body& g = body[(second_lane() ? t.bb.y : t.bb.x) - b0];
     HalfVel e;
     e.q = g.q; e.v = g.v; e.w = g.w; e.pv = g.pv; e.pw = g.pw;
     e.im = g.inv_mass;
     e.Iinv = g.Iinv;
     e.mu_d = g.mu_d; e.e = g.e;
     e.fixed = g.fixed;
-    const Contact* cs = w.contacts + (size_t)item * MAXC;
-    HalfContact k = load_half(cs[0]);
+    const Contact* cs = w.contacts + (size_t)t.code * MAXC;
+    HalfContact k = t.k;
     const double mu_d = (e.mu_d + pair_other(e.mu_d)) / 2.0f;
     const double rest = e.e * pair_other(e.e);
     const M3 I = world_tensor(e.q, e.Iinv);
-    for (int c = 0; c < nc; ++c) {
-        HalfContact next = load_half(cs[min(c + 1, nc - 1)]);
+    for (int c = 0; c < t.nc; ++c) {
+        HalfContact next = load_half(cs[min(c + 1, t.nc - 1)]);
         pair_velocity(k.r, k.n, k.lambda_n, e, I, mu_d, rest, h);
         k = next;
     }
     if (!e.fixed) { g.v = e.v; g.w = e.w; }
+}
+
+// One item of a class or list in global memory, bodies in global memory.
+template <bool kExt, bool kVel>
+__device__ __forceinline__ void solve_item_at(const DevWorld& w, const int* order, const int2* bodies, int idx, double h,
+                                              uint32_t& err) {
+    PairItem t;
+    load_item(t, order, bodies, idx);
+    load_item_contact<true>(t, w);
+    if (kVel) solve_item_vel(w, w.body, 0, t, h);
+    else solve_item_pos<kExt>(w, w.body, 0, t, h, err);
 }
 
 }  // namespace rp

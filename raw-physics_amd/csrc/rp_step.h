@@ -14,7 +14,7 @@ namespace rp {
 // ---------------------------------------------------------------------------
 // Device data layout
 // ---------------------------------------------------------------------------
-template <class S> struct BodyT {   // one record per body (464 bytes for S = double)
+template <class S> struct alignas(16) BodyT {  // one record per body (464 bytes for S = double, copied as 16-byte words)
     V3T<S> x; Q4T<S> q; V3T<S> v; V3T<S> w;      // world_position, world_rotation, velocities
     V3T<S> px; Q4T<S> pq; V3T<S> pv; V3T<S> pw;  // previous_* (entity.h:43-46)
     S deact;                                     // deactivation_time

@@ -458,7 +458,9 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
         int64_t scene_pairs = n * (n - 1) / 2;
         // (at least 65 bodies: the class starts of the coloured solve need
         // more item slots than a tiny scene has)
-        if (n > std::max<int64_t>(hw.large_scene_bodies, 64)) {
+        if (n <= std::max<int64_t>(hw.large_scene_bodies, 64)) {
+            d.small_bodies = std::max(d.small_bodies, (int)n);
+        } else {
             BigScene bs;
             memset(&bs, 0, sizeof(bs));
             bs.s = s;
@@ -544,7 +546,12 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
     d.manifold_group = d.narrow_group > 1 ? 0 : 1;
     d.manifold_blocks = narrow_blocks_for(d, 1, pcap);
     if (!im.ensure_group_work()) return false;
-    d.solve_lanes = few ? 32 : 64;
+    // lanes per scene in the solve: whole waves while the scenes do not fill
+    // the device's SIMDs, then as many scenes per wave as keep the waves
+    // within what it holds (16-body scenes, ms per frame at 64 / 32 / 16
+    // lanes: 64 scenes 1.54 / 1.56 / 1.77, 2048 scenes 2.68 / 2.52 / 2.76,
+    // 4096 scenes 4.17 / 3.89 / 4.22, 8192 scenes 6.81 / 6.23 / 6.15)
+    d.solve_lanes = d.ns < 1536 || d.small_bodies > 64 ? 64 : d.ns < 8192 ? 32 : 16;
     d.big_launch_classes = BIG_LAUNCH_CLASSES;
 
     bool ok = true;
