@@ -307,16 +307,21 @@ uint32_t rp_world_model_matrices(rp_world* w, void* out, int32_t as_float, int32
 /* Mass (1/m, inertia and its inverse as at creation), static and dynamic
  * friction of every non-fixed body; NULL arrays are left unchanged. */
 uint32_t rp_world_set_body_params(rp_world* w, const double* mass, const double* mu_s, const double* mu_d);
-/* Steps `frames` frames (collisions on) from the current state, keeping a
- * device checkpoint of every frame's start state. */
+/* Steps `frames` frames (collisions on) from the current state, recording
+ * every substep's start state and contacts on the device. */
 uint32_t rp_world_adjoint_forward(rp_world* w, double dt, uint32_t frames, uint32_t num_substeps,
                                   uint32_t num_pos_iters, double gravity);
 /* dl_dstate [nb][13]: dL/d(x, q(x,y,z,w), v, w) of the state at the end of the
  * recorded run. Out: grad_state [nb][13] (the same at its start) and
  * grad_param [nb][3] (dL/d mass, static friction, dynamic friction). The
- * world is left at the end state. Each frame is recomputed from its
- * checkpoint, then its substeps are reversed. */
+ * world is left at the end state. */
 uint32_t rp_world_adjoint_backward(rp_world* w, const double* dl_dstate, double* grad_state, double* grad_param);
+/* Most device memory (bytes, 0: the default 16 GiB) the record of a run may
+ * take, from the next rp_world_adjoint_forward on; never more than half of
+ * what is free, and at least one frame. A run whose record is larger is
+ * recorded in segments of whole frames: the backward pass steps each segment
+ * but the last again from a checkpoint. Identical results. Returns 0. */
+uint32_t rp_world_set_adjoint_memory(rp_world* w, uint64_t bytes);
 /* Substeps whose recomputation in the backward pass did not reproduce the
  * recorded forward state bit for bit (0 when the backward pass is exact). */
 uint64_t rp_world_adjoint_mismatches(rp_world* w);

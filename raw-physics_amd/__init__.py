@@ -62,6 +62,7 @@ def library():
         "rp_world_set_body_params": (u32, [_P, _P, _P, _P]),
         "rp_world_adjoint_forward": (u32, [_P, f64, u32, u32, u32, f64]),
         "rp_world_adjoint_backward": (u32, [_P, _P, _P, _P]),
+        "rp_world_set_adjoint_memory": (u32, [_P, u64]),
         "rp_world_adjoint_mismatches": (u64, [_P]),
         "rp_world_adjoint_amplification": (u32, [_P, _P]),
         "rp_world_set_narrow_group": (i32, [_P, i32]),
@@ -181,8 +182,13 @@ class World:
         return int(self.lib.rp_world_set_body_params(self.h, *ptrs))
 
     def adjoint_forward(self, frames: int, dt=1.0 / 60.0, substeps=20, iters=1, gravity=10.0) -> int:
-        """Steps `frames` frames keeping per-frame checkpoints for adjoint_backward."""
+        """Steps `frames` frames, recorded for adjoint_backward."""
         return int(self.lib.rp_world_adjoint_forward(self.h, dt, frames, substeps, iters, gravity))
+
+    def set_adjoint_memory(self, num_bytes: int):
+        """Most device memory of a run's record (0: the default); longer runs
+        are recorded in segments, with identical results."""
+        self.lib.rp_world_set_adjoint_memory(self.h, num_bytes)
 
     def adjoint_backward(self, dl_dstate: np.ndarray):
         """dl_dstate (nb, 13): dL/d(x, q, v, w) at the end of the recorded run.

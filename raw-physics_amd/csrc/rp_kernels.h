@@ -92,6 +92,7 @@ struct DevWorld {
     int32_t* body_last;             // [nb]          last level per body (large scenes)
     int32_t *uf_parent, *uf_flag;   // [nb]
     const int32_t* scene_big;       // [ns] 1: large scene (grid broad phase, coloured solve)
+    double* rec_state;              // [nb][REC_STATE] where an integration records its start states, or null
     // diagnostics
     uint32_t* scene_err;            // [ns]
     unsigned long long* stats;      // [STAT_COUNT]
@@ -138,14 +139,30 @@ struct BigScene {
     int32_t* scan_blocks;        // [scan block sums]
 };
 
-// Substep records of one frame for the adjoint's recomputation: body
-// states at the start of each substep and the contacts the narrow phase made
-// (the frozen contact set).
+// What the kernels of one recorded frame write beside their own results, for
+// the adjoint: each substep's contacts and contact counts (the narrow phase
+// and the solve work on them in place) and the bodies' states at its start.
+constexpr int REC_STATE = 14;  // x, q, v, w, and whether the body is active
 struct Recorder {
-    Body* body;          // [substeps][nb]
-    int32_t* ncontact;   // [substeps][pair capacity]
-    Contact* contacts;   // [substeps][pair capacity * MAXC]
+    double* state;       // [substeps][nb][REC_STATE]
+    int32_t* ncontact;   // [substeps][pair_cap]
+    Contact* contacts;   // [substeps][pair_cap][MAXC]
     int64_t pair_cap;
+    int64_t p0;          // first live-pair slot of the view
+    int nb;              // bodies of the whole world
+};
+// A recorded run (or its last frames): the frozen contact set and the states.
+struct AdjContact { V3 r1, r2, n; };
+struct AdjRecord {
+    int ns, nb, steps;            // steps: recorded substeps
+    int64_t pair_cap;
+    const double* state;          // [steps][nb][REC_STATE]
+    const int32_t* ncontact;      // [steps][pair_cap]
+    const AdjContact* contacts;   // [steps][pair_cap][MAXC]
+    const int2* pair;             // [frames][pair_cap] bodies of the live pairs
+    const int32_t *g0, *np;       // [frames][ns] first live pair and count of each scene
+    const Body* next_state;       // [nb] after the last recorded substep
+    const Body* end_state;        // [nb] at the end of the run (fixed bodies, constants)
 };
 
 struct FrameParams {
@@ -154,6 +171,7 @@ struct FrameParams {
     bool collisions = true;
     bool forces_given = false;  // body F/T already hold the frame's force sums
     bool keep_pose = false;     // record every body's pose after the last substep's integration
+    bool record = false;        // record contacts and states for the adjoint
 };
 
 // Kernel classes timed by the profiling mode.
@@ -188,13 +206,19 @@ struct KernelTimer {
 
 hipError_t launch_frame(const DevWorld& w, const FrameParams& fp, hipStream_t st, KernelTimer* kt = nullptr,
                         const BigScene* bigs = nullptr, int nbig = 0, const Recorder* rec = nullptr);
-// Adjoint of one recorded frame for scenes with one dynamic body
+// Adjoint of a recorded run for scenes with one dynamic body
 // (rp_adjoint.hip): abar [nb][13] is the adjoint of (x, q, v, w) at the end
-// of the frame on entry and at its start on exit; gparam [nb][3] accumulates
+// of the record on entry and at its start on exit; gparam [nb][3] accumulates
 // d/d(mass, static friction, dynamic friction); amax [nb] keeps the largest
-// |abar| component of each dynamic body seen at a frame start.
-hipError_t launch_adjoint_frame(const DevWorld& w, const Recorder& rec, const int32_t* scene_dyn, const Body* end_state,
-                                double* abar, double* gparam, double* amax, const FrameParams& fp, hipStream_t st);
+// |abar| component of each dynamic body seen at a frame start. `jac` holds
+// the Jacobians of `chunk` substeps (adjoint_jacobian_bytes).
+int adjoint_steps_per_chunk(int ns, size_t bytes);
+size_t adjoint_jacobian_bytes(int ns, int steps);
+hipError_t launch_adjoint(const AdjRecord& r, const int32_t* scene_dyn, int chunk, double* jac, double* abar,
+                          double* gparam, double* amax, unsigned long long* stats, uint32_t* scene_err,
+                          const FrameParams& fp, hipStream_t st);
+hipError_t launch_adjoint_pack(const DevWorld& w, const Recorder& st, const AdjRecord& r, int f, int s0, int64_t p0,
+                               int substeps, bool all, hipStream_t s);
 // Large-scene stages (rp_large.hip), in frame order.
 void big_broad(const DevWorld& w, const BigScene& b, hipStream_t st);
 void big_islands(const DevWorld& w, const BigScene& b, double dt, hipStream_t st);

@@ -184,16 +184,18 @@ __global__ void k_scatter_live(DevWorld w) {
 }
 
 // ---------------------------------------------------------------------------
-// Integration of body b (pbd.cpp:565-596) and its model matrix.
-__device__ __forceinline__ void integrate_body(const DevWorld& w, int b, double h) {
-    Body e = w.body[b];
+// Integration of body b (pbd.cpp:565-596), held at e, and its model matrix;
+// in a recorded frame the state it starts from is kept.
+__device__ __forceinline__ void integrate_body(const DevWorld& w, int b, Body& e, double h) {
+    if (w.rec_state && !e.fixed) {
+        double* r = w.rec_state + (size_t)b * REC_STATE;
+        r[0] = e.x.x; r[1] = e.x.y; r[2] = e.x.z;
+        r[3] = e.q.x; r[4] = e.q.y; r[5] = e.q.z; r[6] = e.q.w;
+        r[7] = e.v.x; r[8] = e.v.y; r[9] = e.v.z;
+        r[10] = e.w.x; r[11] = e.w.y; r[12] = e.w.z;
+        r[13] = e.active ? 1.0 : 0.0;
+    }
     integrate(e, h);
-    w.body[b].x = e.x;
-    w.body[b].q = e.q;
-    w.body[b].v = e.v;
-    w.body[b].w = e.w;
-    w.body[b].px = e.px;
-    w.body[b].pq = e.pq;
     w.model[b] = model_matrix(e.x, e.q);
 }
 
@@ -201,7 +203,15 @@ __global__ void k_integrate(DevWorld w, double h) {
     int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b == 0) w.counters[CNT_MANIFOLD] = 0;  // the substep's manifold queue starts empty
     if (b >= w.nb) return;
-    integrate_body(w, b + w.body_base, h);
+    b += w.body_base;
+    Body e = w.body[b];
+    integrate_body(w, b, e, h);
+    w.body[b].x = e.x;
+    w.body[b].q = e.q;
+    w.body[b].v = e.v;
+    w.body[b].w = e.w;
+    w.body[b].px = e.px;
+    w.body[b].pq = e.pq;
 }
 
 // The pose every body has when the substep's collision pass reads it
@@ -718,10 +728,7 @@ k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next, int
     // the next substep's integration of the scene's bodies (worlds without
     // large scenes), in place of a k_integrate launch
     if (integrate_next) {
-        for (int i = lane; i < n; i += LPS) {
-            integrate(body[i], h);
-            w.model[b0 + i] = model_matrix(body[i].x, body[i].q);
-        }
+        for (int i = lane; i < n; i += LPS) integrate_body(w, b0 + i, body[i], h);
         if (blockIdx.x == 0 && threadIdx.x == 0) w.counters[CNT_MANIFOLD] = 0;
     }
     if constexpr (kLds) {
@@ -822,25 +829,10 @@ __global__ void k_fp64_selftest(const double* a, const double* b, double* out, i
 // ---------------------------------------------------------------------------
 static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
-// Recording for the adjoint: body states at the start of substep k, and the
-// substep's contacts after the narrow phase.
-__global__ void k_rec_bodies(DevWorld w, Recorder r, int k) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < w.nb) r.body[(size_t)k * w.nb + b] = w.body[b];
-}
-__global__ void k_rec_contacts(DevWorld w, Recorder r, int k) {
-    int total = w.live_prefix[w.ns];
-    for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < total; g += gridDim.x * blockDim.x) {
-        int nc = w.ncontact[g];
-        r.ncontact[(size_t)k * r.pair_cap + g] = nc;
-        for (int c = 0; c < nc; ++c)
-            r.contacts[((size_t)k * r.pair_cap + g) * MAXC + c] = w.contacts[(size_t)g * MAXC + c];
-    }
-}
-
-hipError_t launch_frame(const DevWorld& w, const FrameParams& fp, hipStream_t st, KernelTimer* kt,
+hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_t st, KernelTimer* kt,
                         const BigScene* bigs, int nbig, const Recorder* rec) {
-    if (w.nb == 0) return hipSuccess;
+    if (world.nb == 0) return hipSuccess;
+    DevWorld w = world;
     KernelTimer none;
     KernelTimer& t = kt ? *kt : none;
     t.begin(KC_FRAME, st);
@@ -855,11 +847,19 @@ hipError_t launch_frame(const DevWorld& w, const FrameParams& fp, hipStream_t st
     hipLaunchKernelGGL(k_levels, dim3(w.ns), dim3(64), 0, st, w, fp.collisions ? 1 : 0);
     for (int k = 0; k < nbig; ++k) big_colour(w, bigs[k], fp.collisions, st);
     t.end(st);
-    // without large scenes or recording, the solve kernel integrates its
-    // scenes' bodies for the next substep
-    bool fuse_integrate = nbig == 0 && !rec;
+    // without large scenes, the solve kernel integrates its scenes' bodies for
+    // the next substep
+    bool fuse_integrate = nbig == 0;
+    // a recorded frame keeps each substep's contacts and start states in its
+    // slice of the record: the kernels work in place, nothing is copied
+    auto record_state = [&](unsigned sub) { return rec->state + (size_t)sub * rec->nb * REC_STATE; };
     for (unsigned sub = 0; sub < fp.substeps; ++sub) {
-        if (rec) hipLaunchKernelGGL(k_rec_bodies, dim3(cdiv(w.nb, 256)), dim3(256), 0, st, w, *rec, (int)sub);
+        if (rec) {
+            size_t slot = (size_t)sub * rec->pair_cap + rec->p0;
+            w.contacts = rec->contacts + slot * MAXC;
+            w.ncontact = rec->ncontact + slot;
+            w.rec_state = record_state(sub);
+        }
         if (sub == 0 || !fuse_integrate) {
             t.begin(KC_INTEGRATE, st);
             hipLaunchKernelGGL(k_integrate, dim3(cdiv(w.nb, 128)), dim3(128), 0, st, w, fp.h);
@@ -920,10 +920,10 @@ hipError_t launch_frame(const DevWorld& w, const FrameParams& fp, hipStream_t st
                 }
                 t.end(st);
             }
-            if (rec) hipLaunchKernelGGL(k_rec_contacts, dim3(256), dim3(256), 0, st, w, *rec, (int)sub);
         }
         t.begin(KC_SOLVE, st);
         int next = fuse_integrate && sub + 1 < fp.substeps ? 1 : 0;
+        if (rec && next) w.rec_state = record_state(sub + 1);
         if (w.n_ext > 0) launch_solve<true>(w, fp, st, next);
         else launch_solve<false>(w, fp, st, next);
         for (int k = 0; k < nbig; ++k) big_solve(w, bigs[k], fp, st);

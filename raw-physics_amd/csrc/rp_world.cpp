@@ -779,6 +779,8 @@ struct rp_world {
     int want_views = 0;  // 0 = automatic
     int nviews = 0;
     DevWorld view[kMaxViews];
+    int view_s0[kMaxViews] = {};      // first scene and first live-pair slot of each view
+    int64_t view_p0[kMaxViews] = {};
     std::vector<BigScene> view_big[kMaxViews];
     hipStream_t view_stream[kMaxViews] = {};
     hipGraphExec_t view_exec[kMaxViews] = {};
@@ -787,29 +789,55 @@ struct rp_world {
     uint64_t sched_gen = 1, graph_gen = 0;  // schedule changes invalidate the captured graphs
     // bounded queue: at most two chunks of frames in flight on each stream
     hipEvent_t chunk_done[2][kMaxViews] = {};
-    // differentiable runs: per-frame body checkpoints of the last recorded
-    // forward pass and the buffers of the backward sweep
-    Body* ckpt = nullptr;
-    uint32_t ck_frames = 0;
+    // differentiable runs (adjoint_forward / adjoint_backward): the record of
+    // the last run, kept from run to run and grown as needed
+    uint32_t ck_frames = 0;                 // frames of the recorded run, 0: none
     FrameParams ck_fp;
+    uint32_t seg_frames = 0;                // frames one record holds: the run is recorded in segments
+    Body* ckpt = nullptr;                   // [segments + 1][nb] bodies at each segment's start and at the end
     int32_t* scene_dyn = nullptr;
-    Recorder rec = {nullptr, nullptr, nullptr, 0};
+    Recorder stage = {};                    // the frame being recorded
+    AdjRecord rec = {};                     // the segment's record
+    double* jac = nullptr;
+    int jac_steps = 0;                      // substeps whose Jacobians `jac` holds
+    int rec_seg = -1;                       // segment held by `rec`
+    size_t adj_record_bytes = 0;            // most bytes of a record, 0: the default
     double* abar = nullptr;
     double* gparam = nullptr;
     double* amax = nullptr;                 // [nb] largest state adjoint at a frame start
+    std::map<void**, size_t> adj_bytes;     // sizes of the buffers above
     std::vector<double> dl_norm;            // [nb] largest |dL/dstate| component at the run's end
     bool last_collisions = true;  // of the last frame run (its solve items include live pairs)
     int device = -1;              // HIP device the world was created on
 };
 
+// A buffer of the adjoint, grown to `bytes` (its contents are not kept). A
+// moved buffer invalidates the captured graphs, which hold its address.
+template <class T>
+static bool adjoint_grow(rp_world* w, T*& p, size_t bytes) {
+    size_t& have = w->adj_bytes[(void**)&p];
+    if (p && have >= bytes) return true;
+    (void)hipStreamSynchronize(w->stream);
+    if (p) (void)hipFree((void*)p);
+    p = nullptr;
+    have = 0;
+    ++w->sched_gen;
+    void* q = nullptr;
+    if (hipMalloc(&q, std::max<size_t>(bytes, 16)) != hipSuccess) {
+        set_msg("adjoint: device allocation failed");
+        return false;
+    }
+    p = (T*)q;
+    have = bytes;
+    return true;
+}
+
 static void adjoint_free(rp_world* w) {
-    void* ps[] = {w->ckpt, w->scene_dyn, w->rec.body, w->rec.ncontact, w->rec.contacts, w->abar, w->gparam, w->amax};
-    for (void* p : ps)
-        if (p) (void)hipFree(p);
-    w->ckpt = nullptr;
-    w->scene_dyn = nullptr;
-    w->rec = {nullptr, nullptr, nullptr, 0};
-    w->abar = w->gparam = w->amax = nullptr;
+    for (auto& [p, bytes] : w->adj_bytes) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
+    w->adj_bytes.clear();
     w->ck_frames = 0;
 }
 
@@ -818,7 +846,8 @@ constexpr uint32_t kFramesPerChunk = 32;
 
 static bool same_params(const FrameParams& a, const FrameParams& b) {
     return a.dt == b.dt && a.h == b.h && a.gravity == b.gravity && a.substeps == b.substeps && a.iters == b.iters &&
-           a.collisions == b.collisions && a.forces_given == b.forces_given && a.keep_pose == b.keep_pose;
+           a.collisions == b.collisions && a.forces_given == b.forces_given && a.keep_pose == b.keep_pose &&
+           a.record == b.record;
 }
 
 // Every world launches on one process-wide stream. The runtime keeps, per
@@ -860,6 +889,8 @@ static bool build_views(rp_world* w) {
     }
     if (K == 1) {
         w->view[0] = d;
+        w->view_s0[0] = 0;
+        w->view_p0[0] = 0;
         w->view_big[0] = im.big;
         w->nviews = 1;
         return true;
@@ -897,6 +928,8 @@ static bool build_views(rp_world* w) {
                                      std::max(1, d.manifold_blocks / K));
         v.group_work = nullptr;
         w->view[k] = v;
+        w->view_s0[k] = s0;
+        w->view_p0[k] = P0;
         w->view_big[k].clear();
         for (const BigScene& bs : im.big)
             if (bs.s >= s0 && bs.s < s1) {
@@ -939,7 +972,10 @@ static hipError_t frame_graph(rp_world* w, const FrameParams& fp) {
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
         if (e != hipSuccess) return e;
-        hipError_t le = launch_frame(w->view[k], fp, st, nullptr, w->view_big[k].data(), (int)w->view_big[k].size());
+        Recorder rec = w->stage;
+        rec.p0 = w->view_p0[k];
+        hipError_t le = launch_frame(w->view[k], fp, st, nullptr, w->view_big[k].data(), (int)w->view_big[k].size(),
+                                     fp.record ? &rec : nullptr);
         e = hipStreamEndCapture(st, &g);
         if (le != hipSuccess) e = le;
         if (e == hipSuccess) e = hipGraphInstantiate(&w->view_exec[k], g, nullptr, nullptr, 0);
@@ -1034,7 +1070,8 @@ static uint32_t world_run(rp_world* w, const FrameParams& fp, uint32_t frames, b
     }
     for (uint32_t f = 0; f < frames; ++f) {
         w->timer.used = 0;
-        hipError_t e = launch_frame(w->im.d, fp, w->stream, &w->timer, w->im.big.data(), (int)w->im.big.size());
+        hipError_t e = launch_frame(w->im.d, fp, w->stream, &w->timer, w->im.big.data(), (int)w->im.big.size(),
+                                    fp.record ? &w->stage : nullptr);
         if (e == hipSuccess && !w->timer.on) e = chunk_mark(w, f, 0, w->stream);
         if (e != hipSuccess) {
             set_msg(std::string("kernel launch: ") + hipGetErrorString(e));
@@ -1386,9 +1423,83 @@ uint32_t rp_world_set_body_params(rp_world* w, const double* mass, const double*
     return err;
 }
 
+// Device memory the record of a differentiable run may take; a longer run is
+// recorded in segments of whole frames, and the backward pass steps each
+// earlier segment again from its checkpoint before reversing it. The
+// Jacobians of a part of the record at a time take JAC_BYTES.
+static const size_t kAdjRecordBytes = (size_t)16 << 30;
+static const size_t kAdjJacBytes = (size_t)512 << 20;
+
+static bool adjoint_prepare(rp_world* w, const FrameParams& fp, uint32_t frames, const std::vector<int32_t>& dyn) {
+    const DevWorld& d = w->im.d;
+    size_t nb = (size_t)d.nb, ns = (size_t)d.ns, P = (size_t)std::max<int64_t>(1, w->im.pair_capacity);
+    size_t per_step = nb * REC_STATE * sizeof(double) + P * (sizeof(int32_t) + MAXC * sizeof(AdjContact));
+    size_t per_frame = fp.substeps * per_step + P * sizeof(int2) + 2 * ns * sizeof(int32_t);
+    size_t limit = w->adj_record_bytes ? w->adj_record_bytes : kAdjRecordBytes, avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) == hipSuccess) {
+        for (const auto& b : w->adj_bytes) avail += b.second;
+        limit = std::min(limit, avail / 2);
+    }
+    w->seg_frames = (uint32_t)std::max<size_t>(1, std::min<size_t>(frames, limit / per_frame));
+    size_t F = w->seg_frames, steps = F * fp.substeps, segs = (frames + F - 1) / F;
+    w->jac_steps = (int)std::min<size_t>(steps, adjoint_steps_per_chunk(d.ns, kAdjJacBytes));
+    w->rec_seg = -1;
+    bool ok = adjoint_grow(w, w->ckpt, (segs + 1) * nb * sizeof(Body)) &&
+              adjoint_grow(w, w->scene_dyn, ns * sizeof(int32_t)) &&
+              adjoint_grow(w, w->stage.state, fp.substeps * nb * REC_STATE * sizeof(double)) &&
+              adjoint_grow(w, w->stage.ncontact, fp.substeps * P * sizeof(int32_t)) &&
+              adjoint_grow(w, w->stage.contacts, fp.substeps * P * MAXC * sizeof(Contact)) &&
+              adjoint_grow(w, w->rec.state, steps * nb * REC_STATE * sizeof(double)) &&
+              adjoint_grow(w, w->rec.ncontact, steps * P * sizeof(int32_t)) &&
+              adjoint_grow(w, w->rec.contacts, steps * P * MAXC * sizeof(AdjContact)) &&
+              adjoint_grow(w, w->rec.pair, F * P * sizeof(int2)) &&
+              adjoint_grow(w, w->rec.g0, F * ns * sizeof(int32_t)) &&
+              adjoint_grow(w, w->rec.np, F * ns * sizeof(int32_t)) &&
+              adjoint_grow(w, w->jac, adjoint_jacobian_bytes(d.ns, w->jac_steps)) &&
+              adjoint_grow(w, w->abar, nb * 13 * sizeof(double)) && adjoint_grow(w, w->gparam, nb * 3 * sizeof(double)) &&
+              adjoint_grow(w, w->amax, nb * sizeof(double));
+    if (!ok) {
+        adjoint_free(w);
+        return false;
+    }
+    w->stage.pair_cap = w->rec.pair_cap = (int64_t)P;
+    w->stage.p0 = 0;
+    w->stage.nb = w->rec.nb = d.nb;
+    w->rec.ns = d.ns;
+    if (!dyn.empty() && hipMemcpy(w->scene_dyn, dyn.data(), dyn.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
+        set_msg("adjoint_forward: copy failed");
+        return false;
+    }
+    return true;
+}
+
+// Steps the `n` frames of segment k and records them, from the current state
+// (kept as the segment's checkpoint) or, again, from the checkpoint.
+static uint32_t adjoint_record(rp_world* w, const FrameParams& fp, int k, uint32_t n, bool first) {
+    const DevWorld& d = w->im.d;
+    size_t bytes = (size_t)d.nb * sizeof(Body);
+    Body* ck = w->ckpt + (size_t)k * d.nb;
+    hipError_t e = hipMemcpyAsync(first ? ck : d.body, first ? d.body : ck, bytes, hipMemcpyDeviceToDevice, w->stream);
+    for (uint32_t f = 0; f < n && e == hipSuccess; ++f) {
+        uint32_t err = world_run(w, fp, 1, false);
+        if (err) return err;
+        bool views = w->use_graphs && !w->timer.on;  // else one launch over the whole world
+        for (int v = 0; e == hipSuccess && v < (views ? w->nviews : 1); ++v)
+            e = launch_adjoint_pack(views ? w->view[v] : d, w->stage, w->rec, (int)f, views ? w->view_s0[v] : 0,
+                                    views ? w->view_p0[v] : 0, (int)fp.substeps, v == 0, w->stream);
+    }
+    if (e != hipSuccess) {
+        set_msg(std::string("adjoint: ") + hipGetErrorString(e));
+        return RP_ERR_RUNTIME;
+    }
+    w->rec_seg = k;
+    return 0;
+}
+
 uint32_t rp_world_adjoint_forward(rp_world* w, double dt, uint32_t frames, uint32_t substeps, uint32_t iters,
                                   double gravity) {
-    adjoint_free(w);
+    w->ck_frames = 0;
+    w->dl_norm.clear();
     if (dt <= 0.0 || substeps == 0 || frames == 0) {
         set_msg("adjoint_forward: dt, substeps and frames must be positive");
         return RP_ERR_SELECT;
@@ -1407,14 +1518,6 @@ uint32_t rp_world_adjoint_forward(rp_world* w, double dt, uint32_t frames, uint3
             return RP_ERR_ADJOINT_SCOPE;
         }
     }
-    size_t nb = (size_t)d.nb;
-    if (hipMalloc(&w->ckpt, (frames + 1) * nb * sizeof(Body)) != hipSuccess ||
-        hipMalloc(&w->scene_dyn, std::max<size_t>(1, dyn.size()) * 4) != hipSuccess ||
-        hipMemcpy(w->scene_dyn, dyn.data(), dyn.size() * 4, hipMemcpyHostToDevice) != hipSuccess) {
-        set_msg("adjoint_forward: device allocation failed");
-        adjoint_free(w);
-        return RP_ERR_RUNTIME;
-    }
     FrameParams fp;
     fp.dt = dt;
     fp.h = dt / substeps;
@@ -1422,14 +1525,14 @@ uint32_t rp_world_adjoint_forward(rp_world* w, double dt, uint32_t frames, uint3
     fp.substeps = substeps;
     fp.iters = iters;
     fp.collisions = true;
-    for (uint32_t f = 0; f < frames; ++f) {
-        if (hipMemcpyAsync(w->ckpt + f * nb, d.body, nb * sizeof(Body), hipMemcpyDeviceToDevice, w->stream) !=
-            hipSuccess)
-            return RP_ERR_RUNTIME;
-        uint32_t e = world_run(w, fp, 1, false);
-        if (e) return e;
-    }
-    if (hipMemcpyAsync(w->ckpt + frames * nb, d.body, nb * sizeof(Body), hipMemcpyDeviceToDevice, w->stream) !=
+    fp.record = true;
+    if (!adjoint_prepare(w, fp, frames, dyn)) return RP_ERR_RUNTIME;
+    uint32_t e = 0;
+    for (uint32_t f = 0; f < frames && !e; f += w->seg_frames)
+        e = adjoint_record(w, fp, f / w->seg_frames, std::min(w->seg_frames, frames - f), true);
+    if (e) return e;
+    size_t nb = (size_t)d.nb, segs = (frames + w->seg_frames - 1) / w->seg_frames;
+    if (hipMemcpyAsync(w->ckpt + segs * nb, d.body, nb * sizeof(Body), hipMemcpyDeviceToDevice, w->stream) !=
             hipSuccess ||
         hipStreamSynchronize(w->stream) != hipSuccess)
         return RP_ERR_RUNTIME;
@@ -1446,18 +1549,6 @@ uint32_t rp_world_adjoint_backward(rp_world* w, const double* dl_dstate, double*
     const DevWorld& d = w->im.d;
     size_t nb = (size_t)d.nb;
     const FrameParams& fp = w->ck_fp;
-    if (!w->rec.body) {
-        w->rec.pair_cap = std::max<int64_t>(1, w->im.pair_capacity);
-        if (hipMalloc(&w->rec.body, fp.substeps * nb * sizeof(Body)) != hipSuccess ||
-            hipMalloc(&w->rec.ncontact, fp.substeps * w->rec.pair_cap * sizeof(int32_t)) != hipSuccess ||
-            hipMalloc(&w->rec.contacts, fp.substeps * w->rec.pair_cap * MAXC * sizeof(Contact)) != hipSuccess ||
-            hipMalloc(&w->abar, nb * 13 * sizeof(double)) != hipSuccess ||
-            hipMalloc(&w->gparam, nb * 3 * sizeof(double)) != hipSuccess ||
-            hipMalloc(&w->amax, nb * sizeof(double)) != hipSuccess) {
-            set_msg("adjoint_backward: device allocation failed");
-            return RP_ERR_RUNTIME;
-        }
-    }
     w->dl_norm.assign(nb, 0.0);
     for (size_t i = 0; i < nb; ++i)
         for (int j = 0; j < 13; ++j) w->dl_norm[i] = std::max(w->dl_norm[i], std::fabs(dl_dstate[13 * i + j]));
@@ -1465,26 +1556,38 @@ uint32_t rp_world_adjoint_backward(rp_world* w, const double* dl_dstate, double*
         hipMemcpy(w->amax, w->dl_norm.data(), nb * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(w->gparam, 0, nb * 3 * sizeof(double)) != hipSuccess)
         return RP_ERR_RUNTIME;
-    for (int f = (int)w->ck_frames - 1; f >= 0; --f) {
-        hipError_t e = hipMemcpyAsync(d.body, w->ckpt + f * nb, nb * sizeof(Body), hipMemcpyDeviceToDevice, w->stream);
-        if (e == hipSuccess)
-            e = launch_frame(d, fp, w->stream, nullptr, w->im.big.data(), (int)w->im.big.size(), &w->rec);
-        if (e == hipSuccess)
-            e = launch_adjoint_frame(d, w->rec, w->scene_dyn, w->ckpt + (f + 1) * nb, w->abar, w->gparam, w->amax, fp,
-                                     w->stream);
+    int segs = (int)((w->ck_frames + w->seg_frames - 1) / w->seg_frames);
+    for (int k = segs - 1; k >= 0; --k) {
+        uint32_t n = std::min(w->seg_frames, w->ck_frames - (uint32_t)k * w->seg_frames);
+        // the record holds the segment recorded last
+        if (w->rec_seg != k) {
+            uint32_t err = adjoint_record(w, fp, k, n, false);
+            if (err) return err;
+        }
+        AdjRecord r = w->rec;
+        r.steps = (int)(n * fp.substeps);
+        r.next_state = w->ckpt + (size_t)(k + 1) * nb;
+        r.end_state = w->ckpt + (size_t)segs * nb;
+        hipError_t e = launch_adjoint(r, w->scene_dyn, w->jac_steps, w->jac, w->abar, w->gparam, w->amax, d.stats,
+                                      d.scene_err, fp, w->stream);
         if (e != hipSuccess) {
             set_msg(std::string("adjoint_backward: ") + hipGetErrorString(e));
             return RP_ERR_RUNTIME;
         }
     }
     // the world continues from the end of the recorded run
-    if (hipMemcpyAsync(d.body, w->ckpt + w->ck_frames * nb, nb * sizeof(Body), hipMemcpyDeviceToDevice, w->stream) !=
+    if (hipMemcpyAsync(d.body, w->ckpt + (size_t)segs * nb, nb * sizeof(Body), hipMemcpyDeviceToDevice, w->stream) !=
             hipSuccess ||
         hipStreamSynchronize(w->stream) != hipSuccess)
         return RP_ERR_RUNTIME;
     if ((grad_state && hipMemcpy(grad_state, w->abar, nb * 13 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) ||
         (grad_param && hipMemcpy(grad_param, w->gparam, nb * 3 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess))
         return RP_ERR_RUNTIME;
+    return 0;
+}
+
+uint32_t rp_world_set_adjoint_memory(rp_world* w, uint64_t bytes) {
+    w->adj_record_bytes = (size_t)bytes;
     return 0;
 }
 
