@@ -44,11 +44,9 @@ struct DevWorld {
     const int32_t* body_hull;       // [nb]
     const int32_t* body_tv_off;     // [nb]
     // hull instances (vertices scaled, local frame)
-    const int32_t *hull_nv, *hull_nf, *hull_v_off, *hull_fn_off, *hull_topo;
+    const int32_t *hull_nv, *hull_v_off;
     const V3* hull_v;
-    const V3* hull_fn;
-    const int32_t* topo_base;       // 8 offsets into topo_pool per topology
-    const int32_t* topo_pool;
+    HullTables hulls;               // topology records, face normals, model matrices
     // transformed geometry
     V3* tv;
     const int4* xf;                 // [n_xf] (body, hull instance, vertex, tv slot)

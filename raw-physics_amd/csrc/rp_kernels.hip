@@ -257,25 +257,10 @@ __global__ void k_transform(DevWorld w, int all) {
 // View of hull instance `hid` of body b whose transformed vertices start at tv_off.
 __device__ __forceinline__ HullView hull_view_of(const DevWorld& w, int b, int hid, int tv_off) {
     HullView hv;
-    int tp = w.hull_topo[hid];
-    const int32_t* tb = w.topo_base + 8 * tp;
     hv.tv = w.tv + tv_off;
-    hv.fn = w.hull_fn + w.hull_fn_off[hid];
-    const M4& M = w.model[b];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) hv.R.m[i][j] = M.m[i][j];
     hv.nv = w.hull_nv[hid];
-    hv.nf = w.hull_nf[hid];
-    hv.fe_off = w.topo_pool + tb[0];
-    hv.fe = w.topo_pool + tb[1];
-    hv.vf_off = w.topo_pool + tb[2];
-    hv.vf = w.topo_pool + tb[3];
-    hv.vn_off = w.topo_pool + tb[4];
-    hv.vn = w.topo_pool + tb[5];
-    hv.ff_off = w.topo_pool + tb[6];
-    hv.ff = w.topo_pool + tb[7];
+    hv.hid = hid;
+    hv.body = b;
     return hv;
 }
 // The hull of a body with one hull collider (the fast narrow path).
@@ -331,9 +316,10 @@ __device__ __forceinline__ void pair_views(const DevWorld& w, int g, V3* st, int
     int4 r = w.live_rec[g];  // bodies and hull instances: no pair-slot and scene-offset loads first
     b1 = r.x;
     b2 = r.y;
-    h1 = hull_view_of(w, b1, r.z, w.body_tv_off[b1]);
-    h2 = hull_view_of(w, b2, r.w, w.body_tv_off[b2]);
-    if constexpr (G > 1) {
+    if constexpr (G == 1) {
+        h1 = hull_view_of(w, b1, r.z, w.body_tv_off[b1]);
+        h2 = hull_view_of(w, b2, r.w, w.body_tv_off[b2]);
+    } else {
         // vertex offsets and counts from the pair's record: the vertex loads
         // depend on that one load only
         int4 hv = w.live_hull[g];
@@ -360,9 +346,22 @@ __device__ __forceinline__ void pair_views(const DevWorld& w, int g, V3* st, int
             }
         }
         group_lds_sync();
-        h1.tv = st;
-        h2.tv = st + nv1;
+        h1 = HullView{st, nv1, r.z, b1};
+        h2 = HullView{st + nv1, nv2, r.w, b2};
     }
+}
+
+// The contact manifold of live pair g with EPA normal n: its contacts become
+// collision constraints as they are made. Returns their count.
+template <int G>
+__device__ __forceinline__ int pair_manifold(const DevWorld& w, int g, const HullView& h1, const HullView& h2, V3 n,
+                                             uint32_t& err, char* work, V3* spare, int spare_n) {
+    const Body& e1 = w.body[h1.body];
+    const Body& e2 = w.body[h2.body];
+    Contact* out = w.contacts + (size_t)g * MAXC;
+    auto emit = [&](int k, const ContactPt& c) { contact_to_constraint(e1, e2, c, out[k]); };
+    if constexpr (G == 1) return manifold_lane(w.hulls, h1, h2, n, emit, err);
+    else return manifold_group<G>(w.hulls, h1, h2, n, emit, err, work, spare, spare_n);
 }
 
 // kManifold: the contact manifold of a converged pair is built here too, on
@@ -394,19 +393,11 @@ __device__ __forceinline__ void gjk_epa_pairs(DevWorld& w, const int32_t* list, 
         bool hit = gjk<G>(h1, h2, sx, err, cycled);
         if (hit) r = epa<G>(h1, h2, sx, n, pen, err, work);
         if constexpr (kManifold) {
-            ContactPt local[G == 1 ? MAXC : 1];
-            ContactPt* cts = G == 1 ? local : (ContactPt*)(work + CLIP_BYTES);
             int nc = 0;
             if (r == 1) {
                 int used = h1.nv + h2.nv;  // the rest of the pair's LDS slice is free
-                nc = manifold<G>(h1, h2, n, cts, err, work, st + used, G > 1 ? stage - used : 0);
+                nc = pair_manifold<G>(w, g, h1, h2, n, err, work, st + used, stage - used);
             }
-            // one contact per lane (the group's count is uniform)
-            if constexpr (G > 1) group_lds_sync();
-            const Body& e1 = w.body[b1];
-            const Body& e2 = w.body[b2];
-            Contact* out = w.contacts + (size_t)g * MAXC;
-            for (int c = gl; c < nc; c += G) contact_to_constraint(e1, e2, cts[c], out[c]);
             if (gl == 0) w.ncontact[g] = nc;
         }
         if (gl == 0) {
@@ -439,11 +430,11 @@ __global__ void __launch_bounds__(64) k_gjk_epa_lane(DevWorld w) {
 }
 
 template <int G>
-__global__ void __launch_bounds__(64) k_manifold(DevWorld w) {
+__global__ void __launch_bounds__(64) k_manifold(DevWorld w, int stage) {
     extern __shared__ V3 rp_stage[];
     constexpr int NG = 64 / G;
     int grp = threadIdx.x / G, gl = threadIdx.x & (G - 1);
-    V3* st = rp_stage + grp * w.stage_cap;
+    V3* st = rp_stage + grp * stage;
     int total = w.counters[CNT_MANIFOLD];
     for (int k = blockIdx.x * NG + grp; k < total; k += gridDim.x * NG) {
         int g = w.mlist[k];
@@ -452,15 +443,8 @@ __global__ void __launch_bounds__(64) k_manifold(DevWorld w) {
         pair_views<G>(w, g, st, gl, s, b1, b2, h1, h2);
         uint32_t err = 0;
         char* work = G > 1 ? w.group_work + (size_t)(blockIdx.x * NG + grp) * GROUP_WORK_BYTES : nullptr;
-        ContactPt local[G == 1 ? MAXC : 1];
-        ContactPt* cts = G == 1 ? local : (ContactPt*)(work + CLIP_BYTES);
         int used = h1.nv + h2.nv;
-        int nc = manifold<G>(h1, h2, w.pair_normal[g], cts, err, work, st + used, G > 1 ? w.stage_cap - used : 0);
-        if constexpr (G > 1) group_lds_sync();
-        const Body& e1 = w.body[b1];
-        const Body& e2 = w.body[b2];
-        Contact* out = w.contacts + (size_t)g * MAXC;
-        for (int c = gl; c < nc; c += G) contact_to_constraint(e1, e2, cts[c], out[c]);
+        int nc = pair_manifold<G>(w, g, h1, h2, w.pair_normal[g], err, work, st + used, stage - used);
         if (gl == 0) {
             w.ncontact[g] = nc;
             if (err) atomicOr(&w.scene_err[s], err);
@@ -485,7 +469,7 @@ __global__ void __launch_bounds__(64) k_narrow_general(DevWorld w) {
         for (int c1 = w.body_col_off[b1]; c1 < w.body_col_off[b1 + 1]; ++c1)
             for (int c2 = w.body_col_off[b2]; c2 < w.body_col_off[b2 + 1]; ++c2) {
                 ColView v1 = col_view(w, b1, c1), v2 = col_view(w, b2, c2);
-                nc += collider_contacts(v1, v2, cts + nc, MAXC - nc, err, flags);
+                nc += collider_contacts(w.hulls, v1, v2, cts + nc, MAXC - nc, err, flags);
             }
         const Body& e1 = w.body[b1];
         const Body& e2 = w.body[b2];
@@ -790,16 +774,14 @@ __global__ void __launch_bounds__(64) k_pair_contacts(DevWorld w, int b1, int b2
     HullView h1 = hull_view(w, b1), h2 = hull_view(w, b2);
     uint32_t err = 0;
     int flags = 0;
-    char* work = w.group_work;
-    ContactPt* cts = (ContactPt*)(work + CLIP_BYTES);
-    int nc = pair_contacts<8>(h1, h2, cts, err, flags, work);
-    if (threadIdx.x != 0) return;
-    for (int k = 0; k < nc; ++k) {
+    auto emit = [&](int k, const ContactPt& c) {
         double* o = out + 9 * k;
-        o[0] = cts[k].p1.x; o[1] = cts[k].p1.y; o[2] = cts[k].p1.z;
-        o[3] = cts[k].p2.x; o[4] = cts[k].p2.y; o[5] = cts[k].p2.z;
-        o[6] = cts[k].n.x; o[7] = cts[k].n.y; o[8] = cts[k].n.z;
-    }
+        o[0] = c.p1.x; o[1] = c.p1.y; o[2] = c.p1.z;
+        o[3] = c.p2.x; o[4] = c.p2.y; o[5] = c.p2.z;
+        o[6] = c.n.x; o[7] = c.n.y; o[8] = c.n.z;
+    };
+    int nc = pair_contacts<8>(w.hulls, h1, h2, emit, err, flags, w.group_work);
+    if (threadIdx.x != 0) return;
     *count = nc;
     *err_out = err;
 }
@@ -828,6 +810,23 @@ __global__ void k_fp64_selftest(const double* a, const double* b, double* out, i
 // Launchers
 // ---------------------------------------------------------------------------
 static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+// LDS vertices of a pair's slice in the lane-group kernels: both hulls (`base`
+// vertices at most) and room beside them for the clipping polygons, which
+// otherwise go through the group's working memory on one lane (a pair of the
+// world's largest hulls, or any pair of a world of boxes, had none: 45 000 to
+// 62 000 cycles per manifold instead of 21 000). 8 points per polygon always,
+// up to 16 while eight blocks (two waves per SIMD) still share a CU's 160 KiB,
+// and never beyond the world's LDS limit.
+static int stage_slice(const DevWorld& w, int group, int base) {
+    if (group <= 1) return 0;
+    int per = 64 / group * (int)sizeof(V3);
+    int extra = std::max(16, std::min(32, 20 * 1024 / per - base));
+    return std::max(base, std::min(base + extra, w.lds_limit / per));
+}
+static size_t stage_bytes(int group, int stage) {
+    return group > 1 ? (size_t)(64 / group) * stage * sizeof(V3) : 0;
+}
 
 hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_t st, KernelTimer* kt,
                         const BigScene* bigs, int nbig, const Recorder* rec) {
@@ -875,7 +874,8 @@ hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_
                 t.end(st);
             }
             t.begin(KC_NARROW, st);
-            size_t lds = w.narrow_group > 1 ? (size_t)(64 / w.narrow_group) * w.stage_cap * sizeof(V3) : 0;
+            int stage = stage_slice(w, w.narrow_group, w.stage_cap);
+            size_t lds = stage_bytes(w.narrow_group, stage);
             dim3 nb(w.narrow_blocks), t64(64);
             if (fused && w.small_nv > 0 && w.narrow_group > 1) {
                 // two size classes: small-hull pairs with small LDS slices on the
@@ -883,26 +883,26 @@ hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_
                 // groups per block that fits
                 const int32_t* small = w.pair_lists;
                 const int32_t* big = w.pair_lists + w.list_stride;
-                size_t lds_s = (size_t)(64 / w.narrow_group) * w.stage_small * sizeof(V3);
+                int stage_s = stage_slice(w, w.narrow_group, w.stage_small), stage_b = stage_slice(w, 16, w.stage_cap);
+                size_t lds_s = stage_bytes(w.narrow_group, stage_s), lds_b = stage_bytes(16, stage_b);
                 switch (w.narrow_group) {
-                case 4: hipLaunchKernelGGL((k_gjk_epa<4, true>), nb, t64, lds_s, st, w, small, w.counters + CNT_SMALL, w.stage_small); break;
-                case 8: hipLaunchKernelGGL((k_gjk_epa<8, true>), nb, t64, lds_s, st, w, small, w.counters + CNT_SMALL, w.stage_small); break;
-                default: hipLaunchKernelGGL((k_gjk_epa<16, true>), nb, t64, lds_s, st, w, small, w.counters + CNT_SMALL, w.stage_small); break;
+                case 4: hipLaunchKernelGGL((k_gjk_epa<4, true>), nb, t64, lds_s, st, w, small, w.counters + CNT_SMALL, stage_s); break;
+                case 8: hipLaunchKernelGGL((k_gjk_epa<8, true>), nb, t64, lds_s, st, w, small, w.counters + CNT_SMALL, stage_s); break;
+                default: hipLaunchKernelGGL((k_gjk_epa<16, true>), nb, t64, lds_s, st, w, small, w.counters + CNT_SMALL, stage_s); break;
                 }
-                size_t lds_b = (size_t)(64 / 16) * w.stage_cap * sizeof(V3);
-                hipLaunchKernelGGL((k_gjk_epa<16, true>), nb, t64, lds_b, st, w, big, w.counters + CNT_BIG, w.stage_cap);
+                hipLaunchKernelGGL((k_gjk_epa<16, true>), nb, t64, lds_b, st, w, big, w.counters + CNT_BIG, stage_b);
             } else if (fused) {
                 switch (w.narrow_group) {
-                case 4: hipLaunchKernelGGL((k_gjk_epa<4, true>), nb, t64, lds, st, w, nullptr, nullptr, w.stage_cap); break;
-                case 8: hipLaunchKernelGGL((k_gjk_epa<8, true>), nb, t64, lds, st, w, nullptr, nullptr, w.stage_cap); break;
-                case 16: hipLaunchKernelGGL((k_gjk_epa<16, true>), nb, t64, lds, st, w, nullptr, nullptr, w.stage_cap); break;
+                case 4: hipLaunchKernelGGL((k_gjk_epa<4, true>), nb, t64, lds, st, w, nullptr, nullptr, stage); break;
+                case 8: hipLaunchKernelGGL((k_gjk_epa<8, true>), nb, t64, lds, st, w, nullptr, nullptr, stage); break;
+                case 16: hipLaunchKernelGGL((k_gjk_epa<16, true>), nb, t64, lds, st, w, nullptr, nullptr, stage); break;
                 default: hipLaunchKernelGGL(k_gjk_epa_lane<true>, nb, t64, 0, st, w); break;
                 }
             } else {
                 switch (w.narrow_group) {
-                case 4: hipLaunchKernelGGL((k_gjk_epa<4, false>), nb, t64, lds, st, w, nullptr, nullptr, w.stage_cap); break;
-                case 8: hipLaunchKernelGGL((k_gjk_epa<8, false>), nb, t64, lds, st, w, nullptr, nullptr, w.stage_cap); break;
-                case 16: hipLaunchKernelGGL((k_gjk_epa<16, false>), nb, t64, lds, st, w, nullptr, nullptr, w.stage_cap); break;
+                case 4: hipLaunchKernelGGL((k_gjk_epa<4, false>), nb, t64, lds, st, w, nullptr, nullptr, stage); break;
+                case 8: hipLaunchKernelGGL((k_gjk_epa<8, false>), nb, t64, lds, st, w, nullptr, nullptr, stage); break;
+                case 16: hipLaunchKernelGGL((k_gjk_epa<16, false>), nb, t64, lds, st, w, nullptr, nullptr, stage); break;
                 default: hipLaunchKernelGGL(k_gjk_epa_lane<false>, nb, t64, 0, st, w); break;
                 }
             }
@@ -910,13 +910,14 @@ hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_
             t.end(st);
             if (!fused) {
                 t.begin(KC_MANIFOLD, st);
-                lds = w.manifold_group > 1 ? (size_t)(64 / w.manifold_group) * w.stage_cap * sizeof(V3) : 0;
+                stage = stage_slice(w, w.manifold_group, w.stage_cap);
+                lds = stage_bytes(w.manifold_group, stage);
                 dim3 mb(w.manifold_blocks);
                 switch (w.manifold_group) {
-                case 4: hipLaunchKernelGGL(k_manifold<4>, mb, t64, lds, st, w); break;
-                case 8: hipLaunchKernelGGL(k_manifold<8>, mb, t64, lds, st, w); break;
-                case 16: hipLaunchKernelGGL(k_manifold<16>, mb, t64, lds, st, w); break;
-                default: hipLaunchKernelGGL(k_manifold<1>, mb, t64, 0, st, w); break;
+                case 4: hipLaunchKernelGGL(k_manifold<4>, mb, t64, lds, st, w, stage); break;
+                case 8: hipLaunchKernelGGL(k_manifold<8>, mb, t64, lds, st, w, stage); break;
+                case 16: hipLaunchKernelGGL(k_manifold<16>, mb, t64, lds, st, w, stage); break;
+                default: hipLaunchKernelGGL(k_manifold<1>, mb, t64, 0, st, w, 0); break;
                 }
                 t.end(st);
             }

@@ -387,9 +387,11 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
     d.nb = (int)hw.body.size();
     d.n_ext = (int)hw.ext.size();
     // topology dedupe: bodies of the same shape share index lists
-    std::map<std::vector<int32_t>, int32_t> topo_ids;
-    std::vector<int32_t> topo_base, topo_pool;
-    std::vector<int32_t> hull_nv, hull_nf, hull_v_off, hull_fn_off, hull_topo;
+    std::map<std::vector<int32_t>, int2> topo_ids;  // first vertex and first face record
+    std::vector<int32_t> topo_list;
+    std::vector<int4> topo_rec, hull_rec;
+    std::vector<int2> topo_nbr;
+    std::vector<int32_t> hull_nv, hull_v_off;
     std::vector<V3> hull_v, hull_fn;
     for (const HostHull& h : hw.hulls) {
         std::vector<int32_t> key;
@@ -400,18 +402,30 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
         }
         auto it = topo_ids.find(key);
         if (it == topo_ids.end()) {
-            int32_t id = (int32_t)topo_ids.size();
-            for (auto* p : parts) {
-                topo_base.push_back((int32_t)topo_pool.size());
-                topo_pool.insert(topo_pool.end(), p->begin(), p->end());
+            // the lists, then one record per vertex and per face (HullTables)
+            auto append = [&](const std::vector<int32_t>& v) {
+                int32_t at = (int32_t)topo_list.size();
+                topo_list.insert(topo_list.end(), v.begin(), v.end());
+                return at;
+            };
+            int32_t fe = append(h.fe), vf = append(h.vf), vn = append(h.vn), ff = (int32_t)topo_nbr.size();
+            for (int32_t f : h.ff) {
+                bool any = f >= 0 && (size_t)f < h.fn.size() && h.fe_off[f + 1] > h.fe_off[f];
+                topo_nbr.push_back(make_int2(f, any ? h.fe[h.fe_off[f]] : 0));
             }
-            it = topo_ids.emplace(key, id).first;
+            int2 first = make_int2((int32_t)topo_rec.size(), 0);
+            for (size_t v = 0; v < h.v.size(); ++v)
+                topo_rec.push_back(make_int4(vf + h.vf_off[v], h.vf_off[v + 1] - h.vf_off[v], vn + h.vn_off[v],
+                                             h.vn_off[v + 1] - h.vn_off[v]));
+            first.y = (int32_t)topo_rec.size();
+            for (size_t f = 0; f < h.fn.size(); ++f)
+                topo_rec.push_back(make_int4(fe + h.fe_off[f], h.fe_off[f + 1] - h.fe_off[f], ff + h.ff_off[f],
+                                             h.ff_off[f + 1] - h.ff_off[f]));
+            it = topo_ids.emplace(key, first).first;
         }
-        hull_topo.push_back(it->second);
+        hull_rec.push_back(make_int4(it->second.x, it->second.y, (int32_t)hull_fn.size(), (int32_t)hull_v.size()));
         hull_nv.push_back((int32_t)h.v.size());
-        hull_nf.push_back((int32_t)h.fn.size());
         hull_v_off.push_back((int32_t)hull_v.size());
-        hull_fn_off.push_back((int32_t)hull_fn.size());
         hull_v.insert(hull_v.end(), h.v.begin(), h.v.end());
         hull_fn.insert(hull_fn.end(), h.fn.begin(), h.fn.end());
     }
@@ -561,6 +575,7 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
     ok &= im.upload(d.scene_item_base, con_base);
     ok &= im.upload_mut(d.body, hw.body);
     ok &= im.alloc(d.model, d.nb);
+    d.hulls.model = d.model;
     ok &= im.alloc(d.pose, (size_t)d.nb * 7);
     std::vector<V3> scale = hw.body_scale;
     scale.resize(d.nb, v3(1.0, 1.0, 1.0));
@@ -569,14 +584,13 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
     const int32_t* p;
     ok &= im.upload(p, im.body_tv_off); d.body_tv_off = p;
     ok &= im.upload(d.hull_nv, hull_nv);
-    ok &= im.upload(d.hull_nf, hull_nf);
     ok &= im.upload(d.hull_v_off, hull_v_off);
-    ok &= im.upload(d.hull_fn_off, hull_fn_off);
-    ok &= im.upload(d.hull_topo, hull_topo);
+    ok &= im.upload(d.hulls.hull, hull_rec);
+    ok &= im.upload(d.hulls.rec, topo_rec);
+    ok &= im.upload(d.hulls.list, topo_list);
+    ok &= im.upload(d.hulls.nbr, topo_nbr);
     ok &= im.upload(d.hull_v, hull_v);
-    ok &= im.upload(d.hull_fn, hull_fn);
-    ok &= im.upload(d.topo_base, topo_base);
-    ok &= im.upload(d.topo_pool, topo_pool);
+    ok &= im.upload(d.hulls.fn, hull_fn);
     ok &= im.alloc(d.tv, (size_t)ntv);
     ok &= im.alloc(d.need, d.nb);
     ok &= im.upload(d.xf, xf);
