@@ -228,6 +228,19 @@ int scan_block_count(int64_t n);
 hipError_t launch_pair_contacts(const DevWorld& w, int b1, int b2, double* out, int* count, uint32_t* err,
                                 hipStream_t st);
 hipError_t launch_broad(const DevWorld& w, hipStream_t st, const BigScene* bigs = nullptr, int nbig = 0);
+// State I/O: the arrays of rp_state for nb bodies one after another: the
+// sections of doubles in the body record's order (position, rotation, linear
+// and angular velocity, the previous four, deactivation time), then `active`.
+constexpr int STATE_SECTIONS = 9, STATE_DOUBLES = 27;
+__host__ __device__ constexpr int state_section(int s) {  // first double of section s
+    constexpr int first[STATE_SECTIONS + 1] = {0, 3, 7, 10, 13, 16, 20, 23, 26, 27};
+    return first[s];
+}
+static_assert(offsetof(Body, x) == 0 && offsetof(Body, px) == 13 * 8 && offsetof(Body, pw) == 23 * 8 &&
+                  offsetof(Body, deact) == 26 * 8,
+              "the state leads the body record");
+hipError_t launch_state_out(const DevWorld& w, double* out, hipStream_t st);
+hipError_t launch_state_in(const DevWorld& w, const double* in, unsigned mask, hipStream_t st);
 // entity_get_model_matrix of every body into out ([nb][4][4] row-major,
 // double or float), device memory.
 hipError_t launch_model_matrices(const DevWorld& w, void* out, bool f32, hipStream_t st);

@@ -228,6 +228,37 @@ __global__ void k_keep_pose(DevWorld w) {
     p[3] = e.q.x; p[4] = e.q.y; p[5] = e.q.z; p[6] = e.q.w;
 }
 
+// The bodies' states as the flat arrays of rp_state, one after another
+// (StateSection), and back: of the arrays in `mask` only.
+__global__ void k_state_out(DevWorld w, double* out) {
+    int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= w.nb) return;
+    const double* e = (const double*)&w.body[b];  // the state leads the record
+    double v[STATE_DOUBLES];
+#pragma unroll
+    for (int c = 0; c < STATE_DOUBLES; ++c) v[c] = e[c];
+#pragma unroll
+    for (int s = 0; s < STATE_SECTIONS; ++s)
+#pragma unroll
+        for (int c = state_section(s); c < state_section(s + 1); ++c)
+            out[(size_t)state_section(s) * w.nb + (size_t)b * (state_section(s + 1) - state_section(s)) +
+                (c - state_section(s))] = v[c];
+    ((int32_t*)(out + (size_t)STATE_DOUBLES * w.nb))[b] = w.body[b].active;
+}
+__global__ void k_state_in(DevWorld w, const double* in, unsigned mask) {
+    int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= w.nb) return;
+    double* e = (double*)&w.body[b];
+#pragma unroll
+    for (int s = 0; s < STATE_SECTIONS; ++s)
+        if (mask >> s & 1)
+#pragma unroll
+            for (int c = state_section(s); c < state_section(s + 1); ++c)
+                e[c] = in[(size_t)state_section(s) * w.nb + (size_t)b * (state_section(s + 1) - state_section(s)) +
+                          (c - state_section(s))];
+    if (mask >> STATE_SECTIONS & 1) w.body[b].active = ((const int32_t*)(in + (size_t)STATE_DOUBLES * w.nb))[b];
+}
+
 // entity_get_model_matrix of every body, row-major 4x4, as double or as the
 // float array util_matrix_to_r32_array (util.cpp:77-94) hands to the renderer.
 template <class F>
@@ -938,6 +969,15 @@ hipError_t launch_pair_contacts(const DevWorld& w, int b1, int b2, double* out, 
     hipLaunchKernelGGL(k_model, dim3(cdiv(w.nb, 128)), dim3(128), 0, st, w);
     hipLaunchKernelGGL(k_transform, dim3(cdiv(w.n_xf, 256)), dim3(256), 0, st, w, 1);
     hipLaunchKernelGGL(k_pair_contacts, dim3(1), dim3(64), 0, st, w, b1, b2, out, count, err);
+    return hipGetLastError();
+}
+
+hipError_t launch_state_out(const DevWorld& w, double* out, hipStream_t st) {
+    hipLaunchKernelGGL(k_state_out, dim3(cdiv(w.nb, 256)), dim3(256), 0, st, w, out);
+    return hipGetLastError();
+}
+hipError_t launch_state_in(const DevWorld& w, const double* in, unsigned mask, hipStream_t st) {
+    hipLaunchKernelGGL(k_state_in, dim3(cdiv(w.nb, 256)), dim3(256), 0, st, w, in, mask);
     return hipGetLastError();
 }
 
