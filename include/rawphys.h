@@ -372,8 +372,7 @@ int32_t rp_world_lds_limit(const rp_world* w);
  * of about equal body counts and replays each on a stream of its own, so
  * that one range's latency-bound kernels overlap another's (scenes never
  * interact, so results are identical). Used with the grouped narrow-phase
- * schedules (narrow group > 1, manifold group 0, 4, 8 or 16) in worlds
- * without sphere or compound pairs. views: 0 = automatic (3 from 64
+ * schedules (narrow group > 1, manifold group 0, 4, 8 or 16). views: 0 = automatic (3 from 64
  * scenes: with the runtime's default of four hardware queues per process,
  * a fourth view's stream shares a queue), 1 = none, 2..4. rp_world_views:
  * the number the last captured frame used. Returns 0 or -1. */

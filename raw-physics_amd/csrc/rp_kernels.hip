@@ -338,8 +338,38 @@ __device__ __forceinline__ bool general_pair(const DevWorld& w, int b1, int b2) 
     return w.has_general && (w.body_general[b1] | w.body_general[b2]);
 }
 
-// Hull views of live pair g; for G > 1 the group's lanes transform both
-// hulls' vertices into the group's LDS stage `st`.
+// Two hulls of bodies b1 and b2, transformed by the group's lanes into the
+// group's LDS slice `st`, one after the other. hv: first local vertices and
+// vertex counts.
+template <int G>
+__device__ __forceinline__ void stage_pair(const DevWorld& w, int b1, int b2, int4 hv, V3* st, int gl) {
+    const V3* lv1 = w.hull_v + hv.x;
+    const V3* lv2 = w.hull_v + hv.y;
+    int nv1 = hv.z, nv2 = hv.w;
+    const M4 M1 = w.model[b1], M2 = w.model[b2];
+    // both hulls together, two vertices of each per lane and batch, all
+    // loaded before any is transformed
+    int n = nv1 > nv2 ? nv1 : nv2;
+    for (int i = gl; i < n; i += 2 * G) {
+        V3 va[2], vb[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            int j = i + k * G;
+            if (j < nv1) va[k] = lv1[j];
+            if (j < nv2) vb[k] = lv2[j];
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            int j = i + k * G;
+            if (j < nv1) st[j] = transform_vertex(M1, va[k]);
+            if (j < nv2) st[nv1 + j] = transform_vertex(M2, vb[k]);
+        }
+    }
+    group_lds_sync();
+}
+// Hull views of live pair g, staged in `st` for G > 1 (vertex offsets and
+// counts from the pair's record: the vertex loads depend on that one load
+// only).
 template <int G>
 __device__ __forceinline__ void pair_views(const DevWorld& w, int g, V3* st, int gl, int& s, int& b1, int& b2,
                                            HullView& h1, HullView& h2) {
@@ -351,34 +381,10 @@ __device__ __forceinline__ void pair_views(const DevWorld& w, int g, V3* st, int
         h1 = hull_view_of(w, b1, r.z, w.body_tv_off[b1]);
         h2 = hull_view_of(w, b2, r.w, w.body_tv_off[b2]);
     } else {
-        // vertex offsets and counts from the pair's record: the vertex loads
-        // depend on that one load only
         int4 hv = w.live_hull[g];
-        const V3* lv1 = w.hull_v + hv.x;
-        const V3* lv2 = w.hull_v + hv.y;
-        int nv1 = hv.z, nv2 = hv.w;
-        const M4 M1 = w.model[b1], M2 = w.model[b2];
-        // both hulls together, two vertices of each per lane and batch, all
-        // loaded before any is transformed
-        int n = nv1 > nv2 ? nv1 : nv2;
-        for (int i = gl; i < n; i += 2 * G) {
-            V3 va[2], vb[2];
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                int j = i + k * G;
-                if (j < nv1) va[k] = lv1[j];
-                if (j < nv2) vb[k] = lv2[j];
-            }
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                int j = i + k * G;
-                if (j < nv1) st[j] = transform_vertex(M1, va[k]);
-                if (j < nv2) st[nv1 + j] = transform_vertex(M2, vb[k]);
-            }
-        }
-        group_lds_sync();
-        h1 = HullView{st, nv1, r.z, b1};
-        h2 = HullView{st + nv1, nv2, r.w, b2};
+        stage_pair<G>(w, b1, b2, hv, st, gl);
+        h1 = HullView{st, hv.z, r.z, b1};
+        h2 = HullView{st + hv.z, hv.w, r.w, b2};
     }
 }
 
@@ -391,7 +397,7 @@ __device__ __forceinline__ int pair_manifold(const DevWorld& w, int g, const Hul
     const Body& e2 = w.body[h2.body];
     Contact* out = w.contacts + (size_t)g * MAXC;
     auto emit = [&](int k, const ContactPt& c) { contact_to_constraint(e1, e2, c, out[k]); };
-    if constexpr (G == 1) return manifold_lane(w.hulls, h1, h2, n, emit, err);
+    if constexpr (G == 1) return manifold_lane(w.hulls, h1, h2, n, emit, err, work);
     else return manifold_group<G>(w.hulls, h1, h2, n, emit, err, work, spare, spare_n);
 }
 
@@ -404,6 +410,7 @@ template <int G, bool kManifold>
 __device__ __forceinline__ void gjk_epa_pairs(DevWorld& w, const int32_t* list, const int32_t* count, int stage) {
     extern __shared__ V3 rp_stage[];
     constexpr int NG = 64 / G;
+    alignas(16) char own[G == 1 ? (kManifold ? GROUP_WORK_BYTES : EPA_BYTES) : 1];  // a lone lane's working memory
     int grp = threadIdx.x / G, gl = threadIdx.x & (G - 1);
     V3* st = rp_stage + grp * stage;
     int total = list ? *count : w.live_prefix[w.ns];
@@ -420,7 +427,7 @@ __device__ __forceinline__ void gjk_epa_pairs(DevWorld& w, const int32_t* list, 
         V3 n = v3(0.0, 0.0, 0.0);
         double pen;
         int r = 0;
-        char* work = G > 1 ? w.group_work + (size_t)(blockIdx.x * NG + grp) * GROUP_WORK_BYTES : nullptr;
+        char* work = G > 1 ? w.group_work + (size_t)(blockIdx.x * NG + grp) * GROUP_WORK_BYTES : own;
         bool hit = gjk<G>(h1, h2, sx, err, cycled);
         if (hit) r = epa<G>(h1, h2, sx, n, pen, err, work);
         if constexpr (kManifold) {
@@ -466,6 +473,7 @@ __global__ void __launch_bounds__(64) k_manifold(DevWorld w, int stage) {
     constexpr int NG = 64 / G;
     int grp = threadIdx.x / G, gl = threadIdx.x & (G - 1);
     V3* st = rp_stage + grp * stage;
+    alignas(16) char own[G == 1 ? CLIP_BYTES : 1];
     int total = w.counters[CNT_MANIFOLD];
     for (int k = blockIdx.x * NG + grp; k < total; k += gridDim.x * NG) {
         int g = w.mlist[k];
@@ -473,7 +481,7 @@ __global__ void __launch_bounds__(64) k_manifold(DevWorld w, int stage) {
         HullView h1, h2;
         pair_views<G>(w, g, st, gl, s, b1, b2, h1, h2);
         uint32_t err = 0;
-        char* work = G > 1 ? w.group_work + (size_t)(blockIdx.x * NG + grp) * GROUP_WORK_BYTES : nullptr;
+        char* work = G > 1 ? w.group_work + (size_t)(blockIdx.x * NG + grp) * GROUP_WORK_BYTES : own;
         int used = h1.nv + h2.nv;
         int nc = pair_manifold<G>(w, g, h1, h2, w.pair_normal[g], err, work, st + used, stage - used);
         if (gl == 0) {
@@ -484,32 +492,61 @@ __global__ void __launch_bounds__(64) k_manifold(DevWorld w, int stage) {
     }
 }
 
-// Live pairs with a sphere collider or a multi-collider body, one lane per
-// pair: colliders_get_contacts (collider.cpp:560-572) over every collider
-// pair in order, each by collider_get_contacts (collider.cpp:523-558).
-__global__ void __launch_bounds__(64) k_narrow_general(DevWorld w) {
+// Live pairs with a sphere collider or a multi-collider body:
+// colliders_get_contacts (collider.cpp:560-572) over every collider pair in
+// order, each by collider_get_contacts (collider.cpp:523-558), at most MAXC
+// contacts of the pair kept. One lane group per pair, each collider pair's
+// hulls staged in its LDS slice (G = 8 or 16), as the fast path (256 scenes of
+// spheres, boxes and dumbbells: 170 -> 97 us per launch, and the world may be
+// stepped in concurrent views, 4.9 -> 2.8 ms per frame); in worlds whose hulls
+// leave no room for that, one lane per pair over the pre-transformed vertices
+// with private arrays (G = 1).
+template <int G>
+__global__ void __launch_bounds__(64) k_narrow_general(DevWorld w, int stage) {
+    extern __shared__ V3 rp_stage[];
+    constexpr int NG = 64 / G;
+    const int grp = threadIdx.x / G, gl = threadIdx.x & (G - 1);
+    V3* st = rp_stage + grp * stage;
+    alignas(16) char own[G == 1 ? GROUP_WORK_BYTES : 1];
+    char* work = G > 1 ? w.group_work + (size_t)(blockIdx.x * NG + grp) * GROUP_WORK_BYTES : own;
     int total = w.live_prefix[w.ns];
-    for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < total; g += gridDim.x * blockDim.x) {
+    for (int g = blockIdx.x * NG + grp; g < total; g += gridDim.x * NG) {
         int s, b1, b2;
         pair_bodies(w, g, s, b1, b2);
         if (!general_pair(w, b1, b2)) continue;
         uint32_t err = 0;
-        int flags = 0;
-        ContactPt cts[MAXC];
-        int nc = 0;
-        for (int c1 = w.body_col_off[b1]; c1 < w.body_col_off[b1 + 1]; ++c1)
-            for (int c2 = w.body_col_off[b2]; c2 < w.body_col_off[b2 + 1]; ++c2) {
-                ColView v1 = col_view(w, b1, c1), v2 = col_view(w, b2, c2);
-                nc += collider_contacts(w.hulls, v1, v2, cts + nc, MAXC - nc, err, flags);
-            }
+        int flags = 0, nc = 0;
         const Body& e1 = w.body[b1];
         const Body& e2 = w.body[b2];
         Contact* out = w.contacts + (size_t)g * MAXC;
-        for (int c = 0; c < nc; ++c) contact_to_constraint(e1, e2, cts[c], out[c]);
-        w.ncontact[g] = nc;
-        if (err) atomicOr(&w.scene_err[s], err);
-        if (flags & PAIR_EPA_FAIL) atomicAdd(&w.stats[STAT_EPA_FAIL], 1ull);
-        if (flags & PAIR_GJK_CYCLE) atomicAdd(&w.stats[STAT_GJK_CYCLE], 1ull);
+        const int c1e = w.body_col_off[b1 + 1], c2e = w.body_col_off[b2 + 1];
+        for (int c1 = w.body_col_off[b1]; c1 < c1e; ++c1)
+            for (int c2 = w.body_col_off[b2]; c2 < c2e; ++c2) {
+                ColView v1 = col_view(w, b1, c1), v2 = col_view(w, b2, c2);
+                int used = v1.h.nv + v2.h.nv;
+                if constexpr (G > 1) {
+                    if (used > 0) {
+                        int4 hv = make_int4(v1.h.nv ? w.hull_v_off[v1.h.hid] : 0, v2.h.nv ? w.hull_v_off[v2.h.hid] : 0,
+                                            v1.h.nv, v2.h.nv);
+                        stage_pair<G>(w, b1, b2, hv, st, gl);
+                    }
+                    v1.h.tv = st;
+                    v2.h.tv = st + v1.h.nv;
+                }
+                auto emit = [&](int k, const ContactPt& c) {
+                    if (nc + k < MAXC) contact_to_constraint(e1, e2, c, out[nc + k]);
+                };
+                int n = collider_contacts<G>(w.hulls, v1, v2, emit, err, flags, work, st + used, stage - used);
+                if (nc + n > MAXC) err |= ERR_CONTACT_CAPACITY;
+                nc = min(nc + n, MAXC);
+                if constexpr (G > 1) group_lds_sync();
+            }
+        if (gl == 0) {
+            w.ncontact[g] = nc;
+            if (err) atomicOr(&w.scene_err[s], err);
+            if (flags & PAIR_EPA_FAIL) atomicAdd(&w.stats[STAT_EPA_FAIL], 1ull);
+            if (flags & PAIR_GJK_CYCLE) atomicAdd(&w.stats[STAT_GJK_CYCLE], 1ull);
+        }
     }
 }
 
@@ -899,7 +936,7 @@ hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_
             hipLaunchKernelGGL(k_keep_pose, dim3(cdiv(w.nb, 256)), dim3(256), 0, st, w);
         if (fp.collisions) {
             bool fused = w.manifold_group == 0;
-            if (w.narrow_group == 1 || w.manifold_group == 1 || w.has_general) {
+            if (w.narrow_group == 1 || w.manifold_group == 1) {
                 t.begin(KC_TRANSFORM, st);
                 hipLaunchKernelGGL(k_transform, dim3(cdiv(w.n_xf, 256)), dim3(256), 0, st, w, 0);
                 t.end(st);
@@ -937,7 +974,17 @@ hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_
                 default: hipLaunchKernelGGL(k_gjk_epa_lane<false>, nb, t64, 0, st, w); break;
                 }
             }
-            if (w.has_general) hipLaunchKernelGGL(k_narrow_general, dim3(1024), t64, 0, st, w);
+            if (w.has_general) {
+                // (at least 8 lanes per pair: the working memory is sized for
+                // the narrow schedule's groups)
+                int gg = w.narrow_group == 4 ? 8 : w.narrow_group;
+                int gs = stage_slice(w, gg, w.stage_cap);
+                switch (gg) {
+                case 8: hipLaunchKernelGGL(k_narrow_general<8>, nb, t64, stage_bytes(8, gs), st, w, gs); break;
+                case 16: hipLaunchKernelGGL(k_narrow_general<16>, nb, t64, stage_bytes(16, gs), st, w, gs); break;
+                default: hipLaunchKernelGGL(k_narrow_general<1>, dim3(1024), t64, 0, st, w, 0); break;
+                }
+            }
             t.end(st);
             if (!fused) {
                 t.begin(KC_MANIFOLD, st);
@@ -1033,7 +1080,8 @@ hipError_t allow_narrow_lds(int bytes) {
     const void* k[] = {(const void*)k_gjk_epa<4, true>, (const void*)k_gjk_epa<8, true>,
                        (const void*)k_gjk_epa<16, true>, (const void*)k_gjk_epa<4, false>,
                        (const void*)k_gjk_epa<8, false>, (const void*)k_gjk_epa<16, false>,
-                       (const void*)k_manifold<4>, (const void*)k_manifold<8>, (const void*)k_manifold<16>};
+                       (const void*)k_manifold<4>, (const void*)k_manifold<8>, (const void*)k_manifold<16>,
+                       (const void*)k_narrow_general<8>, (const void*)k_narrow_general<16>};
     for (const void* f : k) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         if (e != hipSuccess) return e;

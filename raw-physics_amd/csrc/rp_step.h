@@ -347,17 +347,17 @@ RP_HD V3 support_md(const HullView& a, const HullView& b, V3 d, uint32_t& err) {
     return sub(a.tv[i1], b.tv[i2]);
 }
 
-// support_point of one collider (support.cpp:19-31); the general path runs
-// one lane per pair.
+// support_point of one collider (support.cpp:19-31).
+template <int G = 1>
 RP_HD V3 support_point(const ColView& c, V3 d, uint32_t& err) {
     if (c.type == COL_SPHERE) return add(c.center, scl((double)c.radius, nrm(d)));
-    return c.h.tv[support_index<1>(c.h, d, err)];
+    return c.h.tv[support_index<G>(c.h, d, err)];
 }
 // support_point_of_minkowski_difference (support.cpp:34-39)
 template <int G = 1>
 RP_HD V3 support_md(const ColView& a, const ColView& b, V3 d, uint32_t& err) {
-    V3 s1 = support_point(a, d, err);
-    V3 s2 = support_point(b, scl(-1.0, d), err);
+    V3 s1 = support_point<G>(a, d, err);
+    V3 s2 = support_point<G>(b, scl(-1.0, d), err);
     return sub(s1, s2);
 }
 
@@ -905,22 +905,13 @@ __device__ int epa_group(const View& h1, const View& h2, const Simplex& s, V3& n
 }
 
 // epa (epa.cpp:118-237): 0 = no convergence, 1 = converged, -1 = error.
-// G > 1: the group's lanes compute each support point together; the
-// polytope lives in lane 0 alone (in the group's working memory `work`),
-// which expands it and hands the next direction and the status to the group. Every lane returns
-// the status and, on convergence, lane 0's n_out / pen_out; the EPA error
-// bits are set in lane 0's err only.
+// On one lane (G = 1) with its working memory, or on a lane group (epa_group).
 template <int G = 1, class View = HullView>
 RP_HD int epa(const View& h1, const View& h2, const Simplex& s, V3& n_out, double& pen_out, uint32_t& err,
-              char* work = nullptr) {
+              char* work) {
     if constexpr (G == 1) {
-        V3 poly[EPA_MAXV];
-        I3 faces[EPA_MAXF];
-        V3 normals[EPA_MAXF];
-        double dist[EPA_MAXF];
-        int2 edges[EPA_MAXE];
         EpaPoly P;
-        P.poly = poly; P.faces = faces; P.normals = normals; P.dist = dist; P.edges = edges;
+        epa_bind(P, work);
         if (!P.init(s, err)) return -1;
         for (int it = 0; it < 100; ++it) {
             V3 sp = support_md<G>(h1, h2, P.min_n, err);
@@ -1181,10 +1172,11 @@ __device__ __forceinline__ int contacts_from_clip_group(const V3* pts, int n, co
     return nc;
 }
 
-// convex_convex_contact_manifold (clipping.cpp:249-341), one lane per pair.
-// Returns the number of contacts handed to emit(k, contact) (at most MAXC).
+// convex_convex_contact_manifold (clipping.cpp:249-341), one lane per pair,
+// with working memory `work`. Returns the number of contacts handed to emit(k, contact) (at most MAXC).
 template <class Emit>
-RP_HD int manifold_lane(const HullTables& T, const HullView& h1, const HullView& h2, V3 normal, Emit emit, uint32_t& err) {
+RP_HD int manifold_lane(const HullTables& T, const HullView& h1, const HullView& h2, V3 normal, Emit emit, uint32_t& err,
+                        char* work) {
     const double EPSILON = 0.0001;
     V3 inormal = inv3(normal);
     HullFaces hf1 = hull_faces(T, h1), hf2 = hull_faces(T, h2);
@@ -1233,9 +1225,8 @@ RP_HD int manifold_lane(const HullTables& T, const HullView& h1, const HullView&
     rp.normal = inv3(ref1 ? n1 : n2);
     rp.point = rtv[T.list[rf.x]];
     const V3* res = nullptr;
-    V3 bufA[CLIP_MAX], bufB[CLIP_MAX];  // here, in the frame that reads the result
-    int n = clip_serial(T, rtv, ref1 ? hf1.fn : hf2.fn, ref1 ? hf1.R : hf2.R, rf, ref1 ? h2.tv : h1.tv, inf, rp, bufA, bufB,
-                        res, err);
+    int n = clip_serial(T, rtv, ref1 ? hf1.fn : hf2.fn, ref1 ? hf1.R : hf2.R, rf, ref1 ? h2.tv : h1.tv, inf, rp, (V3*)work,
+                        (V3*)work + CLIP_MAX, res, err);
     return contacts_from_clip(res, n, rp, normal, ref1, emit, err);
 }
 
@@ -1428,66 +1419,60 @@ __device__ __forceinline__ int pair_contacts(const HullTables& T, const HullView
     return manifold_group<G>(T, h1, h2, n, emit, err, work, nullptr, 0);
 }
 
-// clipping_get_contact_manifold (clipping.cpp:343-371) for colliders: a
-// sphere gives one contact at its support point along the normal.
-RP_HD int collider_manifold(const HullTables& T, const ColView& c1, const ColView& c2, V3 normal, double penetration,
-                            ContactPt* out, uint32_t& err) {
+// clipping_get_contact_manifold (clipping.cpp:343-371) where a collider is a
+// sphere: one contact at its support point along the normal.
+template <int G>
+RP_HD ContactPt sphere_contact(const ColView& c1, const ColView& c2, V3 normal, double penetration, uint32_t& err) {
+    ContactPt c;
+    c.n = normal;
     if (c1.type == COL_SPHERE) {
-        V3 p = support_point(c1, normal, err);
-        out[0].p1 = p;
-        out[0].p2 = sub(p, scl(penetration, normal));
-        out[0].n = normal;
-        return 1;
+        c.p1 = support_point<G>(c1, normal, err);
+        c.p2 = sub(c.p1, scl(penetration, normal));
+    } else {
+        c.p2 = support_point<G>(c2, inv3(normal), err);
+        c.p1 = add(c.p2, scl(penetration, normal));
     }
-    if (c2.type == COL_SPHERE) {
-        V3 inormal = inv3(normal);
-        V3 p = support_point(c2, inormal, err);
-        out[0].p1 = add(p, scl(penetration, normal));
-        out[0].p2 = p;
-        out[0].n = normal;
-        return 1;
-    }
-    return manifold_lane(T, c1.h, c2.h, normal, [&](int k, const ContactPt& c) { out[k] = c; }, err);
+    return c;
 }
 
-// collider_get_contacts (collider.cpp:523-558) for any two colliders. Two
-// spheres are resolved with the reference's float arithmetic; the float
-// square root is taken in double and rounded once, which is the correctly
-// rounded result (a 53-bit square root of a 24-bit value). `cap` is the room
-// left in `out`.
-RP_HD int collider_contacts(const HullTables& T, const ColView& c1, const ColView& c2, ContactPt* out, int cap, uint32_t& err,
-                            int& flags) {
-    ContactPt tmp[MAXC];
-    int n = 0;
+// collider_get_contacts (collider.cpp:523-558) for any two colliders, on one
+// lane (G = 1) or on a lane group, whose lanes emit the contacts they made
+// (emit(k, contact)). Two spheres are resolved with the reference's float
+// arithmetic; the float square root is taken in double and rounded once,
+// which is the correctly rounded result (a 53-bit square root of a 24-bit
+// value). `spare` as for manifold_group.
+template <int G, class Emit>
+RP_HD int collider_contacts(const HullTables& T, const ColView& c1, const ColView& c2, Emit emit, uint32_t& err, int& flags,
+                            char* work = nullptr, V3* spare = nullptr, int spare_n = 0) {
+    V3 n;
+    double pen;
     if (c1.type == COL_SPHERE && c2.type == COL_SPHERE) {
         V3 dv = sub(c1.center, c2.center);
         float dsq = (float)dot(dv, dv);
         float mind = c1.radius + c2.radius;
-        if (dsq < (mind * mind)) {
-            V3 nrm_ = nrm(sub(c2.center, c1.center));
-            float root = (float)sqrt((double)dsq);
-            double pen = (double)(mind - root);
-            n = collider_manifold(T, c1, c2, nrm_, pen, tmp, err);
-        }
+        if (!(dsq < (mind * mind))) return 0;
+        n = nrm(sub(c2.center, c1.center));
+        float root = (float)sqrt((double)dsq);
+        pen = (double)(mind - root);
     } else {
         Simplex s;
         bool cycled = false;
-        if (gjk<1>(c1, c2, s, err, cycled)) {
-            V3 nn;
-            double pen;
-            int r = epa<1>(c1, c2, s, nn, pen, err);
-            if (r != 1) flags |= PAIR_EPA_FAIL;
-            else n = collider_manifold(T, c1, c2, nn, pen, tmp, err);
-        } else if (cycled) {
-            flags |= PAIR_GJK_CYCLE;
+        if (!gjk<G>(c1, c2, s, err, cycled)) {
+            if (cycled) flags |= PAIR_GJK_CYCLE;
+            return 0;
+        }
+        if (epa<G>(c1, c2, s, n, pen, err, work) != 1) {
+            flags |= PAIR_EPA_FAIL;
+            return 0;
         }
     }
-    if (n > cap) {
-        err |= ERR_CONTACT_CAPACITY;
-        n = cap;
+    if (c1.type == COL_SPHERE || c2.type == COL_SPHERE) {
+        ContactPt c = sphere_contact<G>(c1, c2, n, pen, err);
+        if (G == 1 || (__lane_id() & (G - 1)) == 0) emit(0, c);
+        return 1;
     }
-    for (int k = 0; k < n; ++k) out[k] = tmp[k];
-    return n;
+    if constexpr (G == 1) return manifold_lane(T, c1.h, c2.h, n, emit, err, work);
+    else return manifold_group<G>(T, c1.h, c2.h, n, emit, err, work, spare, spare_n);
 }
 
 // ---------------------------------------------------------------------------

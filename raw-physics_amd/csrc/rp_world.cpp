@@ -883,9 +883,8 @@ static hipStream_t pool_stream(int k) {
 }
 static hipStream_t shared_stream() { return pool_stream(0); }
 
-// Views for graph replay: with a grouped narrow schedule whose kernels keep
-// no large private memory (no one-lane kernels, no sphere or compound pairs)
-// and enough scenes, the world is cut into up to kMaxViews scene ranges of
+// Views for graph replay: with a grouped narrow schedule, whose kernels keep
+// no large private memory, and enough scenes, the world is cut into up to kMaxViews scene ranges of
 // about equal body counts, each replayed on a stream of its own. A scene's
 // work never touches another's, so the views only run concurrently: while
 // one view's latency-bound solve runs, another's narrow phase fills the
@@ -895,7 +894,7 @@ static bool build_views(rp_world* w) {
     const DevWorld& d = w->im.d;
     DeviceImage& im = w->im;
     int K = 1;
-    if (d.narrow_group > 1 && d.manifold_group != 1 && !d.has_general) {
+    if (d.narrow_group > 1 && d.manifold_group != 1) {
         int want = w->want_views > 0 ? w->want_views : (d.ns >= 64 ? kAutoViews : 1);
         K = std::max(1, std::min({want, kMaxViews, d.ns}));
     }

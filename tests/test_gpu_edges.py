@@ -79,3 +79,20 @@ def test_scene_of_fixed_bodies_stays_put():
     assert g.error(0) == 0
     g.close()
     _compare(w, frames=30, check_every=10)
+
+
+@pytest.mark.parametrize("lanes,num_scenes", [(1, 3), (4, 3), (8, 3), (16, 3), (8, 67)])
+def test_general_pairs_on_lane_groups_bit_exact(lanes, num_scenes):
+    """Spheres against spheres, hulls and compounds on every lane-group width
+    (one lane: the schedule of worlds without lane groups), and in concurrent
+    views (64 scenes or more)."""
+    world = scenes.batched_mixed(num_scenes, first_seed=11, n_spheres=4, n_cubes=2, n_dumbbells=3)
+    o, g = SimWorld("orc", world), SimWorld("rp", world)
+    assert g.lib.rp_world_set_narrow_group(g.h, lanes) == 0
+    for f in range(90 if num_scenes < 10 else 45):
+        o.step(1)
+        g.step(1)
+        if f % 15 == 14:
+            bad = state_bits_equal(o.state(), g.state())
+            assert not bad, f"frame {f}: differs in {bad}"
+    assert not any(g.error(s) for s in range(num_scenes))
