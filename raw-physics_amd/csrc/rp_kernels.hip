@@ -429,13 +429,11 @@ __device__ __forceinline__ void gjk_epa_pairs(DevWorld& w, const int32_t* list, 
         int r = 0;
         char* work = G > 1 ? w.group_work + (size_t)(blockIdx.x * NG + grp) * GROUP_WORK_BYTES : own;
         bool hit = gjk<G>(h1, h2, sx, err, cycled);
-        if (hit) r = epa<G>(h1, h2, sx, n, pen, err, work);
+        const int used = h1.nv + h2.nv;  // the rest of the pair's LDS slice is free
+        if (hit) r = epa<G>(h1, h2, sx, n, pen, err, work, st + used, stage - used);
         if constexpr (kManifold) {
             int nc = 0;
-            if (r == 1) {
-                int used = h1.nv + h2.nv;  // the rest of the pair's LDS slice is free
-                nc = pair_manifold<G>(w, g, h1, h2, n, err, work, st + used, stage - used);
-            }
+            if (r == 1) nc = pair_manifold<G>(w, g, h1, h2, n, err, work, st + used, stage - used);
             if (gl == 0) w.ncontact[g] = nc;
         }
         if (gl == 0) {
@@ -502,7 +500,8 @@ __global__ void __launch_bounds__(64) k_manifold(DevWorld w, int stage) {
 // leave no room for that, one lane per pair over the pre-transformed vertices
 // with private arrays (G = 1).
 template <int G>
-__global__ void __launch_bounds__(64) k_narrow_general(DevWorld w, int stage) {
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+k_narrow_general(DevWorld w, int stage) {
     extern __shared__ V3 rp_stage[];
     constexpr int NG = 64 / G;
     const int grp = threadIdx.x / G, gl = threadIdx.x & (G - 1);
@@ -880,16 +879,17 @@ __global__ void k_fp64_selftest(const double* a, const double* b, double* out, i
 static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // LDS vertices of a pair's slice in the lane-group kernels: both hulls (`base`
-// vertices at most) and room beside them for the clipping polygons, which
-// otherwise go through the group's working memory on one lane (a pair of the
-// world's largest hulls, or any pair of a world of boxes, had none: 45 000 to
-// 62 000 cycles per manifold instead of 21 000). 8 points per polygon always,
-// up to 16 while eight blocks (two waves per SIMD) still share a CU's 160 KiB,
-// and never beyond the world's LDS limit.
+// vertices at most) and room beside them for the EPA polytope and then the
+// clipping polygons, which otherwise go through the group's working memory
+// (the polygons on one lane: a pair of the world's largest hulls, or any pair
+// of a world of boxes, had no room and took 45 000 to 62 000 cycles per
+// manifold instead of 21 000). 8 points per polygon always, up to 96 vertices
+// (40 faces) while eight blocks (two waves per SIMD) still share a CU's
+// 160 KiB, and never beyond the world's LDS limit.
 static int stage_slice(const DevWorld& w, int group, int base) {
     if (group <= 1) return 0;
     int per = 64 / group * (int)sizeof(V3);
-    int extra = std::max(16, std::min(32, 20 * 1024 / per - base));
+    int extra = std::max(16, std::min(96, 20 * 1024 / per - base));
     return std::max(base, std::min(base + extra, w.lds_limit / per));
 }
 static size_t stage_bytes(int group, int stage) {

@@ -584,13 +584,12 @@ struct EpaPoly {
     }
     // add_edge (epa.cpp:79-110): an edge equal to a listed one, by index or
     // by position, cancels it (swap-remove), else it is appended; false when
-    // the list is full. `dup`: two points of the polytope may be equal; else
-    // positions are equal only where indices are, and are not read.
-    RP_HD bool add_edge(int2 e, uint32_t& err, bool dup = true) {
+    // the list is full.
+    RP_HD bool add_edge(int2 e, uint32_t& err) {
         for (int j = 0; j < ne; ++j) {
             int2 cur = edges[j];
             bool hit = (e.x == cur.x && e.y == cur.y) || (e.x == cur.y && e.y == cur.x);
-            if (!hit && dup) {
+            if (!hit) {
                 V3 c1 = poly[cur.x], c2 = poly[cur.y], e1 = poly[e.x], e2 = poly[e.y];
                 hit = (veq(c1, e1) && veq(c2, e2)) || (veq(c1, e2) && veq(c2, e1));
             }
@@ -603,12 +602,6 @@ struct EpaPoly {
         if (ne == EPA_MAXE) { err |= ERR_EPA_CAPACITY; return false; }
         edges[ne++] = e;
         return true;
-    }
-    // triangle_centroid (epa.cpp:112-116) test: does face i see sp?
-    RP_HD bool sees(int i, V3 sp) const {
-        I3 f = faces[i];
-        V3 c = scl(1.0 / 3.0, add(add(poly[f.y], poly[f.z]), poly[f.x]));
-        return dot(normals[i], sub(sp, c)) > 0.0;
     }
     // One iteration with the support point sp in direction min_n:
     // 1 = converged (n_out, pen_out set), 2 = expanded, -1 = error.
@@ -757,7 +750,32 @@ struct FaceBits {
         w2 |= k == 2 ? b : 0ull;
         w3 |= k == 3 ? b : 0ull;
     }
+    // lowest set flag (EPA_MAXF if none)
+    __device__ int first() const {
+        return w0 ? __ffsll((long long)w0) - 1 : w1 ? 63 + __ffsll((long long)w1) : w2 ? 127 + __ffsll((long long)w2)
+                 : w3 ? 191 + __ffsll((long long)w3) : EPA_MAXF;
+    }
 };
+
+// The polytope of a lane group: in the free end of the pair's LDS slice, or
+// in the group's working memory (the pointers are generic: one copy of the
+// code serves both). Faces and edges hold their point indices in bytes.
+struct GroupPoly {
+    V3 *poly, *normals;
+    double* dist;
+    uint32_t *faces, *edges;
+    int max_v, max_f, max_e;
+    __device__ void bind(char* m, int v, int f, int e) {
+        max_v = v; max_f = f; max_e = e;
+        poly = (V3*)m;
+        normals = poly + v;
+        dist = (double*)(normals + f);
+        faces = (uint32_t*)(dist + f);
+        edges = faces + f;
+    }
+};
+constexpr int GROUP_POLY_FACE_BYTES = sizeof(V3) / 2 + sizeof(V3) + sizeof(double) + 2 * sizeof(uint32_t);
+
 // epa for a lane group (G > 1), with the results of EpaPoly::step. The
 // simplex's four faces are computed side by side, one per lane, in
 // registers: nine of ten resting contacts converge on the first support
@@ -765,21 +783,25 @@ struct FaceBits {
 // these touch no memory but the staged hulls. (Lane 0 used to build the four
 // faces one after another in the group's working memory, about 20 000 cycles
 // per pair; now 3 700. Narrow launch: 4096 scenes of 16 bodies 200 -> 193 us,
-// 150 uneven scenes 243 -> 214, 500 chains of 6 links 181 -> 143.) At the first expansion the
-// polytope moves to the group's working memory; then the lanes test which
-// faces see the support point, compute the new faces' normals and distances,
-// and search the closest face (first minimum), while lane 0 keeps the edge
-// list and the face list's swap-remove order (epa.cpp:165-195). Every lane
-// returns the status and the result; the EPA error bits are lane 0's.
+// 150 uneven scenes 243 -> 214, 500 chains of 6 links 181 -> 143.)
+//
+// At the first expansion the polytope moves to memory: to `spare` (LDS) while
+// it fits there, then to `work`. The lanes test which faces see the support
+// point, look an edge up in the edge list, compute the new faces' normals and
+// distances, and search the closest face (first minimum); faces are removed
+// and edges listed in the sequential order (epa.cpp:165-195). Links that
+// overlap deeply take 2 to 6 expansions, a sphere more. (Lane 0 used to keep
+// the edge and face lists in the working memory alone, comparing positions
+// with every edge: 500 chains of 6 links 131 -> 85 us per narrow launch, 150
+// uneven scenes 193 -> 163.) Every lane returns
+// the status and the result; the EPA error bits are lane 0's.
 template <int G, class View>
 __device__ int epa_group(const View& h1, const View& h2, const Simplex& s, V3& n_out, double& pen_out, uint32_t& err,
-                         char* work) {
-    EpaPoly P;
-    epa_bind(P, work);
-    int gl = (int)(__lane_id() & (G - 1));
-    bool leader = gl == 0;
-    int gbase = (int)__lane_id() & ~(G - 1);
-    int st = 2;
+                         char* work, V3* spare, int spare_n) {
+    const int gl = (int)(__lane_id() & (G - 1));
+    const bool leader = gl == 0;
+    const int gbase = (int)__lane_id() & ~(G - 1);
+    auto group_ballot = [&](bool v) { return (__ballot(v) >> gbase) & ((1ull << G) - 1ull); };
     // lane i (and i + 4, ...): face i of 012, 023, 031, 123
     const int fi = gl & 3;
     const I3 f0 = {fi == 3 ? 1 : 0, fi == 0 ? 1 : fi == 2 ? 3 : 2, fi == 0 ? 2 : fi == 2 ? 1 : 3};
@@ -788,7 +810,7 @@ __device__ int epa_group(const View& h1, const View& h2, const Simplex& s, V3& n
     V3 n0 = v3(0.0, 0.0, 0.0);
     double d0 = 0.0;
     bool ok0 = epa_face(corner(f0.x), corner(f0.y), corner(f0.z), corner, 4, n0, d0);
-    if ((__ballot(!ok0) >> gbase) & 0xFull) {
+    if (group_ballot(!ok0) & 0xFull) {
         if (leader) err |= ERR_EPA_DEGENERATE;
         return -1;
     }
@@ -800,6 +822,9 @@ __device__ int epa_group(const View& h1, const View& h2, const Simplex& s, V3& n
     if (mi0 == NO_SEL) min_n = v3(0.0, 0.0, 0.0);
     int np = 4, nf = 4;
     bool dup = false;  // equal points in the polytope
+    GroupPoly P;
+    P.bind(work, EPA_MAXV, EPA_MAXF, EPA_MAXE);
+    bool lds = false;
     for (int it = 0; it < 100; ++it) {
         V3 sp = support_md<G>(h1, h2, min_n, err);
         double d = dot(min_n, sp);
@@ -808,71 +833,121 @@ __device__ int epa_group(const View& h1, const View& h2, const Simplex& s, V3& n
             pen_out = min_d;
             return 1;
         }
+        int ne = 0;
+        // the polytope to the working memory, if it is not there
+        auto grow = [&] {
+            if (!lds) return;
+            lds = false;
+            GroupPoly Q = P;
+            P.bind(work, EPA_MAXV, EPA_MAXF, EPA_MAXE);
+            group_mem_sync();
+            for (int i = gl; i < np; i += G) P.poly[i] = Q.poly[i];
+            for (int i = gl; i < nf; i += G) {
+                P.normals[i] = Q.normals[i];
+                P.dist[i] = Q.dist[i];
+                P.faces[i] = Q.faces[i];
+            }
+            for (int i = gl; i < ne; i += G) P.edges[i] = Q.edges[i];
+            group_mem_sync();
+        };
         if (it == 0) {
+            // half as many points as faces and a few more, as many edges
+            int f = (spare_n * (int)sizeof(V3) - 6 * (int)sizeof(V3)) / GROUP_POLY_FACE_BYTES;
+            f = f < EPA_MAXE ? f : EPA_MAXE;
+            if (f >= 8) {
+                lds = true;
+                P.bind((char*)spare, f / 2 + 6, f & ~1, f & ~1);
+            }
             if (gl < 4) {
                 P.poly[gl] = corner(gl);
-                P.faces[gl] = f0;
+                P.faces[gl] = (uint32_t)(f0.x | f0.y << 8 | f0.z << 16);
                 P.normals[gl] = n0;
                 P.dist[gl] = d0;
             }
             dup = veq(sa, sb) | veq(sa, sc) | veq(sa, sd) | veq(sb, sc) | veq(sb, sd) | veq(sc, sd);
             group_mem_sync();
         }
+        if (np == P.max_v) grow();
         bool same = false;
         for (int i = gl; i < np; i += G) same |= veq(P.poly[i], sp);
-        dup |= ((__ballot(same) >> gbase) & ((1ull << G) - 1ull)) != 0;
-        int new_idx = np;
+        dup |= group_ballot(same) != 0;
+        const int new_idx = np;
         if (leader) P.poly[np] = sp;
         ++np;
-        // which faces see sp (a property of each face: computed up front)
+        // which faces see sp (triangle_centroid, epa.cpp:112-116; a property
+        // of each face: computed up front)
         FaceBits vis;
         for (int c0 = 0; c0 < nf; c0 += G) {
             int i = c0 + gl;
-            bool v = i < nf && P.sees(i, sp);
-            unsigned long long m = (__ballot(v) >> gbase) & ((1ull << G) - 1ull);
-            vis.or_bits(c0, m);
+            bool v = false;
+            if (i < nf) {
+                uint32_t f = P.faces[i];
+                V3 c = scl(1.0 / 3.0, add(add(P.poly[f >> 8 & 255], P.poly[f >> 16]), P.poly[f & 255]));
+                v = dot(P.normals[i], sub(sp, c)) > 0.0;
+            }
+            vis.or_bits(c0, group_ballot(v));
         }
-        // lane 0: edges of the visible faces and the swap-removes, in order
-        int ne = 0;
-        if (leader) {
-            P.nf = nf;
-            P.ne = 0;
-            for (int i = 0; i < P.nf; ++i) {
-                if (vis.get(i)) {
-                    I3 f = P.faces[i];
-                    if (!P.add_edge(make_int2(f.x, f.y), err, dup) || !P.add_edge(make_int2(f.y, f.z), err, dup) ||
-                        !P.add_edge(make_int2(f.z, f.x), err, dup)) {
-                        st = -1;
-                        break;
+        // add_edge (epa.cpp:79-110): an edge equal to a listed one, by index
+        // or (only where points are equal) by position, cancels it
+        // (swap-remove), else it is appended; false when the list is full
+        auto add_edge = [&](uint32_t x, uint32_t y) {
+            for (int c0 = 0; c0 < ne; c0 += G) {
+                int j = c0 + gl;
+                bool hit = false;
+                if (j < ne) {
+                    uint32_t cur = P.edges[j], cx = cur & 255, cy = cur >> 8;
+                    hit = (x == cx && y == cy) || (x == cy && y == cx);
+                    if (dup && !hit) {
+                        V3 c1 = P.poly[cx], c2 = P.poly[cy], e1 = P.poly[x], e2 = P.poly[y];
+                        hit = (veq(c1, e1) && veq(c2, e2)) || (veq(c1, e2) && veq(c2, e1));
                     }
-                    --P.nf;
-                    P.faces[i] = P.faces[P.nf];
-                    P.dist[i] = P.dist[P.nf];
-                    P.normals[i] = P.normals[P.nf];
-                    vis.put(i, vis.get(P.nf));
-                    --i;
+                }
+                unsigned long long m = group_ballot(hit);
+                if (m) {
+                    --ne;
+                    if (leader) P.edges[c0 + __ffsll((long long)m) - 1] = P.edges[ne];
+                    group_mem_sync();
+                    return true;
                 }
             }
-            nf = P.nf;
-            ne = P.ne;
-        }
-        st = group_bcast<G>(st);
-        if (st != 2) return st;
-        nf = group_bcast<G>(nf);
-        ne = group_bcast<G>(ne);
+            if (ne == P.max_e) grow();
+            if (ne == P.max_e) return false;
+            if (leader) P.edges[ne] = x | y << 8;
+            ++ne;
+            group_mem_sync();
+            return true;
+        };
         group_mem_sync();
+        // the visible faces' edges and the swap-removes, in order
+        // (epa.cpp:191-195: faces, distances and normals together)
+        for (int i = vis.first(); i < nf; i = vis.first()) {
+            uint32_t f = P.faces[i], fx = f & 255, fy = f >> 8 & 255, fz = f >> 16;
+            if (!add_edge(fx, fy) || !add_edge(fy, fz) || !add_edge(fz, fx)) {
+                if (leader) err |= ERR_EPA_CAPACITY;
+                return -1;
+            }
+            --nf;
+            if (gl < 3) ((double*)&P.normals[i])[gl] = ((double*)&P.normals[nf])[gl];
+            if (gl == 3) {
+                P.dist[i] = P.dist[nf];
+                P.faces[i] = P.faces[nf];
+            }
+            vis.put(i, vis.get(nf) && i < nf);
+            vis.put(nf, false);
+            group_mem_sync();
+        }
+        if (nf + ne > P.max_f) grow();
         // the new faces (edge i, new point) at nf + i; the sequential loop
         // stops at the first full list or degenerate face, in that order
         int room = EPA_MAXF - nf;
         int nnew = ne < room ? ne : room;
         int first_bad = nnew;
         for (int i = gl; i < nnew; i += G) {
-            int2 e = P.edges[i];
-            I3 f = {e.x, e.y, new_idx};
+            uint32_t e = P.edges[i];
             V3 n;
             double fd;
-            bool ok = epa_face(f, P.poly, np, n, fd);
-            P.faces[nf + i] = f;
+            bool ok = epa_face(P.poly[e & 255], P.poly[e >> 8], sp, [&](int k) { return P.poly[k]; }, np, n, fd);
+            P.faces[nf + i] = e | (uint32_t)new_idx << 16;
             P.normals[nf + i] = n;
             P.dist[nf + i] = fd;
             if (!ok && i < first_bad) first_bad = i;
@@ -908,7 +983,7 @@ __device__ int epa_group(const View& h1, const View& h2, const Simplex& s, V3& n
 // On one lane (G = 1) with its working memory, or on a lane group (epa_group).
 template <int G = 1, class View = HullView>
 RP_HD int epa(const View& h1, const View& h2, const Simplex& s, V3& n_out, double& pen_out, uint32_t& err,
-              char* work) {
+              char* work, V3* spare = nullptr, int spare_n = 0) {
     if constexpr (G == 1) {
         EpaPoly P;
         epa_bind(P, work);
@@ -920,7 +995,7 @@ RP_HD int epa(const View& h1, const View& h2, const Simplex& s, V3& n_out, doubl
         }
         return 0;
     } else {
-        return epa_group<G>(h1, h2, s, n_out, pen_out, err, work);
+        return epa_group<G>(h1, h2, s, n_out, pen_out, err, work, spare, spare_n);
     }
 }
 
@@ -1461,7 +1536,7 @@ RP_HD int collider_contacts(const HullTables& T, const ColView& c1, const ColVie
             if (cycled) flags |= PAIR_GJK_CYCLE;
             return 0;
         }
-        if (epa<G>(c1, c2, s, n, pen, err, work) != 1) {
+        if (epa<G>(c1, c2, s, n, pen, err, work, spare, spare_n) != 1) {
             flags |= PAIR_EPA_FAIL;
             return 0;
         }
