@@ -303,9 +303,10 @@ class World:
 
     def set_colour_launches(self, classes: int):
         """Large scenes: colour classes solved one launch each before the
-        one-block tail (0..25, default 6; identical results)."""
+        one-block tail (0..64; the default follows earlier frames' class
+        sizes; identical results)."""
         if self.lib.rp_world_set_colour_launches(self.h, classes) != 0:
-            raise ValueError(f"colour launches must be 0..25, not {classes}")
+            raise ValueError(f"colour launches must be 0..64, not {classes}")
 
     def set_solve_lanes(self, lanes_per_scene: int):
         if self.lib.rp_world_set_solve_lanes(self.h, lanes_per_scene) != 0:

@@ -30,7 +30,8 @@ struct DevWorld {
     int stage_small;                // LDS vertices per pair of that list: 2 x small_nv
     int small_bodies;               // most bodies of a scene that is not large
     int solve_lanes;                // lanes per scene in the solve: 64, 32 or 16
-    int big_launch_classes;         // large scenes: colour classes solved one launch each, the rest in one block
+    int big_launch_classes;         // large scenes: colour classes solved one launch each, the rest in one block (BIG_AUTO: big_classes)
+    int big_classes, big_rounds;    // the host's present choice of launched classes and colour rounds
     // scenes
     const int32_t* scene_body_off;  // [ns+1]
     const int32_t* scene_pair_base; // [ns+1]  candidate pair capacity prefix: n(n-1)/2 per scene
@@ -107,11 +108,18 @@ constexpr int BIG_COLOURS = 63;             // parallel colours (one 64-bit mask
 constexpr int BIG_SERIAL = BIG_COLOURS;     // class solved one item after another, in item order
 constexpr int BIG_CLASSES = BIG_COLOURS + 1;
 constexpr int BIG_COLOUR_ROUNDS = 64;       // Jones-Plassmann rounds per frame (launches end at once when all are coloured)
-// Default: every class launched one by one over the device (a settled
-// 10^5-body pile leaves about 100 000 items beyond the first 16 colours,
-// 4 ms per substep on the one-block tail; an empty class's launch costs a
-// few microseconds).
-constexpr int BIG_LAUNCH_CLASSES = BIG_CLASSES;
+// Colour classes launched one by one over the device, the rest on one block
+// with a block barrier between classes. By default the host chooses how many,
+// before a frame is captured or launched, from what an earlier frame's
+// colouring left in BigScene::hint: the classes up to the last of more than
+// BIG_TAIL_ITEMS items. A launch costs about 3 us even where the class is
+// empty (128 launches per substep; 20000 falling bodies: 6.0 ms per frame with
+// every class launched, 2.6 with 8), while on one block a settled pile's 26
+// classes beyond the first 24 would cost milliseconds. The colour rounds
+// launched follow the same way. Any choice gives the same bits.
+constexpr int BIG_AUTO = -1;
+constexpr int BIG_TAIL_T = 512;             // threads of that block: 256 items side by side
+constexpr int BIG_TAIL_ITEMS = 512;
 constexpr int LARGE_CHUNK = 256;            // bodies per wave in a large body's pair scan
 struct BigScene {
     int s, b0, n;                // scene, first body, bodies
@@ -133,7 +141,8 @@ struct BigScene {
     int32_t* bi_start;           // [n + 1] body -> items CSR
     int32_t* bi_cursor;          // [n]
     int32_t* bi_items;           // [2 item_cap]
-    int32_t* remaining;          // [1] uncoloured items
+    int32_t* remaining;          // [2] uncoloured items; rounds that coloured some
+    int32_t* hint;               // [2] host memory: classes worth a launch, colour rounds of the last frame
     int32_t* scan_blocks;        // [scan block sums]
 };
 

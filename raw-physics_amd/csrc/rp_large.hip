@@ -445,7 +445,8 @@ __global__ void k_big_csr_count(DevWorld w, BigScene b, int collisions) {
         colour[t] = -1;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *b.remaining = K;
+        b.remaining[0] = K;
+        b.remaining[1] = 0;
         if (big_items(w, b, collisions) > b.item_cap) atomicOr(&w.scene_err[b.s], (uint32_t)ERR_SOLVER_CAPACITY);
     }
 }
@@ -465,47 +466,72 @@ __global__ void k_big_csr_fill(DevWorld w, BigScene b, int collisions) {
 // no coloured neighbour has. Reads see only the previous round, so the
 // colouring does not depend on thread timing, and two neighbours never
 // colour in the same round (one of them has the lower priority).
-__global__ void k_big_colour_round(DevWorld w, BigScene b, int collisions, const int* __restrict__ src,
+// The colour of uncoloured item t after the round, or -1.
+__device__ __forceinline__ int colour_item(const DevWorld& w, const BigScene& b, const int* src, int t) {
+    uint32_t pt = item_priority(t);
+    int2 bb = item_free_bodies(w, b, t);
+    uint64_t used = 0;
+    for (int side = 0; side < 2; ++side) {
+        int body = side ? bb.y : bb.x;
+        if (body < 0 || (side && body == bb.x)) continue;
+        for (int m = b.bi_start[body]; m < b.bi_start[body + 1]; ++m) {
+            int u = b.bi_items[m];
+            if (u == t) continue;
+            int cu = src[u];
+            if (cu < 0) {
+                uint32_t pu = item_priority(u);
+                if (pu > pt || (pu == pt && u > t)) return -1;
+            } else if (cu < 64) {
+                used |= 1ull << cu;
+            }
+        }
+    }
+    int c = __ffsll((unsigned long long)~used) - 1;
+    return c < 0 || c >= BIG_COLOURS ? BIG_SERIAL : c;
+}
+__global__ void k_big_colour_round(DevWorld w, BigScene b, int collisions, int round, const int* __restrict__ src,
                                    int* __restrict__ dst) {
     int K = min(big_items(w, b, collisions), b.item_cap);
     // all coloured: copy. (The count falls during this launch too, but it
     // reaches 0 only once every item is coloured in src or by a block that
     // has run, so a block that sees 0 late copies what it would have kept.)
     bool done = __hip_atomic_load(b.remaining, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+    if (!done && blockIdx.x == 0 && threadIdx.x == 0) b.remaining[1] = round + 1;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < K; t += gridDim.x * blockDim.x) {
         int ct = src[t];
-        if (done || ct >= 0) {
-            dst[t] = ct;
-            continue;
+        if (!done && ct < 0) {
+            ct = colour_item(w, b, src, t);
+            if (ct >= 0) atomicSub(b.remaining, 1);
         }
-        uint32_t pt = item_priority(t);
-        int2 bb = item_free_bodies(w, b, t);
-        bool best = true;
-        uint64_t used = 0;
-        for (int side = 0; side < 2 && best; ++side) {
-            int body = side ? bb.y : bb.x;
-            if (body < 0 || (side && body == bb.x)) continue;
-            for (int m = b.bi_start[body]; m < b.bi_start[body + 1]; ++m) {
-                int u = b.bi_items[m];
-                if (u == t) continue;
-                int cu = src[u];
-                if (cu < 0) {
-                    uint32_t pu = item_priority(u);
-                    if (pu > pt || (pu == pt && u > t)) { best = false; break; }
-                } else if (cu < 64) {
-                    used |= 1ull << cu;
-                }
-            }
-        }
-        if (!best) {
-            dst[t] = -1;
-            continue;
-        }
-        int c = __ffsll((unsigned long long)~used) - 1;
-        if (c < 0 || c >= BIG_COLOURS) c = BIG_SERIAL;
-        dst[t] = c;
-        atomicSub(b.remaining, 1);
+        dst[t] = ct;
     }
+}
+// The rounds from `round` (even) on that a frame still needs, on one block:
+// none where the launched rounds coloured every item.
+__global__ void __launch_bounds__(1024) k_big_colour_rest(DevWorld w, BigScene b, int collisions, int round, int* colour,
+                                                          int* spare) {
+    int K = min(big_items(w, b, collisions), b.item_cap);
+    __shared__ int left;
+    for (; round < BIG_COLOUR_ROUNDS; ++round) {
+        __syncthreads();
+        if (threadIdx.x == 0) left = __hip_atomic_load(b.remaining, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (left == 0) break;
+        if (threadIdx.x == 0) b.remaining[1] = round + 1;
+        const int* src = (round & 1) ? spare : colour;
+        int* dst = (round & 1) ? colour : spare;
+        for (int t = threadIdx.x; t < K; t += blockDim.x) {
+            int ct = src[t];
+            if (ct < 0) {
+                ct = colour_item(w, b, src, t);
+                if (ct >= 0) atomicSub(b.remaining, 1);
+            }
+            dst[t] = ct;
+        }
+    }
+    __syncthreads();
+    if (round & 1)
+        for (int t = threadIdx.x; t < K; t += blockDim.x) colour[t] = spare[t];
 }
 
 // Items still uncoloured join the serial class; class sizes and starts.
@@ -523,12 +549,16 @@ __global__ void k_big_classes(DevWorld w, BigScene b, int collisions) {
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        int run = 0, used = 0;
+        int run = 0, used = 0, lead = 0;
         for (int c = 0; c < BIG_CLASSES; ++c) {
             ls[c] = run;
             run += cnt[c];
             if (cnt[c]) used = c + 1;
+            if (c != BIG_SERIAL && cnt[c] > BIG_TAIL_ITEMS) lead = c + 1;
         }
+        // what later frames plan their launches by (host memory)
+        b.hint[0] = lead;
+        b.hint[1] = b.remaining[1];
         ls[BIG_CLASSES] = run;
         w.scene_nlevels[b.s] = used;
     }
@@ -596,9 +626,12 @@ void big_colour(const DevWorld& w, const BigScene& b, bool collisions, hipStream
     static_assert(BIG_COLOUR_ROUNDS % 2 == 0, "the last colour round must write item_level");
     int* colour = w.item_level + b.item_base;
     int* spare = w.item_order + b.item_base;
-    for (int r = 0; r < BIG_COLOUR_ROUNDS; ++r)
-        hipLaunchKernelGGL(k_big_colour_round, dim3(gi), dim3(256), 0, st, w, b, co, (r & 1) ? spare : colour,
+    int rounds = std::min(std::max(w.big_rounds & ~1, 2), BIG_COLOUR_ROUNDS);
+    for (int r = 0; r < rounds; ++r)
+        hipLaunchKernelGGL(k_big_colour_round, dim3(gi), dim3(256), 0, st, w, b, co, r, (r & 1) ? spare : colour,
                            (r & 1) ? colour : spare);
+    if (rounds < BIG_COLOUR_ROUNDS)
+        hipLaunchKernelGGL(k_big_colour_rest, dim3(1), dim3(1024), 0, st, w, b, co, rounds, colour, spare);
     hipLaunchKernelGGL(k_big_classes, dim3(1), dim3(1024), 0, st, w, b, co);
     hipLaunchKernelGGL(k_big_cursor, dim3(1), dim3(64), 0, st, w, b);
     hipLaunchKernelGGL(k_big_serial_flags, dim3(gi), dim3(256), 0, st, w, b, co);
@@ -643,7 +676,7 @@ __global__ void __launch_bounds__(64) k_big_class(DevWorld w, BigScene b, double
 // Colour classes c0.. and then the serial class, on one block: a block
 // barrier between classes instead of a launch per class.
 template <bool kExt, bool kVel>
-__global__ void __launch_bounds__(1024) k_big_tail(DevWorld w, BigScene b, double h, int c0) {
+__global__ void __launch_bounds__(BIG_TAIL_T) k_big_tail(DevWorld w, BigScene b, double h, int c0) {
     const int* ls = w.item_lstart + b.item_base + b.s;
     const int* order = w.item_order + b.item_base;
     const int2* bodies = w.item_bodies + b.item_base;
@@ -674,21 +707,21 @@ void big_solve(const DevWorld& w, const BigScene& b, const FrameParams& fp, hipS
     bool ext = w.n_ext > 0;
     if (ext) hipLaunchKernelGGL(k_big_ext_zero, dim3(grid_for(w.n_ext, 256)), dim3(256), 0, st, w, b);
     // classes 0..L-1 one launch each (the large ones), the rest on one block
-    int L = std::min(std::max(w.big_launch_classes, 0), BIG_CLASSES);
+    int L = std::min(w.big_launch_classes >= 0 ? w.big_launch_classes : w.big_classes, BIG_CLASSES);
     for (unsigned it = 0; it < fp.iters; ++it) {
         for (int c = 0; c < L; ++c) {
             if (ext) hipLaunchKernelGGL((k_big_class<true, false>), dim3(gi), dim3(64), 0, st, w, b, fp.h, c);
             else hipLaunchKernelGGL((k_big_class<false, false>), dim3(gi), dim3(64), 0, st, w, b, fp.h, c);
         }
         if (L < BIG_CLASSES) {
-            if (ext) hipLaunchKernelGGL((k_big_tail<true, false>), dim3(1), dim3(1024), 0, st, w, b, fp.h, L);
-            else hipLaunchKernelGGL((k_big_tail<false, false>), dim3(1), dim3(1024), 0, st, w, b, fp.h, L);
+            if (ext) hipLaunchKernelGGL((k_big_tail<true, false>), dim3(1), dim3(BIG_TAIL_T), 0, st, w, b, fp.h, L);
+            else hipLaunchKernelGGL((k_big_tail<false, false>), dim3(1), dim3(BIG_TAIL_T), 0, st, w, b, fp.h, L);
         }
     }
     hipLaunchKernelGGL(k_big_velocity_update, dim3(grid_for(b.n, 256)), dim3(256), 0, st, w, b, fp.h);
     for (int c = 0; c < L; ++c)
         hipLaunchKernelGGL((k_big_class<false, true>), dim3(gi), dim3(64), 0, st, w, b, fp.h, c);
-    if (L < BIG_CLASSES) hipLaunchKernelGGL((k_big_tail<false, true>), dim3(1), dim3(1024), 0, st, w, b, fp.h, L);
+    if (L < BIG_CLASSES) hipLaunchKernelGGL((k_big_tail<false, true>), dim3(1), dim3(BIG_TAIL_T), 0, st, w, b, fp.h, L);
 }
 
 }  // namespace rp

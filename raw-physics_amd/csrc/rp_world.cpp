@@ -328,6 +328,7 @@ struct HostWorld {
 struct DeviceImage {
     DevWorld d;
     std::vector<BigScene> big;  // large scenes (device buffers in allocs)
+    int32_t* big_hint = nullptr;  // their BigScene::hint, pinned
     std::vector<void*> allocs;
     std::vector<int32_t> body_tv_off;  // host copy for inspection
     std::vector<int32_t> pair_base;    // host copy of scene_pair_base
@@ -362,6 +363,8 @@ struct DeviceImage {
     void release() {
         for (void* p : allocs) (void)hipFree(p);
         allocs.clear();
+        if (big_hint) (void)hipHostFree(big_hint);
+        big_hint = nullptr;
         if (d.group_work) (void)hipFree(d.group_work);
         d.group_work = nullptr;
         d.group_work_slots = 0;
@@ -566,7 +569,17 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
     // lanes: 64 scenes 1.54 / 1.56 / 1.77, 2048 scenes 2.68 / 2.52 / 2.76,
     // 4096 scenes 4.17 / 3.89 / 4.22, 8192 scenes 6.81 / 6.23 / 6.15)
     d.solve_lanes = d.ns < 1536 || d.small_bodies > 64 ? 64 : d.ns < 8192 ? 32 : 16;
-    d.big_launch_classes = BIG_LAUNCH_CLASSES;
+    d.big_launch_classes = BIG_AUTO;
+    d.big_classes = BIG_CLASSES;
+    d.big_rounds = BIG_COLOUR_ROUNDS;
+    if (!im.big.empty()) {
+        RP_CHECK(hipHostMalloc((void**)&im.big_hint, 2 * im.big.size() * sizeof(int32_t)));
+        for (size_t k = 0; k < im.big.size(); ++k) {
+            im.big[k].hint = im.big_hint + 2 * k;
+            im.big[k].hint[0] = BIG_CLASSES;
+            im.big[k].hint[1] = BIG_COLOUR_ROUNDS;
+        }
+    }
 
     bool ok = true;
     ok &= im.upload(d.scene_body_off, hw.scene_body_off);
@@ -662,7 +675,7 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
         ok &= im.alloc(bs.bi_start, (size_t)bs.n + 1);
         ok &= im.alloc(bs.bi_cursor, (size_t)bs.n);
         ok &= im.alloc(bs.bi_items, 2 * (size_t)bs.item_cap);
-        ok &= im.alloc(bs.remaining, 1);
+        ok &= im.alloc(bs.remaining, 2);
         int64_t scan_n = std::max<int64_t>({tmp_n, (int64_t)bs.T, (int64_t)bs.n + 1, nlc + 1});
         ok &= im.alloc(bs.scan_blocks, (size_t)scan_block_count(scan_n));
     }
@@ -973,9 +986,35 @@ static void drop_graphs(rp_world* w) {
         }
 }
 
+// How many colour classes and colour rounds of the large scenes to launch one
+// by one (BIG_AUTO), from the hints of the last frames that have run. The
+// choice moves in steps and down only by half, so that a captured frame is
+// kept while the scenes change little.
+static void plan_big(rp_world* w) {
+    DevWorld& d = w->im.d;
+    if (w->im.big.empty()) return;
+    int lead = 0, rounds = 0;
+    for (const BigScene& b : w->im.big) {
+        lead = std::max(lead, (int)__atomic_load_n(b.hint, __ATOMIC_RELAXED));
+        rounds = std::max(rounds, (int)__atomic_load_n(b.hint + 1, __ATOMIC_RELAXED));
+    }
+    auto step = [](int n, std::initializer_list<int> steps) {
+        for (int s : steps)
+            if (n <= s) return s;
+        return 64;
+    };
+    int classes = step(lead, {4, 8, 12, 16, 24, 32, 48}), rnd = step(rounds, {8, 16, 24, 32, 48});
+    bool move = classes > d.big_classes || 2 * classes <= d.big_classes || rnd > d.big_rounds || 2 * rnd <= d.big_rounds;
+    if (!move) return;
+    d.big_classes = classes;
+    d.big_rounds = rnd;
+    ++w->sched_gen;
+}
+
 // The graphs of one frame for these parameters and the current schedules,
 // captured once per view and reused while they do not change.
 static hipError_t frame_graph(rp_world* w, const FrameParams& fp) {
+    plan_big(w);
     if (w->nviews > 0 && w->view_exec[0] && same_params(w->graph_fp, fp) && w->graph_gen == w->sched_gen)
         return hipSuccess;
     (void)hipStreamSynchronize(w->stream);
@@ -1070,6 +1109,8 @@ static uint32_t world_run(rp_world* w, const FrameParams& fp, uint32_t frames, b
             for (int k = 1; e == hipSuccess && k < w->nviews; ++k) e = hipStreamWaitEvent(w->view_stream[k], w->fork_ev, 0);
         }
         for (uint32_t f = 0; e == hipSuccess && f < frames; ++f) {
+            // a long run looks at the large scenes again once per chunk
+            if (f > 0 && f % kFramesPerChunk == 0 && !w->im.big.empty() && w->nviews == 1) e = frame_graph(w, fp);
             for (int k = 0; e == hipSuccess && k < w->nviews; ++k) {
                 e = hipGraphLaunch(w->view_exec[k], w->view_stream[k]);
                 if (e == hipSuccess) e = chunk_mark(w, f, k, w->view_stream[k]);
@@ -1087,6 +1128,7 @@ static uint32_t world_run(rp_world* w, const FrameParams& fp, uint32_t frames, b
     }
     for (uint32_t f = 0; f < frames; ++f) {
         w->timer.used = 0;
+        plan_big(w);
         hipError_t e = launch_frame(w->im.d, fp, w->stream, &w->timer, w->im.big.data(), (int)w->im.big.size(),
                                     fp.record ? &w->stage : nullptr);
         if (e == hipSuccess && !w->timer.on) e = chunk_mark(w, f, 0, w->stream);
@@ -1184,6 +1226,7 @@ uint32_t rp_world_step_noalloc(rp_world* w, double dt, uint32_t frames, uint32_t
     // the world's kernels with the lane-group working memory in the static
     // array; the narrow-phase grids are capped to the groups it holds (lane
     // groups take the live pairs in grid-stride order: identical results)
+    plan_big(w);
     DevWorld d = w->im.d;
     int64_t slots = (int64_t)(NOALLOC_SCRATCH_BYTES / GROUP_WORK_BYTES);
     if (d.narrow_group > 1) d.narrow_blocks = (int)std::min<int64_t>(d.narrow_blocks, slots / (64 / d.narrow_group));

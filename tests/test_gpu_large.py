@@ -225,3 +225,28 @@ def test_large_scene_full_size_frames_0_1():
     g.set_state(init)
     g.step(2)
     assert not state_bits_equal(g.state(), st)
+
+
+@pytest.mark.parametrize("iters", [1, 2])
+def test_stale_launch_plan_gives_identical_bits(iters):
+    """The colour classes and rounds launched follow an earlier frame's: a
+    world that has seen falling bodies only (few of both) and is then set to a
+    pile finishes its colouring and its classes on one block, with the bits of
+    a world that launches every class."""
+    w = _large(True)
+    pile = SimWorld("rp", w)
+    pile.step(60)
+    st = pile.state()
+    got = []
+    for classes in (None, 64):
+        g = SimWorld("rp", w)
+        if classes is not None:
+            assert g.lib.rp_world_set_colour_launches(g.h, classes) == 0
+        for _ in range(6):
+            g.step(1)
+        g.set_state(st)
+        g.step(1, iters=iters)
+        g.step(2, iters=iters)
+        assert g.error(0) == 0
+        got.append(g.state())
+    assert not state_bits_equal(got[0], got[1])
