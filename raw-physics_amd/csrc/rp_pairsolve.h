@@ -34,6 +34,7 @@ struct HalfPos {
     double im;   // inverse mass; negated on the second lane (its impulses are)
     M3 Iinv;
     double mu_s;
+    double iinv_max;  // bound on Iinv's eigenvalues; infinite unless the rotation is a unit quaternion
     bool fixed;
 };
 struct HalfVel {
@@ -75,8 +76,18 @@ __device__ __forceinline__ double abs_mass(const HalfPos& e) { return second_lan
 
 // collision_constraint_solve (pbd.cpp:107-154). `I` is the world inverse
 // inertia at e.q when `fresh`: it is computed once per change of the rotation
-// (the second preparation's value serves the item's next contact unless
-// friction moved the body), and not at all for a separated contact.
+// and not at all for a separated contact.
+//
+// Static friction needs the generalized masses after the normal correction,
+// whose values matter only if lambda_t + dl > mu_s lambda_n, that is, with
+// lambda_t <= 0, only if the masses' sum W' grew to c / (mu_s |lambda_n|), about
+// W / mu_s. It hardly changes: in the body's frame the lever arm is fixed and
+// the normal turns by at most the angle |a| of the correction, so by the
+// triangle inequality in the tensor's norm
+//     sqrt(w' - im) <= sqrt(w - im) + sqrt(iinv_max) |r| |a|,
+// hence w' <= im + 1.1 (w - im) + 11 iinv_max |r|^2 |a|^2. Where that bound
+// decides (with margins far above rounding), the second preparation, a fifth
+// of the contact's operations, is left out; its result would not be used.
 __device__ __forceinline__ void pair_collision(V3 r_lc, V3 n, double& lambda_n, double& lambda_t, HalfPos& e, M3& I,
                                                bool& fresh, double mu_s, double h, uint32_t& err) {
     V3 r = q_rot(e.q, r_lc);
@@ -89,18 +100,31 @@ __device__ __forceinline__ void pair_collision(V3 r_lc, V3 n, double& lambda_n, 
     double tc = 0.0 / (h * h);
     bool any = !(c <= 1e-50);
     V3 dir = v3(dx.x / c, dx.y / c, dx.z / c);
-    double dl = 0.0;
+    double dl = 0.0, im = abs_mass(e);
     if (any) {
-        dl = pair_dlambda(half_mass(abs_mass(e), r, I, dir), c, tc, lambda_n, err);
-        half_apply(e, r, I, dl, dir);
+        V3 u = cross(r, dir);
+        double wu = dot(u, m3_mulv(I, u));
+        dl = pair_dlambda(im + wu, c, tc, lambda_n, err);
+        V3 imp = scl(dl, dir);
+        V3 a = m3_mulv(I, cross(r, imp));
+        if (!e.fixed) e.x = add(e.x, scl(e.im, imp));
+        half_rotate(e, a);
+        fresh = false;
+        double top = im + 1.1 * wu + 11.0 * e.iinv_max * dot(r, r) * dot(a, a);
+        top += pair_other(top);
+        lambda_n += dl;
+        if (tc == 0.0 && lambda_t <= 0.0 && lambda_n < 0.0 && top > 0.0 && mu_s >= 0.0 &&
+            mu_s * -lambda_n * top <= c * (1.0 - 1e-9))
+            return;
+    } else {
+        lambda_n += dl;
     }
-    lambda_n += dl;
     r = q_rot(e.q, r_lc);
     I = world_tensor(e.q, e.Iinv);
     fresh = true;
     p = add(e.x, r);
     dl = 0.0;
-    if (any) dl = pair_dlambda(half_mass(abs_mass(e), r, I, dir), c, tc, lambda_t, err);
+    if (any) dl = pair_dlambda(half_mass(im, r, I, dir), c, tc, lambda_t, err);
     if (lambda_t + dl > mu_s * lambda_n) {
         V3 dp_own = sub(p, add(e.px, q_rot(e.pq, r_lc)));
         V3 dp = sub(pair_first(dp_own), pair_second(dp_own));
@@ -278,6 +302,10 @@ __device__ __forceinline__ void solve_item_pos(const DevWorld& w, Body* body, in
     e.im = second ? -g.inv_mass : g.inv_mass;
     e.Iinv = g.Iinv;
     e.mu_s = g.mu_s;
+    {
+        double qq = e.q.x * e.q.x + e.q.y * e.q.y + e.q.z * e.q.z + e.q.w * e.q.w;
+        e.iinv_max = fabs(qq - 1.0) <= 1e-9 ? g.iinv_max : HUGE_VAL;
+    }
     e.fixed = g.fixed;
     if (kExt && t.code < 0) {
         pair_external(w.ext[~t.code], w.ext_lambda + 3 * (~t.code), e, h, err);

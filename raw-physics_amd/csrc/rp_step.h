@@ -7,6 +7,7 @@
 // an error bit if a capacity would be exceeded.
 #pragma once
 #include <float.h>
+#include <math.h>
 #include "rp_math.h"
 
 namespace rp {
@@ -23,8 +24,36 @@ template <class S> struct alignas(16) BodyT {  // one record per body (464 bytes
     S mu_s, mu_d, e, radius;
     V3T<S> F, T;                                 // external force / torque of the frame
     int32_t fixed, active;
+    S iinv_max;                                  // bound on the eigenvalues of Iinv (inverse_inertia_bound)
 };
 using Body = BodyT<double>;
+
+// A bound on the eigenvalues of an inverse inertia tensor (its largest
+// absolute row sum), or infinity where it is not symmetric positive
+// definite or zero, so that nothing is concluded from it.
+inline double inverse_inertia_bound(const M3& A) {
+    double top = 0.0;
+    bool zero = true;
+    for (int i = 0; i < 3; ++i) {
+        double row = 0.0;
+        for (int j = 0; j < 3; ++j) {
+            row += fabs(A.m[i][j]);
+            zero &= A.m[i][j] == 0.0;
+        }
+        top = row > top ? row : top;
+    }
+    if (zero) return 0.0;
+    bool symmetric = true;
+    for (int i = 0; i < 3; ++i)
+        for (int j = 0; j < i; ++j) symmetric &= fabs(A.m[i][j] - A.m[j][i]) <= 1e-12 * top;
+    double m2 = A.m[0][0] * A.m[1][1] - A.m[0][1] * A.m[1][0];
+    double det = A.m[0][0] * (A.m[1][1] * A.m[2][2] - A.m[1][2] * A.m[2][1]) -
+                 A.m[0][1] * (A.m[1][0] * A.m[2][2] - A.m[1][2] * A.m[2][0]) +
+                 A.m[0][2] * (A.m[1][0] * A.m[2][1] - A.m[1][1] * A.m[2][0]);
+    // (margins above the rounding of the minors)
+    bool definite = A.m[0][0] > 0.0 && m2 > 1e-9 * top * top && det > 1e-9 * top * top * top;
+    return symmetric && definite && top < DBL_MAX ? top : HUGE_VAL;
+}
 
 // A collision constraint as built by clipping_contact_to_collision_constraint
 // (pbd.cpp:408-424) plus its multipliers.

@@ -696,6 +696,7 @@ static Body make_body(const HostWorld& hw, int c0, int nc, V3 x, Q4 q, V3 v, V3 
         e.I = colliders_inertia(hw.hulls, hw.cols.data() + c0, nc, mass, err);
         if (!m3_inverse(e.I, e.Iinv)) err |= ERR_HULL;
     }
+    e.iinv_max = inverse_inertia_bound(e.Iinv);
     e.active = 1;
     e.deact = 0.0;
     e.mu_s = mat[0];
@@ -1495,6 +1496,7 @@ uint32_t rp_world_set_body_params(rp_world* w, const double* mass, const double*
             e.I = h.I = colliders_inertia(w->hw.hulls, w->hw.cols.data() + c0, nc, mass[b], err);
             if (!m3_inverse(e.I, e.Iinv)) err |= ERR_HULL;
             h.Iinv = e.Iinv;
+            e.iinv_max = h.iinv_max = inverse_inertia_bound(e.Iinv);
         }
     }
     if (!upload_bodies(w)) return RP_ERR_RUNTIME;
@@ -1941,6 +1943,7 @@ static Body entity_body(const rp_entity* e) {
     b.inv_mass = e->inverse_mass;
     memcpy(b.I.m, e->inertia_tensor.data, 72);
     memcpy(b.Iinv.m, e->inverse_inertia_tensor.data, 72);
+    b.iinv_max = inverse_inertia_bound(b.Iinv);
     b.mu_s = e->static_friction_coefficient;
     b.mu_d = e->dynamic_friction_coefficient;
     b.e = e->restitution_coefficient;

@@ -96,3 +96,23 @@ def test_general_pairs_on_lane_groups_bit_exact(lanes, num_scenes):
             bad = state_bits_equal(o.state(), g.state())
             assert not bad, f"frame {f}: differs in {bad}"
     assert not any(g.error(s) for s in range(num_scenes))
+
+
+@pytest.mark.parametrize("mu", [0.0, 0.4, 0.97, 1.6])
+def test_static_friction_bit_exact(mu):
+    """Thin boxes (inertia of very different axes) tumbling onto each other at
+    friction coefficients on both sides of what the bound on the generalized
+    masses can decide without computing them, in one and in three iterations."""
+    w = scenes.World(name="thin_boxes")
+    cube = w.shape(scenes.cube_corners())
+    rng = np.random.default_rng(17)
+    for _ in range(3):
+        scenes._floor(w, material=(mu, 0.5 * mu, 0.0))
+        for k in range(7):
+            q = rng.normal(size=4)
+            w.add_body(cube, (0.9, 0.15, 0.4), (rng.uniform(-1.0, 1.0), 0.5 + 1.3 * k, rng.uniform(-1.0, 1.0)),
+                       tuple(q / np.linalg.norm(q)), mass=1.0, material=(mu, 0.5 * mu, 0.1),
+                       linear_velocity=(2.0, 0.0, 0.5))
+        w.end_scene()
+    for iters in (1, 3):
+        _compare(w, frames=90, check_every=30, iters=iters)
