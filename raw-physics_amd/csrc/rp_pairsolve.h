@@ -302,14 +302,12 @@ __device__ __forceinline__ void solve_item_pos(const DevWorld& w, Body* body, in
     e.im = second ? -g.inv_mass : g.inv_mass;
     e.Iinv = g.Iinv;
     e.mu_s = g.mu_s;
-    {
-        double qq = e.q.x * e.q.x + e.q.y * e.q.y + e.q.z * e.q.z + e.q.w * e.q.w;
-        e.iinv_max = fabs(qq - 1.0) <= 1e-9 ? g.iinv_max : HUGE_VAL;
-    }
     e.fixed = g.fixed;
     if (kExt && t.code < 0) {
         pair_external(w.ext[~t.code], w.ext_lambda + 3 * (~t.code), e, h, err);
     } else {
+        const double qq = e.q.x * e.q.x + e.q.y * e.q.y + e.q.z * e.q.z + e.q.w * e.q.w;
+        e.iinv_max = fabs(qq - 1.0) <= 1e-9 ? g.iinv_max : HUGE_VAL;
         HalfContact k = t.k;
         Contact* cs = w.contacts + (size_t)t.code * MAXC;
         const double mu_s = (e.mu_s + pair_other(e.mu_s)) / 2.0f;
