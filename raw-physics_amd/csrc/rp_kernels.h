@@ -84,11 +84,13 @@ struct DevWorld {
     // solver scratch
     int32_t* item_level;            // [items]       level of each solve item (frame)
     int32_t* item_order;            // [items]       items grouped by level
-    int2* item_bodies;              // [items]       global body indices of each item_order entry
+    int2* item_bodies;              // [items]       global body indices of each item_order entry (see FIRST_CONTACT)
     int32_t* item_lstart;           // [items + ns]  level starts per scene
     int32_t* item_cursor;           // [items + ns]  fill cursors of the sort
     int32_t* scene_nlevels;         // [ns]
-    int32_t* body_last;             // [nb]          last level per body (large scenes)
+    int32_t* scene_period;          // [ns]          levels from one sweep's start to the next one's
+    int32_t* body_last;             // [2 nb]        last and first level per body (scenes beyond k_levels' LDS)
+    int32_t* body_touch;            // [nb]          whether the body takes part in a contact item this frame
     int32_t *uf_parent, *uf_flag;   // [nb]
     const int32_t* scene_big;       // [ns] 1: large scene (grid broad phase, coloured solve)
     double* rec_state;              // [nb][REC_STATE] where an integration records its start states, or null
@@ -96,6 +98,10 @@ struct DevWorld {
     uint32_t* scene_err;            // [ns]
     unsigned long long* stats;      // [STAT_COUNT]
 };
+
+// Set in a body index of item_bodies where the item is the body's first contact
+// item of the frame's order: its velocity solve updates the body's velocity.
+constexpr int FIRST_CONTACT = INT_MIN;
 
 // A large scene: grid broad phase, parallel islands and a graph-coloured
 // solve instead of the per-scene wave kernels. Device buffers are owned by

@@ -560,7 +560,7 @@ k_narrow_general(DevWorld w, int stage) {
 constexpr int LEV_CHUNK = 512;
 constexpr int LEV_LDS_BODIES = 1024;
 
-__global__ void __launch_bounds__(64) k_levels(DevWorld w, int collisions) {
+__global__ void __launch_bounds__(64) k_levels(DevWorld w, int collisions, int pipelined) {
     int s = blockIdx.x;
     if (w.scene_big[s]) return;
     int lane = threadIdx.x;
@@ -573,12 +573,19 @@ __global__ void __launch_bounds__(64) k_levels(DevWorld w, int collisions) {
     int* lev = w.item_level + ib;
     int* order = w.item_order + ib;
     int* ls = w.item_lstart + ib + s;
-    __shared__ int sb1[LEV_CHUNK], sb2[LEV_CHUNK];
-    __shared__ int slast[LEV_LDS_BODIES];
+    __shared__ int sb1[LEV_CHUNK], sb2[LEV_CHUNK], slev[LEV_CHUNK];
+    __shared__ int slast[LEV_LDS_BODIES], sfirst[LEV_LDS_BODIES], stouch[LEV_LDS_BODIES];
     __shared__ int sL;
-    bool lds_last = n <= LEV_LDS_BODIES;
-    int* last = lds_last ? slast : (w.body_last + b0);
-    for (int i = lane; i < n; i += 64) last[i] = 0;
+    bool in_lds = n <= LEV_LDS_BODIES;
+    // per body: one above its last item's level, its first item's level, its
+    // first contact item's level
+    int* last = in_lds ? slast : (w.body_last + 2 * (size_t)b0);
+    int* first = in_lds ? sfirst : (w.body_last + 2 * (size_t)b0 + n);
+    int* touch = in_lds ? stouch : (w.body_touch + b0);
+    for (int i = lane; i < n; i += 64) {
+        last[i] = 0;
+        first[i] = touch[i] = INT_MAX;
+    }
     if (lane == 0) sL = 0;
     __syncthreads();
     for (int c0 = 0; c0 < K; c0 += LEV_CHUNK) {
@@ -607,13 +614,32 @@ __global__ void __launch_bounds__(64) k_levels(DevWorld w, int collisions) {
                 ++lv;
                 if (i1 >= 0) last[i1] = lv;
                 if (i2 >= 0) last[i2] = lv;
-                lev[c0 + k] = lv - 1;
+                slev[k] = lv - 1;
                 L = max(L, lv);
             }
             sL = L;
         }
         __syncthreads();
+        for (int k = lane; k < cn; k += 64) {
+            int lv = slev[k];
+            lev[c0 + k] = lv;
+            if (!pipelined) continue;
+            for (int i : {sb1[k], sb2[k]}) {
+                if (i < 0) continue;
+                atomicMin(&first[i], lv);
+                if (c0 + k >= next) atomicMin(&touch[i], lv);
+            }
+        }
+        __syncthreads();
     }
+    // The period: the fewest levels by which a sweep may start after the one
+    // before it so that no body's item runs before its last item of that
+    // sweep (at least 2: k_solve reads multipliers one level ahead).
+    int period = 2;
+    for (int i = lane; pipelined && i < n; i += 64)
+        if (last[i] > 0) period = max(period, last[i] - first[i]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) period = max(period, __shfl_xor(period, off));
     int L = sL;
     // counting sort by level; the order inside a level does not matter (its
     // items touch disjoint writable bodies)
@@ -625,6 +651,7 @@ __global__ void __launch_bounds__(64) k_levels(DevWorld w, int collisions) {
     if (lane == 0) {
         for (int l = 0; l < L; ++l) ls[l + 1] += ls[l];
         w.scene_nlevels[s] = L;
+        w.scene_period[s] = period;
     }
     __syncthreads();
     for (int l = lane; l <= L; l += 64) cur[l] = ls[l];
@@ -634,8 +661,16 @@ __global__ void __launch_bounds__(64) k_levels(DevWorld w, int collisions) {
         int pos = atomicAdd(&cur[lev[t]], 1);
         int code = (t < next) ? ~(e0 + t) : (g0 + t - next);
         order[pos] = code;
-        bodies[pos] = item_body_pair(w, code, b0);
+        int2 bb = item_body_pair(w, code, b0);
+        if (pipelined && t >= next) {
+            if (touch[bb.x - b0] == lev[t]) bb.x |= FIRST_CONTACT;
+            if (touch[bb.y - b0] == lev[t]) bb.y |= FIRST_CONTACT;
+        }
+        bodies[pos] = bb;
     }
+    if (!pipelined) return;
+    __syncthreads();
+    for (int i = lane; i < n; i += 64) w.body_touch[b0 + i] = touch[i] == INT_MAX ? 0 : 1;
 }
 
 // Solve of one scene and substep: position Gauss-Seidel (pbd.cpp:615-620),
@@ -658,16 +693,32 @@ constexpr int STATE_VECS = offsetof(Body, deact) / sizeof(int4);  // x, q, v, w,
 constexpr int SOLVE_LDS_LIMIT = 64 * 1024;
 static_assert(sizeof(Body) % sizeof(int4) == 0 && offsetof(Body, deact) % sizeof(int4) == 0, "copied as 16-byte words");
 
+// In worlds with joints, and for scenes on several waves, sweeps are pipelined
+// by the period P of the scene's order (k_levels): level l of position
+// iteration i runs at step l + iP, beside the levels of earlier iterations that
+// are still due, and level l of the velocity sweep at step l + iters P. Items of one step share no body that they write, and every body
+// sees its items in the list's order, so the bits are those of one sweep after
+// another. With several waves per scene (kSplit) the velocity sweep has waves
+// of its own: they follow the position sweep P levels behind instead of waiting
+// for its end. Against one sweep after another on one wave (64 lanes) or four:
+// 10 frames of 500 chains of 6 links (4 iterations) 80.5 -> 65.3 ms, 4 frames
+// of 150 scenes of 4 to 256 bodies with chains 25.3 -> 23.1. Scenes of up to 64
+// bodies without joints keep one sweep after another on one wave: their floor
+// is in a pair with every body at level 0, so P is about their whole depth, and
+// the steps' bookkeeping cost 0.5 to 2 %.
 template <bool kExt, int LPS, bool kLds>
-__global__ void __launch_bounds__(LPS > 64 ? LPS : 64) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(LPS > 64 ? 2 * LPS : 64) __attribute__((amdgpu_waves_per_eu(2)))
 k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next, int cap) {
     extern __shared__ int4 rp_solve_lds[];
+    constexpr bool kSplit = LPS > 64, kPipe = kExt || kSplit;
+    constexpr int TPS = kSplit ? 2 * LPS : LPS;   // threads that serve one scene
     constexpr int SPB = LPS < 64 ? 64 / LPS : 1;  // scenes per block
     constexpr int LPW = LPS < 64 ? LPS : 64;      // lanes of a wave that serve one scene
-    int s = blockIdx.x * SPB + (int)threadIdx.x / LPS;
-    int lane = (int)threadIdx.x % LPS;
+    int s = blockIdx.x * SPB + (int)threadIdx.x / TPS;
+    int thread = (int)threadIdx.x % TPS;
+    int lane = thread % LPS;  // in its sweep
     bool valid = s < w.ns && !w.scene_big[s];  // large scenes: coloured solve (rp_large.hip)
-    int b0 = 0, n = 0, e0 = 0, e1x = 0, L = 0, g0 = 0, np = 0;
+    int b0 = 0, n = 0, e0 = 0, e1x = 0, L = 0, P = 2, g0 = 0, np = 0;
     const int* order = nullptr;
     const int2* bodies = nullptr;
     const int* ls = nullptr;
@@ -681,6 +732,7 @@ k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next, int
         bodies = w.item_bodies + ib;
         ls = w.item_lstart + ib + s;
         L = w.scene_nlevels[s];
+        P = w.scene_period[s];
         g0 = w.live_prefix[s];
         np = collisions ? w.live_count[s] : 0;
     }
@@ -688,105 +740,197 @@ k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next, int
     // contiguous in the live list): without, and without external
     // constraints, there is nothing to sweep
     int touching = 0;
-    for (int k = lane; k < np; k += LPS) touching |= w.ncontact[g0 + k];
+    for (int k = thread; k < np; k += TPS) touching |= w.ncontact[g0 + k];
     Body* body = w.body + b0;
     if constexpr (kLds) {
-        int4* own = rp_solve_lds + (size_t)((int)threadIdx.x / LPS) * cap * BODY_VECS;
+        int4* own = rp_solve_lds + (size_t)((int)threadIdx.x / TPS) * cap * BODY_VECS;
         const int4* src = (const int4*)body;
-        for (int i = lane; i < n * BODY_VECS; i += LPS) own[i] = src[i];
+        for (int i = thread; i < n * BODY_VECS; i += TPS) own[i] = src[i];
         body = (Body*)own;
     }
-    if constexpr (LPS > 64) {
+    if constexpr (kSplit) {
         touching = __syncthreads_or(touching);
     } else {
         unsigned long long m = __ballot(touching != 0);
         if constexpr (LPS < 64) m &= ((1ull << LPS) - 1ull) << ((int)threadIdx.x & ~(LPS - 1));
         touching = m != 0;
     }
+    // levels and steps of both sweeps
     if (!touching && !(kExt && e1x > e0)) L = 0;
-    int Lmax = L;  // levels of the block's busiest scene: every lane joins every barrier
-    if constexpr (SPB > 1) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) Lmax = max(Lmax, __shfl_xor(Lmax, off));
-    }
+    const int pos_levels = !kPipe || iters > 0 ? L : 0;
+    const int vel_levels = touching ? L : 0;
+    int pos_steps = kPipe && pos_levels > 0 ? (iters - 1) * P + L : pos_levels;
+    int vel_steps = kSplit && touching ? iters * P + L : vel_levels;
     // level starts ls[0..L] in the lanes' registers (lane l of the wave's
     // lanes of a scene holds ls[l]) when every scene of the block fits, read
     // back by lane exchange instead of a global load per level (the branch is
     // uniform per block)
-    bool ls_in_lanes = Lmax + 1 <= LPW;
-    int my_ls = (valid && lane % LPW <= L) ? ls[lane % LPW] : 0;
+    int Lmax = L;
+    if constexpr (kSplit) {
+        pos_steps = vel_steps = max(pos_steps, vel_steps);
+    } else if constexpr (SPB > 1) {  // every lane joins every barrier
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            Lmax = max(Lmax, __shfl_xor(Lmax, off));
+            if constexpr (kPipe) pos_steps = max(pos_steps, __shfl_xor(pos_steps, off));
+        }
+        if constexpr (!kPipe) pos_steps = Lmax;
+        vel_steps = Lmax;
+    }
+    const bool ls_in_lanes = Lmax + 1 <= LPW;
+    const int my_ls = (valid && lane % LPW <= L) ? ls[lane % LPW] : 0;
     auto level_start = [&](int l) -> int {
-        if (ls_in_lanes) return __shfl(my_ls, l, LPW);
-        return (valid && l <= L) ? ls[l] : 0;
+        if (!ls_in_lanes) return valid ? ls[l] : 0;
+        if constexpr (kSplit) return __builtin_amdgcn_readlane(my_ls, l);
+        else return __shfl(my_ls, l, LPW);
     };
     uint32_t err = 0;
 
     // multipliers of the external constraints start at zero (pbd.cpp:426-462)
     if constexpr (kExt) {
-        for (int k = e0 + lane; k < e1x; k += LPS) {
+        for (int k = e0 + thread; k < e1x; k += TPS) {
             w.ext_lambda[3 * k] = 0.0;
             w.ext_lambda[3 * k + 1] = 0.0;
             w.ext_lambda[3 * k + 2] = 0.0;
         }
     }
     __syncthreads();
-    // One sweep over the levels. `here` is this pair's first item of level l
-    // with its contact, `next` that of level l + 1 (its code only).
-    auto sweep = [&](auto solve) {
-        int i0 = level_start(0), i1 = level_start(1), i2 = level_start(2);
-        PairItem here, next;
-        bool has = 0 < L && i0 + lane / 2 < i1, has_next = 1 < L && i1 + lane / 2 < i2;
-        if (has) {
-            load_item(here, order, bodies, i0 + lane / 2);
-            if (!kExt) load_item_contact<kExt>(here, w);
-        }
-        if (has_next) load_item(next, order, bodies, i1 + lane / 2);
-        for (int l = 0; l < Lmax; ++l) {
-            int i3 = level_start(min(l + 3, L));
-            bool has_after = l + 2 < L && i2 + lane / 2 < i3;
-            PairItem after;
-            // (with joints the registers go to the joint solve)
-            if (!kExt && has_next) load_item_contact<kExt>(next, w);
-            if (has_after) load_item(after, order, bodies, i2 + lane / 2);
-            if (has) {
-                if (kExt) load_item_contact<kExt>(here, w);
-                for (int idx = i0 + lane / 2;;) {
-                    solve(here);
-                    idx += LPS / 2;
-                    if (idx >= i1) break;
-                    load_item(here, order, bodies, idx);
-                    load_item_contact<kExt>(here, w);
-                }
+    auto position = [&](const PairItem& t) { solve_item_pos<kExt>(w, body, b0, t, h, err); };
+    auto velocity = [&](const PairItem& t) { solve_item_vel<kPipe>(w, body, b0, t, h); };
+    if constexpr (kPipe) {
+        // What a sweep solves at one step: level `l` of its sweep `it`, and the
+        // levels l + P, l + 2P, ... of the sweeps before it.
+        struct Step { int it, l; };
+        // Item `slot` of a step or -1, and the number of its items (all lanes of
+        // a scene take the same turns: the exchanges need their partners).
+        auto locate = [&](Step st, int levels, int slot, int& count) -> int {
+            int idx = -1;
+            count = 0;
+            if (st.l < 0) return -1;
+            for (int l = st.l, it = st.it; l < levels && it >= 0; l += P, --it) {
+                int a = level_start(l), m = level_start(l + 1) - a;
+                if (idx < 0 && slot - count < m) idx = a + slot - count;
+                count += m;
             }
-            __syncthreads();
-            here = next;
-            next = after;
-            has = has_next;
-            has_next = has_after;
-            i0 = i1;
-            i1 = i2;
-            i2 = i3;
-        }
-    };
-    for (int it = 0; it < iters; ++it)
-        sweep([&](const PairItem& t) { solve_item_pos<kExt>(w, body, b0, t, h, err); });
-    // velocity update
-    for (int i = lane; i < n; i += LPS) velocity_update_body(body[i], h);
-    __syncthreads();
-    // velocity solve over the collision items, in the same levels
-    sweep([&](const PairItem& t) { solve_item_vel(w, body, b0, t, h); });
+            return idx;
+        };
+        // `sweeps` sweeps from step `begin` on, up to step `steps`. `here` is this
+        // pair's first item of a step with its contact, `next` that of the step
+        // after it (its code, then its contact), `after` the one two steps ahead.
+        auto sweep = [&](int sweeps, int begin, int levels, int steps, auto solve) {
+            auto advance = [&](Step st) -> Step {
+                ++st.l;
+                if (st.l >= P && st.it + 1 < sweeps) {
+                    st.l -= P;
+                    ++st.it;
+                }
+                return st;
+            };
+            // the items of a step go round the sweep's waves: fewer per wave, and
+            // fewer different branches one after another on one
+            constexpr int WAVES = LPS < 64 ? 1 : LPS / 64;
+            const int slot = (lane % LPW / 2) * WAVES + lane / LPW;
+            Step s0 = {0, -begin}, s1 = advance(s0), s2 = advance(s1);
+            int c0, c1, c2, i0 = locate(s0, levels, slot, c0), i1 = locate(s1, levels, slot, c1);
+            PairItem here, next;
+            if (i0 >= 0) {
+                load_item(here, order, bodies, i0);
+                if (!kExt) load_item_contact<kExt>(here, w);
+            }
+            if (i1 >= 0) load_item(next, order, bodies, i1);
+            for (int g = 0; g < steps; ++g) {
+                int i2 = locate(s2, levels, slot, c2);
+                PairItem after;
+                // (with joints the registers go to the joint solve)
+                if (!kExt && i1 >= 0) load_item_contact<kExt>(next, w);
+                if (i2 >= 0) load_item(after, order, bodies, i2);
+                if (kExt && i0 >= 0) load_item_contact<kExt>(here, w);
+                for (int base = 0;;) {
+                    if (i0 >= 0) solve(here);
+                    base += LPS / 2;
+                    if (base >= c0) break;
+                    int c;
+                    i0 = locate(s0, levels, base + slot, c);
+                    if (i0 >= 0) {
+                        load_item(here, order, bodies, i0);
+                        load_item_contact<kExt>(here, w);
+                    }
+                }
+                __syncthreads();
+                here = next;
+                next = after;
+                i0 = i1;
+                i1 = i2;
+                c0 = c1;
+                c1 = c2;
+                s0 = s1;
+                s1 = s2;
+                s2 = advance(s2);
+            }
+        };
+        // (both branches pass the same number of barriers)
+        if (!kSplit || thread < LPS) sweep(iters, 0, pos_levels, pos_steps, position);
+        if (!kSplit || thread >= LPS) sweep(1, kSplit ? iters * P : 0, vel_levels, vel_steps, velocity);
+    } else {
+        // One sweep over the levels. `here` is this pair's first item of level l
+        // with its contact, `next` that of level l + 1 (its code only).
+        auto sweep = [&](int levels, int steps, auto solve) {
+            auto start = [&](int l) { return level_start(min(l, levels)); };
+            int i0 = start(0), i1 = start(1), i2 = start(2);
+            PairItem here, next;
+            bool has = 0 < levels && i0 + lane / 2 < i1, has_next = 1 < levels && i1 + lane / 2 < i2;
+            if (has) {
+                load_item(here, order, bodies, i0 + lane / 2);
+                load_item_contact<kExt>(here, w);
+            }
+            if (has_next) load_item(next, order, bodies, i1 + lane / 2);
+            for (int l = 0; l < steps; ++l) {
+                int i3 = start(l + 3);
+                bool has_after = l + 2 < levels && i2 + lane / 2 < i3;
+                PairItem after;
+                if (has_next) load_item_contact<kExt>(next, w);
+                if (has_after) load_item(after, order, bodies, i2 + lane / 2);
+                if (has) {
+                    for (int idx = i0 + lane / 2;;) {
+                        solve(here);
+                        idx += LPS / 2;
+                        if (idx >= i1) break;
+                        load_item(here, order, bodies, idx);
+                        load_item_contact<kExt>(here, w);
+                    }
+                }
+                __syncthreads();
+                here = next;
+                next = after;
+                has = has_next;
+                has_next = has_after;
+                i0 = i1;
+                i1 = i2;
+                i2 = i3;
+            }
+        };
+        for (int it = 0; it < iters; ++it) sweep(pos_levels, pos_steps, position);
+        // velocity update
+        for (int i = lane; i < n; i += LPS) velocity_update_body(body[i], h);
+        __syncthreads();
+        // velocity solve over the collision items, in the same levels
+        sweep(vel_levels, vel_steps, velocity);
+    }
     if (err && valid) atomicOr(&w.scene_err[s], err);
+    // the velocity update of the bodies without contact items (pipelined), and
     // the next substep's integration of the scene's bodies (worlds without
     // large scenes), in place of a k_integrate launch
-    if (integrate_next) {
-        for (int i = lane; i < n; i += LPS) integrate_body(w, b0 + i, body[i], h);
-        if (blockIdx.x == 0 && threadIdx.x == 0) w.counters[CNT_MANIFOLD] = 0;
-    }
+    if (kPipe || integrate_next)
+        for (int i = thread; i < n; i += TPS) {
+            if (kPipe && (!touching || !w.body_touch[b0 + i])) velocity_update_body(body[i], h);
+            if (integrate_next) integrate_body(w, b0 + i, body[i], h);
+        }
+    if (integrate_next && blockIdx.x == 0 && threadIdx.x == 0) w.counters[CNT_MANIFOLD] = 0;
     if constexpr (kLds) {
         __syncthreads();
         int4* dst = (int4*)(w.body + b0);
         const int4* src = (const int4*)body;
-        for (int i = lane; i < n * STATE_VECS; i += LPS) {
+        for (int i = thread; i < n * STATE_VECS; i += TPS) {
             int b = i / STATE_VECS, k = i - b * STATE_VECS;
             dst[b * BODY_VECS + k] = src[b * BODY_VECS + k];
         }
@@ -797,7 +941,7 @@ k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next, int
 // global memory: the records may not cost the launch waves that the
 // registers (two waves per SIMD, eight per CU) would allow it to hold.
 static size_t solve_lds_bytes(const DevWorld& w, int lanes, int blocks) {
-    int scenes = std::max(1, 64 / lanes), waves = std::max(1, lanes / 64);
+    int scenes = std::max(1, 64 / lanes), waves = lanes > 64 ? 2 * lanes / 64 : 1;
     size_t bytes = (size_t)scenes * w.small_bodies * sizeof(Body);
     if (bytes == 0 || bytes > (size_t)SOLVE_LDS_LIMIT) return 0;
     size_t per_cu = std::min<size_t>(8 / waves, 160 * 1024 / bytes);
@@ -807,7 +951,7 @@ static size_t solve_lds_bytes(const DevWorld& w, int lanes, int blocks) {
 template <bool kExt, int LPS>
 static void launch_solve_lanes(const DevWorld& w, const FrameParams& fp, hipStream_t st, int integrate_next) {
     constexpr int SPB = LPS < 64 ? 64 / LPS : 1;
-    dim3 grid((w.ns + SPB - 1) / SPB), block(LPS > 64 ? LPS : 64);
+    dim3 grid((w.ns + SPB - 1) / SPB), block(LPS > 64 ? 2 * LPS : 64);
     int it = (int)fp.iters, co = fp.collisions ? 1 : 0;
     size_t lds = solve_lds_bytes(w, LPS, (int)grid.x);
     if (lds > 0)
@@ -816,10 +960,15 @@ static void launch_solve_lanes(const DevWorld& w, const FrameParams& fp, hipStre
     else
         hipLaunchKernelGGL((k_solve<kExt, LPS, false>), grid, block, 0, st, w, fp.h, it, co, integrate_next, 0);
 }
-// Whole waves per scene (solve_lanes 64): scenes of more than 64 bodies have
-// levels of more items than one wave's 32 pairs of lanes, and take four waves
-// (scenes of 4 to 256 bodies, ms per frame at 64 / 128 / 256 lanes: 150
-// scenes 8.40 / 8.03 / 7.81, 600 scenes 9.94 / 9.56 / 9.46).
+// Whole waves per scene (solve_lanes 64): one, two per sweep with joints (a wave solves a
+// joint and a contact one after the other: 500 chains of 6 links 7.3 / 6.5 / 6.7
+// ms per frame at 64 / 128 / 256 lanes per sweep), and four per sweep for scenes
+// of more than 64 bodies, whose steps have more items (150 scenes of 4 to 256
+// bodies 6.6 / 6.1 / 5.8). Scenes of 16 bodies lose by more waves at every
+// barrier (one scene 0.89 / 0.95 / 1.08, 1000 scenes 1.7 / 1.9 / 2.7).
+static bool solve_pipelined(const DevWorld& w) {  // kPipe of the kernel that launch_solve takes
+    return w.n_ext > 0 || (w.solve_lanes == 64 && w.small_bodies > 64);
+}
 template <bool kExt>
 static void launch_solve(const DevWorld& w, const FrameParams& fp, hipStream_t st, int integrate_next) {
     switch (w.solve_lanes) {
@@ -827,7 +976,7 @@ static void launch_solve(const DevWorld& w, const FrameParams& fp, hipStream_t s
     case 32: launch_solve_lanes<kExt, 32>(w, fp, st, integrate_next); break;
     default:
         if (w.small_bodies > 64) launch_solve_lanes<kExt, 256>(w, fp, st, integrate_next);
-        else launch_solve_lanes<kExt, 64>(w, fp, st, integrate_next);
+        else launch_solve_lanes<kExt, kExt ? 128 : 64>(w, fp, st, integrate_next);
         break;
     }
 }
@@ -911,7 +1060,7 @@ hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_
     hipLaunchKernelGGL(k_scan_live, dim3(1), dim3(1024), 0, st, w);
     hipLaunchKernelGGL(k_scatter_live, dim3(w.ns), dim3(64), 0, st, w);
     for (int k = 0; k < nbig; ++k) big_scatter(w, bigs[k], st);
-    hipLaunchKernelGGL(k_levels, dim3(w.ns), dim3(64), 0, st, w, fp.collisions ? 1 : 0);
+    hipLaunchKernelGGL(k_levels, dim3(w.ns), dim3(64), 0, st, w, fp.collisions ? 1 : 0, solve_pipelined(w) ? 1 : 0);
     for (int k = 0; k < nbig; ++k) big_colour(w, bigs[k], fp.collisions, st);
     t.end(st);
     // without large scenes, the solve kernel integrates its scenes' bodies for

@@ -270,12 +270,15 @@ __device__ __forceinline__ HalfContact load_half(const Contact& c) {
 struct PairItem {
     int code;
     int2 bb;
+    int first;  // negative: this lane's body's first contact item
     int nc;
     HalfContact k;
 };
 __device__ __forceinline__ void load_item(PairItem& t, const int* order, const int2* bodies, int idx) {
     t.code = order[idx];
-    t.bb = bodies[idx];
+    int2 bb = bodies[idx];
+    t.first = second_lane() ? bb.y : bb.x;
+    t.bb = make_int2(bb.x & ~FIRST_CONTACT, bb.y & ~FIRST_CONTACT);
 }
 // The contact count and the first contact of a live pair (its slots are
 // always allocated, so both loads are issued together and what an empty
@@ -326,10 +329,13 @@ __device__ __forceinline__ void solve_item_pos(const DevWorld& w, Body* body, in
 }
 
 // Velocity solve of item t's contacts (pbd.cpp:646-711); external constraints
-// take no part.
+// take no part. kUpdate: a body's velocity update (pbd.cpp:623-643) goes before
+// its first item's solve, whether or not that has contacts.
+template <bool kUpdate>
 __device__ __forceinline__ void solve_item_vel(const DevWorld& w, Body* body, int b0, const PairItem& t, double h) {
-    if (t.nc == 0) return;
     Body& g = body[(second_lane() ? t.bb.y : t.bb.x) - b0];
+    if (kUpdate && t.first < 0) velocity_update_body(g, h);
+    if (t.nc == 0) return;
     HalfVel e;
     e.q = g.q; e.v = g.v; e.w = g.w; e.pv = g.pv; e.pw = g.pw;
     e.im = g.inv_mass;
@@ -356,7 +362,7 @@ __device__ __forceinline__ void solve_item_at(const DevWorld& w, const int* orde
     PairItem t;
     load_item(t, order, bodies, idx);
     load_item_contact<true>(t, w);
-    if (kVel) solve_item_vel(w, w.body, 0, t, h);
+    if (kVel) solve_item_vel<false>(w, w.body, 0, t, h);
     else solve_item_pos<kExt>(w, w.body, 0, t, h, err);
 }
 

@@ -636,7 +636,9 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
     ok &= im.alloc(d.item_lstart, (size_t)ccap + d.ns);
     ok &= im.alloc(d.item_cursor, (size_t)ccap + d.ns);
     ok &= im.alloc(d.scene_nlevels, d.ns);
-    ok &= im.alloc(d.body_last, d.nb);
+    ok &= im.alloc(d.scene_period, d.ns);
+    ok &= im.alloc(d.body_last, 2 * (size_t)d.nb);
+    ok &= im.alloc(d.body_touch, d.nb);
     ok &= im.alloc(d.uf_parent, d.nb);
     ok &= im.alloc(d.uf_flag, d.nb);
     uint32_t* errp;
@@ -945,7 +947,7 @@ static bool build_views(rp_world* w) {
         v.n_ext = w->hw.scene_ext_off[s1] - w->hw.scene_ext_off[s0];
         v.scene_body_off += s0; v.scene_pair_base += s0; v.scene_ext_off += s0; v.scene_item_base += s0;
         v.pair_count += s0; v.live_count += s0; v.live_prefix += s0 + k;
-        v.scene_nlevels += s0; v.scene_big += s0; v.scene_err += s0;
+        v.scene_nlevels += s0; v.scene_period += s0; v.scene_big += s0; v.scene_err += s0;
         v.item_lstart += s0; v.item_cursor += s0;
         v.live_global += P0; v.live_rec += P0; v.live_hull += P0; v.ncontact += P0; v.pair_normal += P0; v.mlist += P0; v.pair_lists += P0;
         v.contacts += P0 * MAXC;

@@ -116,3 +116,55 @@ def test_static_friction_bit_exact(mu):
         w.end_scene()
     for iters in (1, 3):
         _compare(w, frames=90, check_every=30, iters=iters)
+
+
+@pytest.mark.parametrize("iters", [1, 2, 5])
+def test_overlapping_sweeps_bit_exact(iters):
+    """Scenes whose orders have periods from 2 to their whole depth (a lone
+    cube, towers, a pile) beside one of more than 64 bodies, so that later
+    sweeps start right behind or only after earlier ones."""
+    w = scenes.World(name="periods")
+    for k, n in enumerate((1, 2, 9, 66)):
+        scenes.stack_scene(w, seed=k, num_cubes=n)
+    scenes.drop_scene(w, 41, n_cubes=12, n_icos=10)
+    _compare(w, frames=60, check_every=20, iters=iters)
+
+
+@pytest.mark.parametrize("iters", [1, 2, 5])
+def test_overlapping_joint_sweeps_change_nothing(iters):
+    """Chains of two and of nine links on the floor: the sweeps on one wave, on
+    half and quarter waves and on their own waves give the same bits, and the
+    oracle's poses (joint limits: libm)."""
+    w = scenes.World(name="chains")
+    for k, n in enumerate((2, 9, 2, 1, 5)):
+        scenes.chain_scene(w, 60 + k, length=n)
+    o = SimWorld("orc", w)
+    gs = []
+    for lanes in (64, 32, 16):
+        gs.append(SimWorld("rp", w))
+        assert gs[-1].lib.rp_world_set_solve_lanes(gs[-1].h, lanes) == 0
+    for f in range(20):
+        # each frame from the device's state: a joint limit's last bit grows
+        # some tenfold every few frames in these scenes
+        o.set_state(gs[0].state())
+        for g in [o] + gs:
+            g.step(1, iters=iters)
+        first = gs[0].state()
+        for g in gs[1:]:
+            assert not state_bits_equal(first, g.state()), f"frame {f}"
+        assert np.allclose(o.state()["position"], first["position"], rtol=0, atol=1e-9), f"frame {f}"
+    assert not any(g.error(s) for g in gs for s in range(w.num_scenes))
+
+
+def test_scene_beyond_the_level_sort_lds_bit_exact():
+    """1100 bodies in one scene that is solved level by level: its per-body
+    levels lie in global memory, its level starts beyond a wave's lanes."""
+    w = scenes.World(name="towers_1100")
+    scenes._floor(w)
+    cube = w.shape(scenes.cube_corners())
+    for k in range(1100):  # 20 x 11 towers of five
+        i, level = divmod(k, 5)
+        w.add_body(cube, (1.0, 1.0, 1.0), (2.4 * (i % 20) - 24.0 + 0.02 * level, 2.01 * level, 2.4 * (i // 20) - 13.0),
+                   scenes.quaternion_new((0.0, 1.0, 0.0), 3.0 * (k % 7)))
+    w.end_scene()
+    _compare(w, frames=24, check_every=8, iters=2)
