@@ -272,6 +272,8 @@ bool narrow_group_supported(const DevWorld& w, int g);
 // Lets the lane-group narrow-phase kernels take up to `bytes` of dynamic LDS
 // per block (gfx950 gives a workgroup up to 160 KiB).
 hipError_t allow_narrow_lds(int bytes);
+// Lets the solve of scenes above 64 bodies hold them in more than 64 KiB of LDS.
+hipError_t allow_solve_lds();
 int narrow_blocks_for(const DevWorld& w, int g, int64_t pair_capacity);
 hipError_t launch_fp64_selftest(const double* a, const double* b, double* out, int64_t n, hipStream_t st);
 

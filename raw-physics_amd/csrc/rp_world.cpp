@@ -538,6 +538,7 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
             RP_CHECK(allow_narrow_lds(lim));
         }
     }
+    if (d.small_bodies > 64) RP_CHECK(allow_solve_lds());
     // size classes: with hulls above SMALL_HULL_NV vertices, the pairs of two
     // smaller hulls get their own list and LDS slices sized for them (if the
     // large-hull pairs fit a 16-lane schedule)
