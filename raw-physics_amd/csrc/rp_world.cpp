@@ -1126,6 +1126,8 @@ static uint32_t world_run(rp_world* w, const FrameParams& fp, uint32_t frames, b
         }
         if (e != hipSuccess) {
             set_msg(std::string("frame graph: ") + hipGetErrorString(e));
+            // (views that were launched but not joined)
+            for (int k = 0; k < w->nviews; ++k) (void)hipStreamSynchronize(w->view_stream[k]);
             return RP_ERR_RUNTIME;
         }
         frames = 0;
@@ -1562,6 +1564,7 @@ static uint32_t adjoint_record(rp_world* w, const FrameParams& fp, int k, uint32
     const DevWorld& d = w->im.d;
     size_t bytes = (size_t)d.nb * sizeof(Body);
     Body* ck = w->ckpt + (size_t)k * d.nb;
+    w->rec_seg = -1;  // a segment recorded in part is none
     hipError_t e = hipMemcpyAsync(first ? ck : d.body, first ? d.body : ck, bytes, hipMemcpyDeviceToDevice, w->stream);
     for (uint32_t f = 0; f < n && e == hipSuccess; ++f) {
         uint32_t err = world_run(w, fp, 1, false);
@@ -1624,11 +1627,8 @@ uint32_t rp_world_adjoint_forward(rp_world* w, double dt, uint32_t frames, uint3
     return 0;
 }
 
-uint32_t rp_world_adjoint_backward(rp_world* w, const double* dl_dstate, double* grad_state, double* grad_param) {
-    if (!w->ckpt || w->ck_frames == 0) {
-        set_msg("adjoint_backward: no recorded forward pass");
-        return RP_ERR_SELECT;
-    }
+// The backward pass over the recorded segments, last to first.
+static uint32_t adjoint_sweep(rp_world* w, const double* dl_dstate, int segs) {
     const DevWorld& d = w->im.d;
     size_t nb = (size_t)d.nb;
     const FrameParams& fp = w->ck_fp;
@@ -1639,7 +1639,6 @@ uint32_t rp_world_adjoint_backward(rp_world* w, const double* dl_dstate, double*
         hipMemcpy(w->amax, w->dl_norm.data(), nb * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(w->gparam, 0, nb * 3 * sizeof(double)) != hipSuccess)
         return RP_ERR_RUNTIME;
-    int segs = (int)((w->ck_frames + w->seg_frames - 1) / w->seg_frames);
     for (int k = segs - 1; k >= 0; --k) {
         uint32_t n = std::min(w->seg_frames, w->ck_frames - (uint32_t)k * w->seg_frames);
         // the record holds the segment recorded last
@@ -1658,11 +1657,27 @@ uint32_t rp_world_adjoint_backward(rp_world* w, const double* dl_dstate, double*
             return RP_ERR_RUNTIME;
         }
     }
-    // the world continues from the end of the recorded run
-    if (hipMemcpyAsync(d.body, w->ckpt + (size_t)segs * nb, nb * sizeof(Body), hipMemcpyDeviceToDevice, w->stream) !=
-            hipSuccess ||
+    return 0;
+}
+
+uint32_t rp_world_adjoint_backward(rp_world* w, const double* dl_dstate, double* grad_state, double* grad_param) {
+    if (!w->ckpt || w->ck_frames == 0) {
+        set_msg("adjoint_backward: no recorded forward pass");
+        return RP_ERR_SELECT;
+    }
+    size_t nb = (size_t)w->im.d.nb;
+    int segs = (int)((w->ck_frames + w->seg_frames - 1) / w->seg_frames);
+    uint32_t err = adjoint_sweep(w, dl_dstate, segs);
+    // the world continues from the end of the recorded run, also where the
+    // pass failed with a segment stepped again in part
+    if (hipMemcpyAsync(w->im.d.body, w->ckpt + (size_t)segs * nb, nb * sizeof(Body), hipMemcpyDeviceToDevice,
+                       w->stream) != hipSuccess ||
         hipStreamSynchronize(w->stream) != hipSuccess)
-        return RP_ERR_RUNTIME;
+        err = err ? err : RP_ERR_RUNTIME;
+    if (err) {
+        w->dl_norm.clear();  // no amplification either
+        return err;
+    }
     if ((grad_state && hipMemcpy(grad_state, w->abar, nb * 13 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) ||
         (grad_param && hipMemcpy(grad_param, w->gparam, nb * 3 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess))
         return RP_ERR_RUNTIME;

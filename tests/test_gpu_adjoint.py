@@ -132,3 +132,68 @@ def test_adjoint_record_segments_give_identical_gradients(scenes_n, memory):
         assert not state_bits_equal(st, gw.state())
         got.append((gs, gp, gw.adjoint_amplification()))
     assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+# hipGraphLaunch that fails, without launching anything, on the call that
+# FAIL_AT counts down to; loaded ahead of the library in a child process.
+FAILING_LAUNCH = r"""
+#include <dlfcn.h>
+int fail_at = 0;
+int hipGraphLaunch(void* exec, void* stream) {
+    static int (*real)(void*, void*);
+    if (!real) {
+        void* hip = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
+        if (!hip) hip = dlopen("libamdhip64.so", RTLD_LAZY);
+        real = (int (*)(void*, void*))dlsym(hip, "hipGraphLaunch");
+    }
+    if (fail_at > 0 && --fail_at == 0) return 1;
+    return real(exec, stream);
+}
+"""
+FAILED_BACKWARD = r"""
+import ctypes, sys
+sys.path.insert(0, sys.argv[1] + "/tests")
+shim = ctypes.CDLL(sys.argv[2], ctypes.RTLD_GLOBAL)
+fail_at = ctypes.c_int.in_dll(shim, "fail_at")
+import numpy as np
+from _libs import pkg, scenes, state_bits_equal
+world, _ = scenes.ramps(3, first_seed=40)
+gw = pkg.World(world)
+gw.set_adjoint_memory(170000)  # two frames of 82848 bytes per segment
+start = gw.state()
+dl = np.random.default_rng(5).normal(size=(world.num_bodies, 13))
+assert gw.adjoint_forward(4) == 0
+end = gw.state()
+want = gw.adjoint_backward(dl)
+gw.set_state(start)
+assert gw.adjoint_forward(4) == 0  # the record holds the second segment again
+fail_at.value = 2
+try:
+    gw.adjoint_backward(dl)
+    raise SystemExit("the second launch was meant to fail")
+except RuntimeError:
+    pass
+assert fail_at.value == 0
+bad = state_bits_equal(end, gw.state())
+assert not bad, f"the world is not left at the end of the run: {bad}"
+got = gw.adjoint_backward(dl)
+assert all(np.array_equal(a, b) for a, b in zip(got, want)), "gradients of a mixed record"
+print("ok")
+"""
+
+
+def test_failed_backward_pass_leaves_no_mixed_record(tmp_path):
+    """A launch that fails while an earlier segment is stepped again: the world
+    is left at the end of the recorded run, and the next backward pass does not
+    take the partly overwritten record for the last segment's."""
+    import subprocess
+    import sys
+
+    from _libs import ROOT
+
+    src, so = tmp_path / "launch.c", tmp_path / "launch.so"
+    src.write_text(FAILING_LAUNCH)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src), "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-c", FAILED_BACKWARD, str(ROOT), str(so)], capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0 and "ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
