@@ -248,7 +248,8 @@ __global__ void __launch_bounds__(64) k_adjoint_jacobian(AdjRecord r, const int3
         out[j] = o.d[0];
         mismatch |= __double_as_longlong(o.v) != __double_as_longlong(next[j]);
     }
-    if (mismatch) atomicAdd(&stats[STAT_ADJ_MISMATCH], 1ull);
+    // (the group's lanes have the same values: a substep counts once)
+    if (mismatch && k == 0) atomicAdd(&stats[STAT_ADJ_MISMATCH], 1ull);
     if (err && k == 0) atomicOr(&scene_err[s], err);
 }
 

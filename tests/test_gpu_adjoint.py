@@ -197,3 +197,25 @@ def test_failed_backward_pass_leaves_no_mixed_record(tmp_path):
     r = subprocess.run([sys.executable, "-c", FAILED_BACKWARD, str(ROOT), str(so)], capture_output=True, text=True,
                        timeout=100)
     assert r.returncode == 0 and "ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+def test_mismatches_count_substeps():
+    """A cube on a floor of fixed blocks whose corners meet under it, with more
+    contacts than the backward pass keeps: the substeps that are not reproduced
+    are counted once each, and the scene's error word says why."""
+    w = scenes.World(name="many_blocks")
+    cube = w.shape(scenes.cube_corners())
+    for i in range(4):
+        for j in range(4):
+            w.add_body(cube, (0.3, 0.5, 0.3), (0.6 * i - 0.9, -0.5, 0.6 * j - 0.9),
+                       scenes.quaternion_new((0.0, 1.0, 0.0), 0.0), fixed=True, material=(0.6, 0.5, 0.0))
+    w.add_body(cube, (1.0, 0.5, 1.0), (0.01, 0.499, 0.02), scenes.quaternion_new((0.0, 1.0, 0.0), 3.0), mass=1.0,
+               material=(0.6, 0.5, 0.0))
+    w.end_scene()
+    gw = pkg.World(w)
+    frames, substeps = 4, 20
+    assert gw.adjoint_forward(frames, substeps=substeps) == 0
+    gw.adjoint_backward(np.ones((w.num_bodies, 13)))
+    assert gw.errors()[0] & 0x800  # RP_ERR_SOLVER_CAPACITY
+    n = gw.adjoint_mismatches()
+    assert 0 < n <= frames * substeps, n
