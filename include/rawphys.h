@@ -320,7 +320,11 @@ uint32_t rp_world_adjoint_backward(rp_world* w, const double* dl_dstate, double*
  * take, from the next rp_world_adjoint_forward on; never more than half of
  * what is free, and at least one frame. A run whose record is larger is
  * recorded in segments of whole frames: the backward pass steps each segment
- * but the last again from a checkpoint. Identical results. Returns 0. */
+ * but the last again from a checkpoint. Identical results. The record is kept
+ * for the next run; what it holds beyond the limit is given back by the next
+ * rp_world_adjoint_forward. The limit is on the record alone: the frame being
+ * recorded (about 1.2 frames of the record), a checkpoint per segment (464 bytes per
+ * body) and up to 512 MiB of Jacobians come on top. Returns 0. */
 uint32_t rp_world_set_adjoint_memory(rp_world* w, uint64_t bytes);
 /* Substeps whose recomputation in the backward pass did not reproduce the
  * recorded forward state bit for bit (0 when the backward pass is exact). */

@@ -1510,8 +1510,10 @@ uint32_t rp_world_set_body_params(rp_world* w, const double* mass, const double*
 
 // Device memory the record of a differentiable run may take; a longer run is
 // recorded in segments of whole frames, and the backward pass steps each
-// earlier segment again from its checkpoint before reversing it. The
-// Jacobians of a part of the record at a time take JAC_BYTES.
+// earlier segment again from its checkpoint before reversing it. Beside the
+// record, the frame being recorded takes its own buffers (`stage`), each
+// segment a checkpoint, and the Jacobians of a part of the record at a time up
+// to kAdjJacBytes.
 static const size_t kAdjRecordBytes = (size_t)16 << 30;
 static const size_t kAdjJacBytes = (size_t)512 << 20;
 
@@ -1529,6 +1531,19 @@ static bool adjoint_prepare(rp_world* w, const FrameParams& fp, uint32_t frames,
     size_t F = w->seg_frames, steps = F * fp.substeps, segs = (frames + F - 1) / F;
     w->jac_steps = (int)std::min<size_t>(steps, adjoint_steps_per_chunk(d.ns, kAdjJacBytes));
     w->rec_seg = -1;
+    // an earlier run's record that holds more than the limit now allows goes
+    void** record[] = {(void**)&w->rec.state, (void**)&w->rec.ncontact, (void**)&w->rec.contacts,
+                       (void**)&w->rec.pair,  (void**)&w->rec.g0,       (void**)&w->rec.np};
+    size_t held = 0;
+    for (void** p : record) held += w->adj_bytes.count(p) ? w->adj_bytes[p] : 0;
+    if (held > std::max(limit, F * per_frame)) {
+        (void)hipStreamSynchronize(w->stream);
+        for (void** p : record) {
+            if (*p) (void)hipFree(*p);
+            *p = nullptr;
+            w->adj_bytes.erase(p);
+        }
+    }
     bool ok = adjoint_grow(w, w->ckpt, (segs + 1) * nb * sizeof(Body)) &&
               adjoint_grow(w, w->scene_dyn, ns * sizeof(int32_t)) &&
               adjoint_grow(w, w->stage.state, fp.substeps * nb * REC_STATE * sizeof(double)) &&

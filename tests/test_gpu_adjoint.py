@@ -219,3 +219,31 @@ def test_mismatches_count_substeps():
     assert gw.errors()[0] & 0x800  # RP_ERR_SOLVER_CAPACITY
     n = gw.adjoint_mismatches()
     assert 0 < n <= frames * substeps, n
+
+
+def test_smaller_adjoint_memory_frees_the_record():
+    """A smaller limit takes effect from the next forward pass on: what the
+    record of the run before it held beyond the limit is given back."""
+    import ctypes
+
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the one the library runs on
+
+    def free_bytes():
+        n, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(n), ctypes.byref(total)) == 0
+        return n.value
+
+    world, _ = scenes.ramps(512, first_seed=40)
+    gw = pkg.World(world)
+    start = gw.state()
+    dl = np.random.default_rng(5).normal(size=(world.num_bodies, 13))
+    free, got = [], []
+    # 20 substeps of 512 scenes: 14 MB per frame
+    for limit in (0, 64 << 20):
+        gw.set_adjoint_memory(limit)
+        gw.set_state(start)
+        assert gw.adjoint_forward(60) == 0
+        got.append(gw.adjoint_backward(dl))
+        free.append(free_bytes())
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+    assert free[1] - free[0] >= 600 << 20, free
