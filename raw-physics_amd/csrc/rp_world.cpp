@@ -807,7 +807,9 @@ struct rp_world {
     double kc_ms[KC_COUNT] = {0};
     uint64_t kc_launches[KC_COUNT] = {0};
     // one frame's launches captured as a HIP graph per view and replayed per
-    // frame; views are scene ranges of the world on streams of their own
+    // frame; views are scene ranges of the world on streams of their own. A
+    // stepped and a recorded frame have graphs of their own, so that a loop
+    // which alternates them captures neither again
     bool use_graphs = true;
     int want_views = 0;  // 0 = automatic
     int nviews = 0;
@@ -816,10 +818,13 @@ struct rp_world {
     int64_t view_p0[kMaxViews] = {};
     std::vector<BigScene> view_big[kMaxViews];
     hipStream_t view_stream[kMaxViews] = {};
-    hipGraphExec_t view_exec[kMaxViews] = {};
+    struct FrameGraph {
+        hipGraphExec_t exec[kMaxViews] = {};
+        FrameParams fp;
+        uint64_t gen = 0;
+    } graph[2];                              // by FrameParams::record
     hipEvent_t fork_ev = nullptr, join_ev[kMaxViews] = {};
-    FrameParams graph_fp;
-    uint64_t sched_gen = 1, graph_gen = 0;  // schedule changes invalidate the captured graphs
+    uint64_t sched_gen = 1, views_gen = 0;  // schedule changes invalidate the views and the captured graphs
     // bounded queue: at most two chunks of frames in flight on each stream
     hipEvent_t chunk_done[2][kMaxViews] = {};
     // differentiable runs (adjoint_forward / adjoint_backward): the record of
@@ -845,7 +850,7 @@ struct rp_world {
 };
 
 // A buffer of the adjoint, grown to `bytes` (its contents are not kept). A
-// moved buffer invalidates the captured graphs, which hold its address.
+// moved buffer invalidates the recorded frame's graphs, which hold its address.
 template <class T>
 static bool adjoint_grow(rp_world* w, T*& p, size_t bytes) {
     size_t& have = w->adj_bytes[(void**)&p];
@@ -854,7 +859,7 @@ static bool adjoint_grow(rp_world* w, T*& p, size_t bytes) {
     if (p) (void)hipFree((void*)p);
     p = nullptr;
     have = 0;
-    ++w->sched_gen;
+    w->graph[1].gen = 0;
     void* q = nullptr;
     if (hipMalloc(&q, std::max<size_t>(bytes, 16)) != hipSuccess) {
         set_msg("adjoint: device allocation failed");
@@ -871,6 +876,7 @@ static void adjoint_free(rp_world* w) {
         *p = nullptr;
     }
     w->adj_bytes.clear();
+    w->graph[1].gen = 0;
     w->ck_frames = 0;
 }
 
@@ -982,8 +988,9 @@ static bool build_views(rp_world* w) {
     return true;
 }
 
-static void drop_graphs(rp_world* w) {
-    for (hipGraphExec_t& e : w->view_exec)
+static void drop_graphs(rp_world::FrameGraph& g) {
+    g.gen = 0;
+    for (hipGraphExec_t& e : g.exec)
         if (e) {
             (void)hipGraphExecDestroy(e);
             e = nullptr;
@@ -1019,12 +1026,17 @@ static void plan_big(rp_world* w) {
 // captured once per view and reused while they do not change.
 static hipError_t frame_graph(rp_world* w, const FrameParams& fp) {
     plan_big(w);
-    if (w->nviews > 0 && w->view_exec[0] && same_params(w->graph_fp, fp) && w->graph_gen == w->sched_gen)
-        return hipSuccess;
+    rp_world::FrameGraph& fg = w->graph[fp.record];
+    if (fg.gen == w->sched_gen && same_params(fg.fp, fp)) return hipSuccess;
     (void)hipStreamSynchronize(w->stream);
     for (int k = 1; k < w->nviews; ++k) (void)hipStreamSynchronize(w->view_stream[k]);
-    drop_graphs(w);
-    if (!build_views(w)) return hipErrorOutOfMemory;
+    drop_graphs(fg);
+    if (w->views_gen != w->sched_gen) {
+        w->views_gen = 0;
+        drop_graphs(w->graph[!fp.record]);  // (captured on the views that go)
+        if (!build_views(w)) return hipErrorOutOfMemory;
+        w->views_gen = w->sched_gen;
+    }
     for (int k = 0; k < w->nviews; ++k) {
         hipStream_t st = w->view_stream[k];
         hipGraph_t g = nullptr;
@@ -1036,15 +1048,15 @@ static hipError_t frame_graph(rp_world* w, const FrameParams& fp) {
                                      fp.record ? &rec : nullptr);
         e = hipStreamEndCapture(st, &g);
         if (le != hipSuccess) e = le;
-        if (e == hipSuccess) e = hipGraphInstantiate(&w->view_exec[k], g, nullptr, nullptr, 0);
+        if (e == hipSuccess) e = hipGraphInstantiate(&fg.exec[k], g, nullptr, nullptr, 0);
         if (g) (void)hipGraphDestroy(g);
         if (e != hipSuccess) {
-            drop_graphs(w);
+            drop_graphs(fg);
             return e;
         }
     }
-    w->graph_fp = fp;
-    w->graph_gen = w->sched_gen;
+    fg.fp = fp;
+    fg.gen = w->sched_gen;
     return hipSuccess;
 }
 
@@ -1075,7 +1087,7 @@ static void world_free(rp_world* w) {
     if (!w) return;
     if (w->stream) (void)hipStreamSynchronize(w->stream);
     for (int k = 1; k < w->nviews; ++k) (void)hipStreamSynchronize(w->view_stream[k]);
-    drop_graphs(w);
+    for (rp_world::FrameGraph& g : w->graph) drop_graphs(g);
     adjoint_free(w);
     if (w->state_dev) (void)hipFree(w->state_dev);
     if (w->state_pin) (void)hipHostFree(w->state_pin);
@@ -1116,7 +1128,7 @@ static uint32_t world_run(rp_world* w, const FrameParams& fp, uint32_t frames, b
             // a long run looks at the large scenes again once per chunk
             if (f > 0 && f % kFramesPerChunk == 0 && !w->im.big.empty() && w->nviews == 1) e = frame_graph(w, fp);
             for (int k = 0; e == hipSuccess && k < w->nviews; ++k) {
-                e = hipGraphLaunch(w->view_exec[k], w->view_stream[k]);
+                e = hipGraphLaunch(w->graph[fp.record].exec[k], w->view_stream[k]);
                 if (e == hipSuccess) e = chunk_mark(w, f, k, w->view_stream[k]);
             }
         }

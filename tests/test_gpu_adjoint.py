@@ -182,21 +182,25 @@ print("ok")
 """
 
 
-def test_failed_backward_pass_leaves_no_mixed_record(tmp_path):
-    """A launch that fails while an earlier segment is stepped again: the world
-    is left at the end of the recorded run, and the next backward pass does not
-    take the partly overwritten record for the last segment's."""
+def _run_with_runtime(tmp_path, runtime, code):
+    """Runs `code` in a child process with functions of the HIP runtime replaced."""
     import subprocess
     import sys
 
     from _libs import ROOT
 
-    src, so = tmp_path / "launch.c", tmp_path / "launch.so"
-    src.write_text(FAILING_LAUNCH)
+    src, so = tmp_path / "runtime.c", tmp_path / "runtime.so"
+    src.write_text(runtime)
     subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src), "-ldl"], check=True)
-    r = subprocess.run([sys.executable, "-c", FAILED_BACKWARD, str(ROOT), str(so)], capture_output=True, text=True,
-                       timeout=100)
+    r = subprocess.run([sys.executable, "-c", code, str(ROOT), str(so)], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+def test_failed_backward_pass_leaves_no_mixed_record(tmp_path):
+    """A launch that fails while an earlier segment is stepped again: the world
+    is left at the end of the recorded run, and the next backward pass does not
+    take the partly overwritten record for the last segment's."""
+    _run_with_runtime(tmp_path, FAILING_LAUNCH, FAILED_BACKWARD)
 
 
 def test_mismatches_count_substeps():
@@ -247,3 +251,49 @@ def test_smaller_adjoint_memory_frees_the_record():
         free.append(free_bytes())
     assert all(np.array_equal(a, b) for a, b in zip(*got))
     assert free[1] - free[0] >= 600 << 20, free
+
+
+# Counts the graphs that are instantiated.
+COUNTING_INSTANTIATE = r"""
+#include <dlfcn.h>
+int instantiated = 0;
+int hipGraphInstantiate(void** exec, void* graph, void** node, char* log, unsigned long size) {
+    static int (*real)(void**, void*, void**, char*, unsigned long);
+    if (!real) {
+        void* hip = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
+        if (!hip) hip = dlopen("libamdhip64.so", RTLD_LAZY);
+        real = (int (*)(void**, void*, void**, char*, unsigned long))dlsym(hip, "hipGraphInstantiate");
+    }
+    ++instantiated;
+    return real(exec, graph, node, log, size);
+}
+"""
+ALTERNATING = r"""
+import ctypes, sys
+sys.path.insert(0, sys.argv[1] + "/tests")
+count = ctypes.c_int.in_dll(ctypes.CDLL(sys.argv[2], ctypes.RTLD_GLOBAL), "instantiated")
+from _libs import SimWorld, pkg, scenes, state_bits_equal
+world, _ = scenes.ramps(70, first_seed=40)
+gw, oracle = pkg.World(world), SimWorld("orc", world)
+for turn in range(4):
+    gw.step(1)
+    assert gw.adjoint_forward(2) == 0
+    oracle.step(3)
+    assert not state_bits_equal(oracle.state(), gw.state()), turn
+    if turn == 0:
+        first = count.value
+assert first > 0 and count.value == first, (first, count.value)
+gw.set_views(1)  # both frames' graphs are captured again, once
+for turn in range(2):
+    gw.step(1)
+    assert gw.adjoint_forward(2) == 0
+    oracle.step(3)
+    assert not state_bits_equal(oracle.state(), gw.state()), turn
+assert count.value == first + 2, (first, count.value)
+print("ok")
+"""
+
+
+def test_alternating_steps_and_recorded_runs_capture_once(tmp_path):
+    """A loop that steps and records in turn keeps both frames' graphs."""
+    _run_with_runtime(tmp_path, COUNTING_INSTANTIATE, ALTERNATING)
