@@ -115,14 +115,18 @@ constexpr int BIG_SERIAL = BIG_COLOURS;     // class solved one item after anoth
 constexpr int BIG_CLASSES = BIG_COLOURS + 1;
 constexpr int BIG_COLOUR_ROUNDS = 64;       // Jones-Plassmann rounds per frame (launches end at once when all are coloured)
 // Colour classes launched one by one over the device, the rest on one block
-// with a block barrier between classes. By default the host chooses how many,
-// before a frame is captured or launched, from what an earlier frame's
-// colouring left in BigScene::hint: the classes up to the last of more than
-// BIG_TAIL_ITEMS items. A launch costs about 3 us even where the class is
-// empty (128 launches per substep; 20000 falling bodies: 6.0 ms per frame with
-// every class launched, 2.6 with 8), while on one block a settled pile's 26
-// classes beyond the first 24 would cost milliseconds. The colour rounds
-// launched follow the same way. Any choice gives the same bits.
+// with a block barrier between classes. By default the host chooses how many
+// from what the colouring left in BigScene::hint: the classes up to the last
+// of more than BIG_TAIL_ITEMS items. A launch costs about 3 us even where the
+// class is empty (128 launches per substep; 20000 falling bodies: 6.0 ms per
+// frame with every class launched, 2.6 with 8), while on one block a settled
+// pile's 26 classes beyond the first 24 would cost milliseconds. The colour
+// rounds launched follow the same way. Any choice gives the same bits.
+// The hint is an earlier frame's, which a pile that forms outgrows by one class
+// in three or four frames, and the host stays few frames ahead of the device
+// (rp_world.cpp). After anything else may have changed (the state was set),
+// a frame is launched in two parts: its begin with every colour round, and,
+// once that has run, its substeps by its own hint.
 constexpr int BIG_AUTO = -1;
 constexpr int BIG_TAIL_T = 512;             // threads of that block: 256 items side by side
 constexpr int BIG_TAIL_ITEMS = 512;
@@ -217,8 +221,12 @@ struct KernelTimer {
     }
 };
 
+// A frame's launches, or one part of them: up to the lists and solve orders of
+// the frame, or its substeps.
+enum FramePart { FRAME_WHOLE, FRAME_BEGIN, FRAME_SUBSTEPS };
 hipError_t launch_frame(const DevWorld& w, const FrameParams& fp, hipStream_t st, KernelTimer* kt = nullptr,
-                        const BigScene* bigs = nullptr, int nbig = 0, const Recorder* rec = nullptr);
+                        const BigScene* bigs = nullptr, int nbig = 0, const Recorder* rec = nullptr,
+                        FramePart part = FRAME_WHOLE);
 // Adjoint of a recorded run for scenes with one dynamic body
 // (rp_adjoint.hip): abar [nb][13] is the adjoint of (x, q, v, w) at the end
 // of the record on entry and at its start on exit; gparam [nb][3] accumulates

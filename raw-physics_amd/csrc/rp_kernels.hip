@@ -1049,12 +1049,8 @@ static size_t stage_bytes(int group, int stage) {
     return group > 1 ? (size_t)(64 / group) * stage * sizeof(V3) : 0;
 }
 
-hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_t st, KernelTimer* kt,
-                        const BigScene* bigs, int nbig, const Recorder* rec) {
-    if (world.nb == 0) return hipSuccess;
-    DevWorld w = world;
-    KernelTimer none;
-    KernelTimer& t = kt ? *kt : none;
+static void launch_frame_begin(const DevWorld& w, const FrameParams& fp, hipStream_t st, KernelTimer& t,
+                               const BigScene* bigs, int nbig) {
     t.begin(KC_FRAME, st);
     if (!fp.forces_given) hipLaunchKernelGGL(k_frame_begin, dim3(cdiv(w.nb, 256)), dim3(256), 0, st, w, fp.gravity);
     hipLaunchKernelGGL(k_broad, dim3(w.ns), dim3(64), 0, st, w);
@@ -1067,6 +1063,16 @@ hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_
     hipLaunchKernelGGL(k_levels, dim3(w.ns), dim3(64), 0, st, w, fp.collisions ? 1 : 0, solve_pipelined(w) ? 1 : 0);
     for (int k = 0; k < nbig; ++k) big_colour(w, bigs[k], fp.collisions, st);
     t.end(st);
+}
+
+hipError_t launch_frame(const DevWorld& world, const FrameParams& fp, hipStream_t st, KernelTimer* kt,
+                        const BigScene* bigs, int nbig, const Recorder* rec, FramePart part) {
+    if (world.nb == 0) return hipSuccess;
+    DevWorld w = world;
+    KernelTimer none;
+    KernelTimer& t = kt ? *kt : none;
+    if (part != FRAME_SUBSTEPS) launch_frame_begin(w, fp, st, t, bigs, nbig);
+    if (part == FRAME_BEGIN) return hipGetLastError();
     // without large scenes, the solve kernel integrates its scenes' bodies for
     // the next substep
     bool fuse_integrate = nbig == 0;

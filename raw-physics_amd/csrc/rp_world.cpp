@@ -819,14 +819,20 @@ struct rp_world {
     std::vector<BigScene> view_big[kMaxViews];
     hipStream_t view_stream[kMaxViews] = {};
     struct FrameGraph {
-        hipGraphExec_t exec[kMaxViews] = {};
+        hipGraphExec_t exec[kMaxViews] = {};      // the frame; with large scenes, its substeps by the present plan
+        hipGraphExec_t begin[2][kMaxViews] = {};  // with large scenes, its begin: by the plan, with every colour round
         FrameParams fp;
-        uint64_t gen = 0;
-    } graph[2];                              // by FrameParams::record
+        uint64_t gen = 0, plan_gen = 0;
+    } graph[2];                                   // by FrameParams::record
     hipEvent_t fork_ev = nullptr, join_ev[kMaxViews] = {};
     uint64_t sched_gen = 1, views_gen = 0;  // schedule changes invalidate the views and the captured graphs
+    // large scenes: generation of the launch plan (plan_big), and whether the
+    // bodies were set since it last was made from a frame of their own
+    uint64_t plan_gen = 1;
+    bool plan_stale = true;
     // bounded queue: at most two chunks of frames in flight on each stream
     hipEvent_t chunk_done[2][kMaxViews] = {};
+    uint32_t chunk_frame = 0;     // frames counted by chunk_mark
     // differentiable runs (adjoint_forward / adjoint_backward): the record of
     // the last run, kept from run to run and grown as needed
     uint32_t ck_frames = 0;                 // frames of the recorded run, 0: none
@@ -880,8 +886,11 @@ static void adjoint_free(rp_world* w) {
     w->ck_frames = 0;
 }
 
-// Frames per chunk of the bounded launch queue.
-constexpr uint32_t kFramesPerChunk = 32;
+// Frames per chunk of the bounded launch queue: two chunks of 32 keep the
+// device busy. With large scenes, whose frames take milliseconds and whose
+// launches follow earlier frames, two of 4 (a pile forming in one call of 120
+// frames of 20000 bodies 12.3 -> 7.3 ms per frame, of 60000 25.8 -> 11.0).
+constexpr uint32_t kFramesPerChunk = 32, kBigFramesPerChunk = 4;
 
 static bool same_params(const FrameParams& a, const FrameParams& b) {
     return a.dt == b.dt && a.h == b.h && a.gravity == b.gravity && a.substeps == b.substeps && a.iters == b.iters &&
@@ -988,13 +997,17 @@ static bool build_views(rp_world* w) {
     return true;
 }
 
+static void drop_graph(hipGraphExec_t& e) {
+    if (e) (void)hipGraphExecDestroy(e);
+    e = nullptr;
+}
 static void drop_graphs(rp_world::FrameGraph& g) {
-    g.gen = 0;
-    for (hipGraphExec_t& e : g.exec)
-        if (e) {
-            (void)hipGraphExecDestroy(e);
-            e = nullptr;
-        }
+    g.gen = g.plan_gen = 0;
+    for (int k = 0; k < kMaxViews; ++k) {
+        drop_graph(g.exec[k]);
+        drop_graph(g.begin[0][k]);
+        drop_graph(g.begin[1][k]);
+    }
 }
 
 // How many colour classes and colour rounds of the large scenes to launch one
@@ -1003,7 +1016,6 @@ static void drop_graphs(rp_world::FrameGraph& g) {
 // kept while the scenes change little.
 static void plan_big(rp_world* w) {
     DevWorld& d = w->im.d;
-    if (w->im.big.empty()) return;
     int lead = 0, rounds = 0;
     for (const BigScene& b : w->im.big) {
         lead = std::max(lead, (int)__atomic_load_n(b.hint, __ATOMIC_RELAXED));
@@ -1019,45 +1031,124 @@ static void plan_big(rp_world* w) {
     if (!move) return;
     d.big_classes = classes;
     d.big_rounds = rnd;
-    ++w->sched_gen;
+    ++w->plan_gen;
 }
 
-// The graphs of one frame for these parameters and the current schedules,
-// captured once per view and reused while they do not change.
-static hipError_t frame_graph(rp_world* w, const FrameParams& fp) {
-    plan_big(w);
-    rp_world::FrameGraph& fg = w->graph[fp.record];
-    if (fg.gen == w->sched_gen && same_params(fg.fp, fp)) return hipSuccess;
+static void sync_views(rp_world* w) {
     (void)hipStreamSynchronize(w->stream);
     for (int k = 1; k < w->nviews; ++k) (void)hipStreamSynchronize(w->view_stream[k]);
-    drop_graphs(fg);
-    if (w->views_gen != w->sched_gen) {
-        w->views_gen = 0;
-        drop_graphs(w->graph[!fp.record]);  // (captured on the views that go)
-        if (!build_views(w)) return hipErrorOutOfMemory;
-        w->views_gen = w->sched_gen;
+}
+
+// One part of the frame on view k (the plan as it is now), as a graph.
+static hipError_t capture_part(rp_world* w, const FrameParams& fp, int k, FramePart part, bool every_round,
+                               hipGraphExec_t& out) {
+    DevWorld v = w->view[k];
+    v.big_classes = w->im.d.big_classes;
+    v.big_rounds = every_round ? BIG_COLOUR_ROUNDS : w->im.d.big_rounds;
+    Recorder rec = w->stage;
+    rec.p0 = w->view_p0[k];
+    hipStream_t st = w->view_stream[k];
+    hipGraph_t g = nullptr;
+    hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
+    if (e != hipSuccess) return e;
+    hipError_t le = launch_frame(v, fp, st, nullptr, w->view_big[k].data(), (int)w->view_big[k].size(),
+                                 fp.record ? &rec : nullptr, part);
+    e = hipStreamEndCapture(st, &g);
+    if (le != hipSuccess) e = le;
+    if (e == hipSuccess) e = hipGraphInstantiate(&out, g, nullptr, nullptr, 0);
+    if (g) (void)hipGraphDestroy(g);
+    return e;
+}
+
+// The graphs of one frame for these parameters, schedules and launch plan,
+// captured once per view and reused while they do not change. Where the plan
+// is stale, only the frame's begin with every colour round.
+static hipError_t frame_graph(rp_world* w, const FrameParams& fp) {
+    rp_world::FrameGraph& fg = w->graph[fp.record];
+    const bool big = !w->im.big.empty();
+    if (big && !w->plan_stale) plan_big(w);
+    if (fg.gen != w->sched_gen || !same_params(fg.fp, fp)) {
+        sync_views(w);
+        drop_graphs(fg);
+        if (w->views_gen != w->sched_gen) {
+            w->views_gen = 0;
+            drop_graphs(w->graph[!fp.record]);  // (captured on the views that go)
+            if (!build_views(w)) return hipErrorOutOfMemory;
+            w->views_gen = w->sched_gen;
+        }
+        fg.fp = fp;
+        fg.gen = w->sched_gen;
     }
-    for (int k = 0; k < w->nviews; ++k) {
-        hipStream_t st = w->view_stream[k];
-        hipGraph_t g = nullptr;
-        hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
-        if (e != hipSuccess) return e;
-        Recorder rec = w->stage;
-        rec.p0 = w->view_p0[k];
-        hipError_t le = launch_frame(w->view[k], fp, st, nullptr, w->view_big[k].data(), (int)w->view_big[k].size(),
-                                     fp.record ? &rec : nullptr);
-        e = hipStreamEndCapture(st, &g);
-        if (le != hipSuccess) e = le;
-        if (e == hipSuccess) e = hipGraphInstantiate(&fg.exec[k], g, nullptr, nullptr, 0);
-        if (g) (void)hipGraphDestroy(g);
-        if (e != hipSuccess) {
-            drop_graphs(fg);
-            return e;
+    const bool planned = !big || !w->plan_stale;
+    hipError_t e = hipSuccess;
+    if (planned && fg.plan_gen != w->plan_gen) {
+        sync_views(w);
+        for (int k = 0; k < w->nviews; ++k) {
+            drop_graph(fg.exec[k]);
+            drop_graph(fg.begin[0][k]);
+        }
+        for (int k = 0; e == hipSuccess && k < w->nviews; ++k) {
+            if (big) e = capture_part(w, fp, k, FRAME_BEGIN, false, fg.begin[0][k]);
+            if (e == hipSuccess) e = capture_part(w, fp, k, big ? FRAME_SUBSTEPS : FRAME_WHOLE, false, fg.exec[k]);
+        }
+        if (e == hipSuccess) fg.plan_gen = w->plan_gen;
+    }
+    for (int k = 0; e == hipSuccess && !planned && k < w->nviews; ++k)
+        if (!fg.begin[1][k]) e = capture_part(w, fp, k, FRAME_BEGIN, true, fg.begin[1][k]);
+    if (e != hipSuccess) {
+        sync_views(w);
+        drop_graphs(fg);
+    }
+    return e;
+}
+
+// The plan of a frame that has begun, on every view.
+static hipError_t plan_begun(rp_world* w) {
+    hipError_t e = hipStreamSynchronize(w->stream);
+    for (int k = 1; e == hipSuccess && k < w->nviews; ++k) e = hipStreamSynchronize(w->view_stream[k]);
+    if (e != hipSuccess) return e;
+    w->plan_stale = false;
+    plan_big(w);
+    return e;
+}
+
+// One frame on every view's stream.
+static hipError_t replay_frame(rp_world* w, const FrameParams& fp) {
+    const rp_world::FrameGraph& fg = w->graph[fp.record];
+    const bool big = !w->im.big.empty();
+    hipError_t e = hipSuccess;
+    if (big) {
+        e = frame_graph(w, fp);
+        const bool stale = w->plan_stale;
+        for (int k = 0; e == hipSuccess && k < w->nviews; ++k) e = hipGraphLaunch(fg.begin[stale][k], w->view_stream[k]);
+        if (e == hipSuccess && stale) {
+            e = plan_begun(w);
+            if (e == hipSuccess) e = frame_graph(w, fp);
         }
     }
-    fg.fp = fp;
-    fg.gen = w->sched_gen;
-    return hipSuccess;
+    for (int k = 0; e == hipSuccess && k < w->nviews; ++k) e = hipGraphLaunch(fg.exec[k], w->view_stream[k]);
+    return e;
+}
+
+// One frame of the whole world, launched kernel by kernel on its stream. `d`:
+// the world's layout, or the caller's copy of it.
+static hipError_t launch_planned(rp_world* w, DevWorld d, const FrameParams& fp, KernelTimer* kt, const Recorder* rec) {
+    const BigScene* bigs = w->im.big.data();
+    const int nbig = (int)w->im.big.size();
+    if (nbig == 0) return launch_frame(d, fp, w->stream, kt, bigs, nbig, rec);
+    hipError_t e = hipSuccess;
+    if (w->plan_stale) {
+        d.big_rounds = BIG_COLOUR_ROUNDS;
+        e = launch_frame(d, fp, w->stream, kt, bigs, nbig, rec, FRAME_BEGIN);
+        if (e == hipSuccess) e = plan_begun(w);
+        d.big_classes = w->im.d.big_classes;
+        if (e == hipSuccess) e = launch_frame(d, fp, w->stream, kt, bigs, nbig, rec, FRAME_SUBSTEPS);
+        return e;
+    }
+    plan_big(w);
+    d.big_classes = w->im.d.big_classes;
+    d.big_rounds = w->im.d.big_rounds;
+    return launch_frame(d, fp, w->stream, kt, bigs, nbig, rec);
 }
 
 static bool world_init(rp_world* w) {
@@ -1102,19 +1193,28 @@ static void world_free(rp_world* w) {
     delete w;
 }
 
-// Keeps the stream's queue bounded: after each chunk of frames an event is
+// Keeps the streams' queues bounded: after each chunk of frames an event is
 // recorded, and the host waits for the chunk before the previous one, so at
-// most two chunks are queued while the device always has one to run.
-static hipError_t chunk_mark(rp_world* w, uint32_t f, int view, hipStream_t st) {
-    if ((f + 1) % kFramesPerChunk != 0) return hipSuccess;
-    uint32_t k = (f + 1) / kFramesPerChunk;
+// most two chunks are queued while the device always has one to run. The
+// frames of one call are counted; with large scenes, whose plan follows the
+// frames that have run, those of every call.
+static hipError_t chunk_mark(rp_world* w, uint32_t f, int views) {
+    const bool big = !w->im.big.empty();
+    const uint32_t frames = big ? kBigFramesPerChunk : kFramesPerChunk;
+    w->chunk_frame = big ? w->chunk_frame + 1 : f + 1;
+    if (w->chunk_frame % frames != 0) return hipSuccess;
+    uint32_t c = w->chunk_frame / frames;
     hipError_t e = hipSuccess;
-    if (k >= 2) e = hipEventSynchronize(w->chunk_done[k & 1][view]);
-    if (e == hipSuccess) e = hipEventRecord(w->chunk_done[k & 1][view], st);
+    for (int k = 0; e == hipSuccess && k < views; ++k) {
+        if (c >= 2) e = hipEventSynchronize(w->chunk_done[c & 1][k]);
+        if (e == hipSuccess) e = hipEventRecord(w->chunk_done[c & 1][k], k ? w->view_stream[k] : w->stream);
+    }
     return e;
 }
 
 static uint32_t world_run(rp_world* w, const FrameParams& fp, uint32_t frames, bool sync) {
+    // (other items than the last frame's)
+    if (fp.collisions != w->last_collisions) w->plan_stale = true;
     w->last_collisions = fp.collisions;
     if (w->use_graphs && !w->timer.on && frames > 0) {
         hipError_t e = frame_graph(w, fp);
@@ -1125,12 +1225,8 @@ static uint32_t world_run(rp_world* w, const FrameParams& fp, uint32_t frames, b
             for (int k = 1; e == hipSuccess && k < w->nviews; ++k) e = hipStreamWaitEvent(w->view_stream[k], w->fork_ev, 0);
         }
         for (uint32_t f = 0; e == hipSuccess && f < frames; ++f) {
-            // a long run looks at the large scenes again once per chunk
-            if (f > 0 && f % kFramesPerChunk == 0 && !w->im.big.empty() && w->nviews == 1) e = frame_graph(w, fp);
-            for (int k = 0; e == hipSuccess && k < w->nviews; ++k) {
-                e = hipGraphLaunch(w->graph[fp.record].exec[k], w->view_stream[k]);
-                if (e == hipSuccess) e = chunk_mark(w, f, k, w->view_stream[k]);
-            }
+            e = replay_frame(w, fp);
+            if (e == hipSuccess) e = chunk_mark(w, f, w->nviews);
         }
         for (int k = 1; e == hipSuccess && k < w->nviews; ++k) {
             e = hipEventRecord(w->join_ev[k], w->view_stream[k]);
@@ -1138,18 +1234,15 @@ static uint32_t world_run(rp_world* w, const FrameParams& fp, uint32_t frames, b
         }
         if (e != hipSuccess) {
             set_msg(std::string("frame graph: ") + hipGetErrorString(e));
-            // (views that were launched but not joined)
-            for (int k = 0; k < w->nviews; ++k) (void)hipStreamSynchronize(w->view_stream[k]);
+            sync_views(w);  // (views that were launched but not joined)
             return RP_ERR_RUNTIME;
         }
         frames = 0;
     }
     for (uint32_t f = 0; f < frames; ++f) {
         w->timer.used = 0;
-        plan_big(w);
-        hipError_t e = launch_frame(w->im.d, fp, w->stream, &w->timer, w->im.big.data(), (int)w->im.big.size(),
-                                    fp.record ? &w->stage : nullptr);
-        if (e == hipSuccess && !w->timer.on) e = chunk_mark(w, f, 0, w->stream);
+        hipError_t e = launch_planned(w, w->im.d, fp, &w->timer, fp.record ? &w->stage : nullptr);
+        if (e == hipSuccess && !w->timer.on) e = chunk_mark(w, f, 1);
         if (e != hipSuccess) {
             set_msg(std::string("kernel launch: ") + hipGetErrorString(e));
             return RP_ERR_RUNTIME;
@@ -1244,7 +1337,6 @@ uint32_t rp_world_step_noalloc(rp_world* w, double dt, uint32_t frames, uint32_t
     // the world's kernels with the lane-group working memory in the static
     // array; the narrow-phase grids are capped to the groups it holds (lane
     // groups take the live pairs in grid-stride order: identical results)
-    plan_big(w);
     DevWorld d = w->im.d;
     int64_t slots = (int64_t)(NOALLOC_SCRATCH_BYTES / GROUP_WORK_BYTES);
     if (d.narrow_group > 1) d.narrow_blocks = (int)std::min<int64_t>(d.narrow_blocks, slots / (64 / d.narrow_group));
@@ -1263,10 +1355,11 @@ uint32_t rp_world_step_noalloc(rp_world* w, double dt, uint32_t frames, uint32_t
     fp.substeps = substeps;
     fp.iters = iters;
     fp.collisions = coll != 0;
+    if (fp.collisions != w->last_collisions) w->plan_stale = true;
     w->last_collisions = fp.collisions;
     for (uint32_t f = 0; f < frames; ++f) {
-        hipError_t e = launch_frame(d, fp, w->stream, nullptr, w->im.big.data(), (int)w->im.big.size());
-        if (e == hipSuccess) e = chunk_mark(w, f, 0, w->stream);
+        hipError_t e = launch_planned(w, d, fp, nullptr, nullptr);
+        if (e == hipSuccess) e = chunk_mark(w, f, 1);
         if (e != hipSuccess) {
             set_msg(std::string("kernel launch: ") + hipGetErrorString(e));
             return g_last_err = RP_ERR_RUNTIME;
@@ -1342,6 +1435,7 @@ void rp_world_set_state(rp_world* w, const rp_state* in) {
         hipMemcpyAsync(w->state_dev, w->state_pin, bytes, hipMemcpyHostToDevice, w->stream) != hipSuccess)
         return;
     (void)launch_state_in(w->im.d, w->state_dev, mask, w->stream);
+    w->plan_stale = true;
 }
 
 uint32_t rp_world_error(rp_world* w, uint32_t scene) {
@@ -2088,8 +2182,16 @@ extern "C" uint32_t rp_pbd_simulate(double dt, rp_entity** ents, rp_constraint* 
         if (dropin_build(ents, n, cons, tmp, e2) && !tmp.ext.empty())
             (void)hipMemcpy((void*)w->im.d.ext, tmp.ext.data(), tmp.ext.size() * sizeof(ExtC), hipMemcpyHostToDevice);
     }
+    // whether the entities go on from the last call (large scenes' launch plan)
+    bool same = !w->im.big.empty() && w->host_bodies.size() == n;
     w->host_bodies.resize(n);
-    for (size_t i = 0; i < n; ++i) w->host_bodies[i] = entity_body(ents[i]);
+    for (size_t i = 0; i < n; ++i) {
+        const Body b = entity_body(ents[i]);
+        Body& last = w->host_bodies[i];
+        same = same && memcmp(&b, &last, offsetof(Body, inv_mass)) == 0 && b.fixed == last.fixed && b.active == last.active;
+        last = b;
+    }
+    if (!same) w->plan_stale = true;
     if (!upload_bodies(w)) return g_last_err = RP_ERR_RUNTIME;
     (void)hipMemset(w->im.d.scene_err, 0, 4);
     FrameParams fp;

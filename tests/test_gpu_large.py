@@ -250,3 +250,40 @@ def test_stale_launch_plan_gives_identical_bits(iters):
         assert g.error(0) == 0
         got.append(g.state())
     assert not state_bits_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("others", [0, 70])
+def test_stale_launch_plan_costs_little(others):
+    """A world of falling bodies (few classes and rounds launched) that is set
+    to a settled pile and stepped 32 frames in one call, alone and with enough
+    small scenes beside it for concurrent views: within 1.5x of a world in the
+    same state that launches every class (nearly four times that before the
+    first frame after a set state planned its own launches)."""
+    import time
+
+    w = _large(True, n=20000)
+    for s in range(others):
+        scenes.drop_scene(w, 3000 + s, n_cubes=1, n_icos=0)
+    g = SimWorld("rp", w)
+    start = g.state()
+    g.step(220)
+    pile = g.state()
+
+    def frames_32(sim):
+        sim.step(3)
+        sim.step(3)
+        sim.set_state(pile)
+        t = time.perf_counter()
+        sim.step(32)
+        return time.perf_counter() - t, sim.state()
+
+    g.set_state(start)
+    got, st = frames_32(g)
+    full = SimWorld("rp", w)
+    assert full.lib.rp_world_set_colour_launches(full.h, 64) == 0
+    full.set_state(pile)
+    full.step(32)  # (its colour rounds follow the pile's too)
+    want, st_full = frames_32(full)
+    print(f"{1e3 * got / 32:.2f} ms per frame after falling, {1e3 * want / 32:.2f} with every class launched")
+    assert not state_bits_equal(st, st_full)
+    assert got <= 1.5 * want
