@@ -125,7 +125,7 @@ constexpr int BIG_COLOUR_ROUNDS = 64;       // Jones-Plassmann rounds per frame 
 // The hint is an earlier frame's, which a pile that forms outgrows by one class
 // in three or four frames, and the host stays few frames ahead of the device
 // (rp_world.cpp). After anything else may have changed (the state was set),
-// a frame is launched in two parts: its begin with every colour round, and,
+// a frame is launched in two parts: its begin with more colour rounds, and,
 // once that has run, its substeps by its own hint.
 constexpr int BIG_AUTO = -1;
 constexpr int BIG_TAIL_T = 512;             // threads of that block: 256 items side by side

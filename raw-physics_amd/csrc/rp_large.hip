@@ -506,32 +506,44 @@ __global__ void k_big_colour_round(DevWorld w, BigScene b, int collisions, int r
         dst[t] = ct;
     }
 }
-// The rounds from `round` (even) on that a frame still needs, on one block:
-// none where the launched rounds coloured every item.
+// The rounds from `round` on that a frame still needs, on one block: none where
+// the launched rounds coloured every item. The block lists the uncoloured items
+// once (`list`, in any order) and then goes over them only: `next` takes their
+// colours of a round before any is stored, so that, as above, a round reads the
+// one before it. (Going over all items each round took 1.7 ms per round of a
+// settled pile of 60000 bodies, 0.4 over the tenth of them that is left after
+// 32 rounds.)
 __global__ void __launch_bounds__(1024) k_big_colour_rest(DevWorld w, BigScene b, int collisions, int round, int* colour,
-                                                          int* spare) {
-    int K = min(big_items(w, b, collisions), b.item_cap);
-    __shared__ int left;
-    for (; round < BIG_COLOUR_ROUNDS; ++round) {
-        __syncthreads();
-        if (threadIdx.x == 0) left = __hip_atomic_load(b.remaining, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        if (left == 0) break;
-        if (threadIdx.x == 0) b.remaining[1] = round + 1;
-        const int* src = (round & 1) ? spare : colour;
-        int* dst = (round & 1) ? colour : spare;
-        for (int t = threadIdx.x; t < K; t += blockDim.x) {
-            int ct = src[t];
-            if (ct < 0) {
-                ct = colour_item(w, b, src, t);
-                if (ct >= 0) atomicSub(b.remaining, 1);
-            }
-            dst[t] = ct;
-        }
+                                                          int* list, int* next) {
+    const int K = min(big_items(w, b, collisions), b.item_cap);
+    __shared__ int n, left;
+    if (threadIdx.x == 0) {
+        n = 0;
+        left = __hip_atomic_load(b.remaining, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    if (round & 1)
-        for (int t = threadIdx.x; t < K; t += blockDim.x) colour[t] = spare[t];
+    if (left == 0) return;
+    for (int t = threadIdx.x; t < K; t += blockDim.x)
+        if (colour[t] < 0) list[atomicAdd(&n, 1)] = t;
+    __syncthreads();
+    for (; round < BIG_COLOUR_ROUNDS; ++round) {
+        if (threadIdx.x == 0) b.remaining[1] = round + 1;
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            int t = list[i];
+            next[i] = colour[t] < 0 ? colour_item(w, b, colour, t) : -1;
+        }
+        __syncthreads();
+        int coloured = 0;
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            int c = next[i];
+            if (c < 0) continue;
+            colour[list[i]] = c;
+            ++coloured;
+        }
+        if (coloured) atomicSub(&left, coloured);
+        __syncthreads();
+        if (left == 0) break;
+    }
 }
 
 // Items still uncoloured join the serial class; class sizes and starts.
@@ -631,7 +643,8 @@ void big_colour(const DevWorld& w, const BigScene& b, bool collisions, hipStream
         hipLaunchKernelGGL(k_big_colour_round, dim3(gi), dim3(256), 0, st, w, b, co, r, (r & 1) ? spare : colour,
                            (r & 1) ? colour : spare);
     if (rounds < BIG_COLOUR_ROUNDS)
-        hipLaunchKernelGGL(k_big_colour_rest, dim3(1), dim3(1024), 0, st, w, b, co, rounds, colour, spare);
+        hipLaunchKernelGGL(k_big_colour_rest, dim3(1), dim3(1024), 0, st, w, b, co, rounds, colour, spare,
+                           w.item_cursor + b.item_base + b.s);
     hipLaunchKernelGGL(k_big_classes, dim3(1), dim3(1024), 0, st, w, b, co);
     hipLaunchKernelGGL(k_big_cursor, dim3(1), dim3(64), 0, st, w, b);
     hipLaunchKernelGGL(k_big_serial_flags, dim3(gi), dim3(256), 0, st, w, b, co);

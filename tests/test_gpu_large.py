@@ -287,3 +287,29 @@ def test_stale_launch_plan_costs_little(others):
     print(f"{1e3 * got / 32:.2f} ms per frame after falling, {1e3 * want / 32:.2f} with every class launched")
     assert not state_bits_equal(st, st_full)
     assert got <= 1.5 * want
+
+
+@pytest.mark.parametrize("n,frames", [(400, 160), (3000, 150)])
+def test_colour_rounds_on_one_block_give_identical_bits(n, frames):
+    """The colour rounds beyond the launched ones, on one block: a world that
+    was falling finishes a settled pile's 50 rounds there, a new world launches
+    every round; both give the same classes and bits."""
+    w = _large(True, n=n, seed=4)
+    pile = SimWorld("rp", w)
+    start = pile.state()
+    pile.step(frames)
+    st = pile.state()
+    fresh, fell = SimWorld("rp", w), SimWorld("rp", w)
+    for _ in range(4):
+        fell.step(1)
+    for g in (fresh, fell):
+        g.set_state(st)
+        g.step(1)
+    assert np.array_equal(_classes(fresh), _classes(fell))
+    assert not state_bits_equal(fresh.state(), fell.state())
+    fell.set_state(start)  # and back: the pile's plan for falling bodies
+    fell.step(2)
+    again = SimWorld("rp", w)
+    again.step(2)
+    assert not state_bits_equal(again.state(), fell.state())
+    assert fell.error(0) == 0
