@@ -29,7 +29,8 @@ struct DevWorld {
     int small_nv;                   // > 0: pairs of two hulls of <= small_nv vertices go to their own list
     int stage_small;                // LDS vertices per pair of that list: 2 x small_nv
     int small_bodies;               // most bodies of a scene that is not large
-    int solve_lanes;                // lanes per scene in the solve: 64, 32 or 16
+    int solve_lanes;                // lanes per scene in the solve: 32, 16, or 64: whole waves (solve_width)
+    int all_scenes;                 // scenes of the whole world (views are launched side by side)
     int big_launch_classes;         // large scenes: colour classes solved one launch each, the rest in one block (BIG_AUTO: big_classes)
     int big_classes, big_rounds;    // the host's present choice of launched classes and colour rounds
     // scenes

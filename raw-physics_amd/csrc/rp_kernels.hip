@@ -964,24 +964,38 @@ static void launch_solve_lanes(const DevWorld& w, const FrameParams& fp, hipStre
     else
         hipLaunchKernelGGL((k_solve<kExt, LPS, false>), grid, block, 0, st, w, fp.h, it, co, integrate_next, 0);
 }
-// Whole waves per scene (solve_lanes 64): one, two per sweep with joints (a wave solves a
-// joint and a contact one after the other: 500 chains of 6 links 7.3 / 6.5 / 6.7
-// ms per frame at 64 / 128 / 256 lanes per sweep), and four per sweep for scenes
-// of more than 64 bodies, whose steps have more items (150 scenes of 4 to 256
-// bodies 6.6 / 6.1 / 5.8). Scenes of 16 bodies lose by more waves at every
-// barrier (one scene 0.89 / 0.95 / 1.08, 1000 scenes 1.7 / 1.9 / 2.7).
+// Lanes per sweep and scene where whole waves serve a scene (solve_lanes 64).
+// One width serves every scene of the world, so it also follows how many there
+// are: with one wave per SIMD slot taken by a small scene's idle waves, the
+// others wait. ms per frame of worlds of n scenes at 64 / 128 / 256 lanes:
+//   above 64 bodies, whose steps have many items: four waves per sweep while
+//   their blocks fit one to a CU, two up to four times as many
+//     150 of 4 to 256 bodies     7.3 /  6.3 /  6.0   256 of them      7.7 /  6.5 /  6.2
+//     600 of them                9.7 /  8.6 /  9.3   1500 of them    15.9 / 17.4 / 20.0
+//     512 of 66 bodies           2.8 /  2.6 /  3.3   3000 of them    11.1 / 13.3 / 18.0
+//     256 of 16 and one of 66    1.9 /  1.7 /  1.8   1500 and one     2.3 /  2.3 /  3.4
+//   with joints: two (a wave solves a joint and a contact one after the other)
+//   up to three scenes per CU
+//     500 chains of 6 links      7.3 /  6.5          600 of them      7.3 /  6.6
+//     800 of them                7.4 /  7.6          1200 of them     7.7 /  9.6
+//   others: one (one scene of 16 bodies 0.89 / 0.95 / 1.08, 1000 scenes 1.7 /
+//   1.9 / 2.7).
+static int solve_width(const DevWorld& w) {
+    if (w.solve_lanes < 64) return w.solve_lanes;
+    if (w.small_bodies > 64) return w.all_scenes <= 256 ? 256 : w.all_scenes <= 1024 ? 128 : 64;
+    return w.n_ext > 0 && w.all_scenes <= 768 ? 128 : 64;
+}
 static bool solve_pipelined(const DevWorld& w) {  // kPipe of the kernel that launch_solve takes
-    return w.n_ext > 0 || (w.solve_lanes == 64 && w.small_bodies > 64);
+    return w.n_ext > 0 || solve_width(w) > 64;
 }
 template <bool kExt>
 static void launch_solve(const DevWorld& w, const FrameParams& fp, hipStream_t st, int integrate_next) {
-    switch (w.solve_lanes) {
+    switch (solve_width(w)) {
     case 16: launch_solve_lanes<kExt, 16>(w, fp, st, integrate_next); break;
     case 32: launch_solve_lanes<kExt, 32>(w, fp, st, integrate_next); break;
-    default:
-        if (w.small_bodies > 64) launch_solve_lanes<kExt, 256>(w, fp, st, integrate_next);
-        else launch_solve_lanes<kExt, kExt ? 128 : 64>(w, fp, st, integrate_next);
-        break;
+    case 64: launch_solve_lanes<kExt, 64>(w, fp, st, integrate_next); break;
+    case 128: launch_solve_lanes<kExt, 128>(w, fp, st, integrate_next); break;
+    default: launch_solve_lanes<kExt, 256>(w, fp, st, integrate_next); break;
     }
 }
 

@@ -386,7 +386,7 @@ struct DeviceImage {
 static bool build_image(const HostWorld& hw, DeviceImage& im) {
     DevWorld& d = im.d;
     memset(&d, 0, sizeof(d));
-    d.ns = (int)hw.scene_body_off.size() - 1;
+    d.ns = d.all_scenes = (int)hw.scene_body_off.size() - 1;
     d.nb = (int)hw.body.size();
     d.n_ext = (int)hw.ext.size();
     // topology dedupe: bodies of the same shape share index lists

@@ -168,3 +168,62 @@ def test_scene_beyond_the_level_sort_lds_bit_exact():
                    scenes.quaternion_new((0.0, 1.0, 0.0), 3.0 * (k % 7)))
     w.end_scene()
     _compare(w, frames=24, check_every=8, iters=2)
+
+
+@pytest.mark.parametrize("joints", [False, True])
+@pytest.mark.parametrize("large", [False, True])
+@pytest.mark.parametrize("others", [300, 800, 1100])
+def test_solve_widths_bit_exact(others, large, joints):
+    """The waves that serve a scene follow the number of scenes: a pile, a
+    stack of 66 boxes and a chain among few and among many scenes keep their
+    bits (against the oracle without joints)."""
+    def world(n):
+        w = scenes.World(name=f"among_{n}")
+        scenes.drop_scene(w, 51, n_cubes=7, n_icos=7)
+        if large:
+            scenes.stack_scene(w, seed=3, num_cubes=66)
+        if joints:
+            scenes.chain_scene(w, 77, length=5)
+        for s in range(n):
+            scenes.drop_scene(w, 5000 + s, n_cubes=1, n_icos=0)
+        return w
+
+    few, many = world(0), world(others)
+    g, h = SimWorld("rp", few), SimWorld("rp", many)
+    o = SimWorld("orc", few)
+    nb = few.num_bodies
+    for f in range(3):
+        for sim in (g, h, o):
+            sim.step(15, iters=2)
+        same = {k: v[:nb] for k, v in h.state().items()}
+        assert not state_bits_equal(g.state(), same), f"after frame {15 * f + 15}"
+        if not joints:
+            assert not state_bits_equal(o.state(), same), f"after frame {15 * f + 15}"
+    assert not any(g.error(s) for s in range(few.num_scenes))
+    assert not any(h.error(s) for s in range(many.num_scenes))
+
+
+def test_one_large_scene_among_many_small_ones_costs_little():
+    """A scene of 66 bodies among 3000 small ones: the solve's waves per scene
+    are not chosen by it alone (2.8 times the frame without it when they were)."""
+    import time
+
+    def frame_ms(extra):
+        w = scenes.World(name="many")
+        if extra:
+            scenes.drop_scene(w, 9001, n_cubes=33, n_icos=32)
+        for s in range(3000):
+            scenes.drop_scene(w, s)
+        g = SimWorld("rp", w)
+        g.step(100)
+        st, ms = g.state(), []
+        for _ in range(5):
+            g.set_state(st)
+            t = time.perf_counter()
+            g.step(10)
+            ms.append(100.0 * (time.perf_counter() - t))
+        return min(ms)
+
+    alone, beside = frame_ms(False), frame_ms(True)
+    print(f"{alone:.2f} ms per frame, {beside:.2f} with a scene of 66 bodies")
+    assert beside <= 1.7 * alone
