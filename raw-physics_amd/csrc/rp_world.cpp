@@ -568,8 +568,12 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
     // the device's SIMDs, then as many scenes per wave as keep the waves
     // within what it holds (16-body scenes, ms per frame at 64 / 32 / 16
     // lanes: 64 scenes 1.54 / 1.56 / 1.77, 2048 scenes 2.68 / 2.52 / 2.76,
-    // 4096 scenes 4.17 / 3.89 / 4.22, 8192 scenes 6.81 / 6.23 / 6.15)
-    d.solve_lanes = d.ns < 1536 || d.small_bodies > 64 ? 64 : d.ns < 8192 ? 32 : 16;
+    // 4096 scenes 4.17 / 3.89 / 4.22, 8192 scenes 6.81 / 6.23 / 6.15). Two
+    // scenes per wave pay while eight such waves' bodies fit a CU's LDS (3000
+    // scenes of 20 bodies 3.27 / 3.03 ms at 64 / 32 lanes, of 22 3.85 / 4.28;
+    // 1600 of 60 bodies 5.52 / 6.39)
+    const bool two_fit = 8 * 2 * (size_t)d.small_bodies * sizeof(Body) <= 160 * 1024;
+    d.solve_lanes = d.ns < 1536 || d.small_bodies > 64 ? 64 : d.ns >= 8192 ? 16 : two_fit ? 32 : 64;
     d.big_launch_classes = BIG_AUTO;
     d.big_classes = BIG_CLASSES;
     d.big_rounds = BIG_COLOUR_ROUNDS;

@@ -227,3 +227,25 @@ def test_one_large_scene_among_many_small_ones_costs_little():
     alone, beside = frame_ms(False), frame_ms(True)
     print(f"{alone:.2f} ms per frame, {beside:.2f} with a scene of 66 bodies")
     assert beside <= 1.7 * alone
+
+
+@pytest.mark.parametrize("bodies,lanes", [(6, 32), (30, 64)])
+def test_two_scenes_per_wave_only_where_their_bodies_fit(bodies, lanes):
+    """Many scenes share a wave by twos while the bodies of the waves that a CU
+    holds fit its LDS; scenes of 30 bodies are faster with a wave each. The
+    bits do not depend on it."""
+    w = scenes.World(name="many")
+    for s in range(1600):
+        scenes.drop_scene(w, s % 40, n_cubes=bodies // 2, n_icos=bodies // 2)
+    g = SimWorld("rp", w)
+    assert g.lib.rp_world_solve_lanes(g.h) == lanes
+    few = scenes.World(name="few")
+    for s in range(40):
+        scenes.drop_scene(few, s, n_cubes=bodies // 2, n_icos=bodies // 2)
+    o = SimWorld("orc", few)
+    g.step(60)
+    o.step(60)
+    st = g.state()
+    for k in (0, 39):
+        part = {n: v[k * few.num_bodies:(k + 1) * few.num_bodies] for n, v in st.items()}
+        assert not state_bits_equal(o.state(), part), f"copy {k}"
