@@ -24,7 +24,8 @@ struct DevWorld {
     int manifold_group;             // lanes per pair in the contact manifold: 1, 4, 8, 16
     int manifold_blocks;
     int narrow_block_cap;           // most blocks of a narrow-phase launch (0: the default, 8192)
-    int lds_limit;                  // dynamic LDS bytes one block may use on the world's device
+    int lds_limit;                  // dynamic LDS bytes a narrow-phase block may use
+    int solve_lds;                  // dynamic LDS bytes a solve block may use on the world's device
     int stage_cap;                  // LDS vertices per pair: 2 x the largest hull
     int small_nv;                   // > 0: pairs of two hulls of <= small_nv vertices go to their own list
     int stage_small;                // LDS vertices per pair of that list: 2 x small_nv
@@ -281,8 +282,14 @@ bool narrow_group_supported(const DevWorld& w, int g);
 // Lets the lane-group narrow-phase kernels take up to `bytes` of dynamic LDS
 // per block (gfx950 gives a workgroup up to 160 KiB).
 hipError_t allow_narrow_lds(int bytes);
-// Lets the solve of scenes above 64 bodies hold them in more than 64 KiB of LDS.
-hipError_t allow_solve_lds();
+// Bodies in LDS per solve block: 64 KiB, and with eight waves per scene up to
+// 150 KiB (one block per CU), less what the block vote takes where the device
+// has no more than that. Scenes of 4 to 256 bodies, ms per frame with the
+// bodies in L2 and in LDS: 150 scenes 5.72 / 5.65, 40 with two iterations 6.21 /
+// 6.07.
+constexpr int SOLVE_LDS_LIMIT = 64 * 1024, SOLVE_LDS_WIDE = 150 * 1024, SOLVE_LDS_VOTE = 1024;
+// Lets the solve of scenes above 64 bodies hold them in `bytes` of LDS.
+hipError_t allow_solve_lds(int bytes);
 int narrow_blocks_for(const DevWorld& w, int g, int64_t pair_capacity);
 hipError_t launch_fp64_selftest(const double* a, const double* b, double* out, int64_t n, hipStream_t st);
 

@@ -690,11 +690,6 @@ __global__ void __launch_bounds__(64) k_levels(DevWorld w, int collisions, int p
 // went from 3.07 to 2.81 ms, a scene of 16 bodies from 25 to 20 us per launch.
 constexpr int BODY_VECS = sizeof(Body) / sizeof(int4);
 constexpr int STATE_VECS = offsetof(Body, deact) / sizeof(int4);  // x, q, v, w, px, pq, pv, pw
-// Bodies in LDS per block: 64 KiB, and with eight waves per scene up to 150 KiB
-// (one block per CU; its block vote takes some of the 160 KiB). Scenes of 4 to
-// 256 bodies, ms per frame with the bodies in L2 and in LDS: 150 scenes 5.72 /
-// 5.65, 40 with two iterations 6.21 / 6.07, 600 6.53 / 6.36.
-constexpr int SOLVE_LDS_LIMIT = 64 * 1024, SOLVE_LDS_WIDE = 150 * 1024;
 static_assert(sizeof(Body) % sizeof(int4) == 0 && offsetof(Body, deact) % sizeof(int4) == 0, "copied as 16-byte words");
 
 // In worlds with joints, and for scenes on several waves, sweeps are pipelined
@@ -947,7 +942,7 @@ k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next, int
 static size_t solve_lds_bytes(const DevWorld& w, int lanes, int blocks) {
     int scenes = std::max(1, 64 / lanes), waves = lanes > 64 ? 2 * lanes / 64 : 1;
     size_t bytes = (size_t)scenes * w.small_bodies * sizeof(Body);
-    if (bytes == 0 || bytes > (size_t)(lanes == 256 ? SOLVE_LDS_WIDE : SOLVE_LDS_LIMIT)) return 0;
+    if (bytes == 0 || bytes > (size_t)(lanes == 256 ? w.solve_lds : std::min(w.solve_lds, SOLVE_LDS_LIMIT))) return 0;
     size_t per_cu = std::min<size_t>(8 / waves, 160 * 1024 / bytes);
     return per_cu * waves == 8 || (size_t)blocks <= 256 * per_cu ? bytes : 0;
 }
@@ -1262,9 +1257,9 @@ hipError_t allow_narrow_lds(int bytes) {
     return hipSuccess;
 }
 
-hipError_t allow_solve_lds() {
+hipError_t allow_solve_lds(int bytes) {
     for (const void* f : {(const void*)k_solve<false, 256, true>, (const void*)k_solve<true, 256, true>}) {
-        hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, SOLVE_LDS_WIDE);
+        hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -528,17 +528,17 @@ static bool build_image(const HostWorld& hw, DeviceImage& im) {
     // device's limit per block (160 KiB on gfx950), for hulls that would
     // otherwise have no lane-group schedule; such worlds run lane groups in
     // the fused kernel only (large_lds_split)
+    int dev = 0, block_lds = 64 * 1024, lim = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && lim > 0)
+        block_lds = lim;
     d.lds_limit = 64 * 1024;
-    if ((size_t)(64 / 16) * d.stage_cap * sizeof(V3) > (size_t)d.lds_limit) {
-        int dev = 0, lim = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
-            lim > d.lds_limit) {
-            d.lds_limit = lim;
-            RP_CHECK(allow_narrow_lds(lim));
-        }
+    if ((size_t)(64 / 16) * d.stage_cap * sizeof(V3) > (size_t)d.lds_limit && block_lds > d.lds_limit) {
+        d.lds_limit = block_lds;
+        RP_CHECK(allow_narrow_lds(block_lds));
     }
-    if (d.small_bodies > 64) RP_CHECK(allow_solve_lds());
+    d.solve_lds = std::min(SOLVE_LDS_WIDE, block_lds - SOLVE_LDS_VOTE);
+    if (d.small_bodies > 64 && d.solve_lds > SOLVE_LDS_LIMIT) RP_CHECK(allow_solve_lds(d.solve_lds));
     // size classes: with hulls above SMALL_HULL_NV vertices, the pairs of two
     // smaller hulls get their own list and LDS slices sized for them (if the
     // large-hull pairs fit a 16-lane schedule)

@@ -191,7 +191,7 @@ def _run_with_runtime(tmp_path, runtime, code):
 
     src, so = tmp_path / "runtime.c", tmp_path / "runtime.so"
     src.write_text(runtime)
-    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src), "-ldl"], check=True)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-I/opt/rocm/include", "-o", str(so), str(src), "-ldl"], check=True)
     r = subprocess.run([sys.executable, "-c", code, str(ROOT), str(so)], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
 

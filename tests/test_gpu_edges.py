@@ -249,3 +249,60 @@ def test_two_scenes_per_wave_only_where_their_bodies_fit(bodies, lanes):
     for k in (0, 39):
         part = {n: v[k * few.num_bodies:(k + 1) * few.num_bodies] for n, v in st.items()}
         assert not state_bits_equal(o.state(), part), f"copy {k}"
+
+
+# A device with 64 KiB of LDS per block, as far as the HIP runtime tells; what
+# the kernels are launched with is recorded.
+SMALL_LDS = r"""
+#define __HIP_PLATFORM_AMD__
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+int largest = 0, refused = 0;
+static void* real(const char* name) {
+    void* hip = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
+    if (!hip) hip = dlopen("libamdhip64.so", RTLD_LAZY);
+    return dlsym(hip, name);
+}
+hipError_t hipDeviceGetAttribute(int* value, hipDeviceAttribute_t attr, int device) {
+    hipError_t e = ((hipError_t(*)(int*, hipDeviceAttribute_t, int))real("hipDeviceGetAttribute"))(value, attr, device);
+    if (attr == hipDeviceAttributeMaxSharedMemoryPerBlock) *value = 65536;
+    return e;
+}
+hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute attr, int value) {
+    if (attr == hipFuncAttributeMaxDynamicSharedMemorySize && value > 65536) {
+        ++refused;
+        return hipErrorInvalidValue;
+    }
+    return ((hipError_t(*)(const void*, hipFuncAttribute, int))real("hipFuncSetAttribute"))(f, attr, value);
+}
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t stream) {
+    if ((int)lds > largest) largest = (int)lds;
+    return ((hipError_t(*)(const void*, dim3, dim3, void**, size_t, hipStream_t))real("hipLaunchKernel"))(
+        f, grid, block, args, lds, stream);
+}
+"""
+LARGE_SCENES_ON_SMALL_LDS = r"""
+import ctypes, sys
+sys.path.insert(0, sys.argv[1] + "/tests")
+shim = ctypes.CDLL(sys.argv[2], ctypes.RTLD_GLOBAL)
+from _libs import SimWorld, scenes, state_bits_equal
+for bodies in (138, 141, 200):  # 64 KiB hold 141 records, less the block vote 139
+    w = scenes.World(name="pile")
+    scenes.drop_scene(w, 7, n_cubes=bodies // 2, n_icos=bodies - 1 - bodies // 2, grid=6)
+    g, o = SimWorld("rp", w), SimWorld("orc", w)
+    for sim in (g, o):
+        sim.step(12)
+    assert not state_bits_equal(o.state(), g.state()), bodies
+    assert g.error(0) == 0
+largest, refused = (ctypes.c_int.in_dll(shim, n).value for n in ("largest", "refused"))
+assert refused == 0 and 138 * 464 <= largest <= 65536 - 1024, (refused, largest)
+print("ok")
+"""
+
+
+def test_scenes_above_the_lds_of_a_small_device(tmp_path):
+    """On a device with 64 KiB of LDS per block, scenes whose bodies do not fit
+    are solved with the bodies in global memory, not refused."""
+    from test_gpu_adjoint import _run_with_runtime
+
+    _run_with_runtime(tmp_path, SMALL_LDS, LARGE_SCENES_ON_SMALL_LDS)
