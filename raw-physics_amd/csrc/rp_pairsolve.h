@@ -86,8 +86,11 @@ __device__ __forceinline__ double abs_mass(const HalfPos& e) { return second_lan
 // triangle inequality in the tensor's norm
 //     sqrt(w' - im) <= sqrt(w - im) + sqrt(iinv_max) |r| |a|,
 // hence w' <= im + 1.1 (w - im) + 11 iinv_max |r|^2 |a|^2. Where that bound
-// decides (with margins far above rounding), the second preparation, a fifth
-// of the contact's operations, is left out; its result would not be used.
+// decides, the second preparation, a fifth of the contact's operations, is left
+// out; its result would not be used. The margin of 1e-9 lies far above rounding
+// and above what a rotation that is no unit quaternion can change: such a
+// rotation moves w' by four times its norm's error, at most 4e-12 where the
+// bound is used at all (solve_item_pos; normalized rotations have 1e-16).
 __device__ __forceinline__ void pair_collision(V3 r_lc, V3 n, double& lambda_n, double& lambda_t, HalfPos& e, M3& I,
                                                bool& fresh, double mu_s, double h, uint32_t& err) {
     V3 r = q_rot(e.q, r_lc);
@@ -142,9 +145,9 @@ __device__ __forceinline__ void pair_collision(V3 r_lc, V3 n, double& lambda_n, 
 // lam[0..2] are the constraint's multipliers for this substep:
 //   positional: lambda; mutual orientation: lambda;
 //   hinge: aligned axes, position, limit; spherical: position, swing, twist.
-// Every constraint is up to three corrections in a row, each positional (dx
-// between the bodies' points at r: pos_dlambda, pos_apply) or angular (dq:
-// ang_dlambda, ang_apply), so one copy of that code runs in a loop: written
+// Every constraint is up to three corrections in a row, each positional (along
+// the difference d of the bodies' points at r) or angular (about d), so one copy
+// of that code runs in a loop: written
 // out per constraint type it is 130 KB of instructions, which do not fit the
 // instruction cache, and a lone wave that misses it waits for every line.
 __device__ __forceinline__ void pair_external(const ExtC& c, double* lam, HalfPos& e, double h, uint32_t& err) {
@@ -310,7 +313,7 @@ __device__ __forceinline__ void solve_item_pos(const DevWorld& w, Body* body, in
         pair_external(w.ext[~t.code], w.ext_lambda + 3 * (~t.code), e, h, err);
     } else {
         const double qq = e.q.x * e.q.x + e.q.y * e.q.y + e.q.z * e.q.z + e.q.w * e.q.w;
-        e.iinv_max = fabs(qq - 1.0) <= 1e-9 ? g.iinv_max : HUGE_VAL;
+        e.iinv_max = fabs(qq - 1.0) <= 1e-12 ? g.iinv_max : HUGE_VAL;
         HalfContact k = t.k;
         Contact* cs = w.contacts + (size_t)t.code * MAXC;
         const double mu_s = (e.mu_s + pair_other(e.mu_s)) / 2.0f;

@@ -306,3 +306,28 @@ def test_scenes_above_the_lds_of_a_small_device(tmp_path):
     from test_gpu_adjoint import _run_with_runtime
 
     _run_with_runtime(tmp_path, SMALL_LDS, LARGE_SCENES_ON_SMALL_LDS)
+
+
+@pytest.mark.parametrize("off", [1e-13, 5e-10, 1e-5])
+def test_static_friction_with_rotations_off_the_unit_sphere(off):
+    """Rotations that are no unit quaternions by less and by more than the bound
+    on the friction masses allows: the floor's, which no substep normalizes,
+    and the bodies' at the frame's start."""
+    w = scenes.World(name="off_unit")
+    cube = w.shape(scenes.cube_corners())
+    scenes._floor(w, material=(0.4, 0.2, 0.0))
+    rng = np.random.default_rng(3)
+    for k in range(7):
+        q = rng.normal(size=4)
+        w.add_body(cube, (0.9, 0.15, 0.4), (rng.uniform(-1.0, 1.0), 0.5 + 1.3 * k, rng.uniform(-1.0, 1.0)),
+                   tuple(q / np.linalg.norm(q)), mass=1.0, material=(0.4, 0.2, 0.1), linear_velocity=(2.0, 0.0, 0.5))
+    w.end_scene()
+    o, g = SimWorld("orc", w), SimWorld("rp", w)
+    for f in range(6):
+        st = o.state()
+        st["rotation"] = st["rotation"] * (1.0 + off)
+        for sim in (o, g):
+            sim.set_state(st)
+            sim.step(10, iters=2)
+        bad = state_bits_equal(o.state(), g.state())
+        assert not bad, f"{bad} differ after frame {10 * f + 10}"
