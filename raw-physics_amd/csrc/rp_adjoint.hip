@@ -59,9 +59,6 @@ __device__ __forceinline__ D1& state_comp(BodyT<D1>& e, int k) {
     case 10: return e.w.x; case 11: return e.w.y; default: return e.w.z;
     }
 }
-__device__ __forceinline__ double state_val(const Body& e, int k) {
-    return ((const double*)&e)[k];  // x, q, v, w lead the record
-}
 
 // The dynamic body against one fixed body. Only the dynamic body's side
 // carries derivatives; a fixed body has no inverse mass and no inverse

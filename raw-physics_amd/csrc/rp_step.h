@@ -717,11 +717,6 @@ template <int G> __device__ __forceinline__ int group_bcast_last(int v) {
     if constexpr (G >= 16) { int m = dpp_int<DPP_MIRROR>(v); v = (gl & 8) ? v : m; }
     return v;
 }
-template <int G> __device__ __forceinline__ double group_bcast(double v) {
-    long long b = __double_as_longlong(v);
-    int lo = group_bcast<G>((int)b), hi = group_bcast<G>((int)(b >> 32));
-    return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
-}
 // Minimum over the group's lanes (every lane gets it).
 template <int G> __device__ __forceinline__ int group_min(int v) {
     static_assert(G == 4 || G == 8 || G == 16, "lane groups of 4, 8 or 16");
@@ -730,9 +725,6 @@ template <int G> __device__ __forceinline__ int group_min(int v) {
     if constexpr (G >= 8) v = min(v, dpp_int<DPP_HALF_MIRROR>(v));
     if constexpr (G >= 16) v = min(v, dpp_int<DPP_MIRROR>(v));
     return v;
-}
-template <int G> __device__ __forceinline__ V3 group_bcast(V3 v) {
-    return v3(group_bcast<G>(v.x), group_bcast<G>(v.y), group_bcast<G>(v.z));
 }
 
 // Working memory of the first lane of a lane group (G > 1): the EPA polytope,
@@ -1029,7 +1021,6 @@ RP_HD int epa(const View& h1, const View& h2, const Simplex& s, V3& n_out, doubl
 }
 
 // ---------------------------------------------------------------------------
-// Contact manifold (clipping.cpp:7-371)// ---------------------------------------------------------------------------
 // Contact manifold (clipping.cpp:7-371)
 // ---------------------------------------------------------------------------
 struct Plane { V3 normal, point; };
@@ -1582,27 +1573,6 @@ RP_HD int collider_contacts(const HullTables& T, const ColView& c1, const ColVie
 // ---------------------------------------------------------------------------
 // XPBD base constraints (pbd_base_constraints.cpp:6-227)
 // ---------------------------------------------------------------------------
-template <class S> struct PosPrepT { V3T<S> r1, r2; M3T<S> I1, I2; };
-
-template <class S>
-RP_HD void pos_prep(const BodyT<S>& e1, const BodyT<S>& e2, V3T<S> r1_lc, V3T<S> r2_lc, PosPrepT<S>& p) {
-    p.r1 = q_rot(e1.q, r1_lc);
-    p.r2 = q_rot(e2.q, r2_lc);
-    p.I1 = world_tensor(e1.q, e1.Iinv);
-    p.I2 = world_tensor(e2.q, e2.Iinv);
-}
-template <class S>
-RP_HD S pos_dlambda(const BodyT<S>& e1, const BodyT<S>& e2, const PosPrepT<S>& p, double h, double compliance, S lambda,
-                    V3T<S> dx, uint32_t& err) {
-    S c = len(dx);
-    if (c <= 1e-50) return S(0.0);
-    V3T<S> n = v3<S>(dx.x / c, dx.y / c, dx.z / c);
-    S w1 = e1.inv_mass + dot(cross(p.r1, n), m3_mulv(p.I1, cross(p.r1, n)));
-    S w2 = e2.inv_mass + dot(cross(p.r2, n), m3_mulv(p.I2, cross(p.r2, n)));
-    if (w1 + w2 == 0.0) err |= ERR_ZERO_MASS;
-    double tc = compliance / (h * h);
-    return (-c - tc * lambda) / (w1 + w2 + tc);
-}
 template <class S>
 RP_HD void rot_update(BodyT<S>& e, V3T<S> a, bool plus) {
     Q4T<S> aq = {a.x, a.y, a.z, S(0.0)};
@@ -1613,52 +1583,6 @@ RP_HD void rot_update(BodyT<S>& e, V3T<S> a, bool plus) {
         e.q.x = e.q.x - 0.5 * qq.x; e.q.y = e.q.y - 0.5 * qq.y; e.q.z = e.q.z - 0.5 * qq.z; e.q.w = e.q.w - 0.5 * qq.w;
     }
     e.q = q_nrm(e.q);
-}
-template <class S>
-RP_HD void pos_apply(BodyT<S>& e1, BodyT<S>& e2, const PosPrepT<S>& p, S dl, V3T<S> dx) {
-    S c = len(dx);
-    if (c <= 1e-50) return;
-    V3T<S> n = v3<S>(dx.x / c, dx.y / c, dx.z / c);
-    V3T<S> imp = scl(dl, n);
-    if (!e1.fixed) e1.x = add(e1.x, scl(e1.inv_mass, imp));
-    if (!e2.fixed) e2.x = add(e2.x, scl(-e2.inv_mass, imp));
-    V3T<S> a1 = m3_mulv(p.I1, cross(p.r1, imp));
-    V3T<S> a2 = m3_mulv(p.I2, cross(p.r2, imp));
-    // quaternion products use the rotation before either body is updated
-    // (pbd_base_constraints.cpp:114-117); e1 and e2 are distinct bodies.
-    if (!e1.fixed) rot_update(e1, a1, true);
-    if (!e2.fixed) rot_update(e2, a2, false);
-}
-
-// collision_constraint_solve (pbd.cpp:107-154)
-template <class S>
-RP_HD void solve_collision(ContactT<S>& c, BodyT<S>& e1, BodyT<S>& e2, double h, uint32_t& err) {
-    PosPrepT<S> p;
-    pos_prep(e1, e2, c.r1, c.r2, p);
-    V3T<S> p1 = add(e1.x, p.r1);
-    V3T<S> p2 = add(e2.x, p.r2);
-    S d = dot(sub(p1, p2), c.n);
-    if (d > 0.0) {
-        V3T<S> dx = scl(d, c.n);
-        S dl = pos_dlambda(e1, e2, p, h, 0.0, c.lambda_n, dx, err);
-        pos_apply(e1, e2, p, dl, dx);
-        c.lambda_n += dl;
-        pos_prep(e1, e2, c.r1, c.r2, p);
-        p1 = add(e1.x, p.r1);
-        p2 = add(e2.x, p.r2);
-        dl = pos_dlambda(e1, e2, p, h, 0.0, c.lambda_t, dx, err);
-        const S mu_s = (e1.mu_s + e2.mu_s) / 2.0f;
-        S lambda_n = c.lambda_n;
-        S lambda_t = c.lambda_t + dl;
-        if (lambda_t > mu_s * lambda_n) {
-            V3T<S> p1_til = add(e1.px, q_rot(e1.pq, c.r1));
-            V3T<S> p2_til = add(e2.px, q_rot(e2.pq, c.r2));
-            V3T<S> dp = sub(sub(p1, p1_til), sub(p2, p2_til));
-            V3T<S> dp_t = sub(dp, scl(dot(dp, c.n), c.n));
-            pos_apply(e1, e2, p, dl, dp_t);
-            c.lambda_t += dl;
-        }
-    }
 }
 
 // limit_angle (pbd.cpp:175-217)
@@ -1675,39 +1599,6 @@ RP_HD bool limit_angle(V3 n, V3 n1, V3 n2, double alpha, double beta, V3& dq) {
         return true;
     }
     return false;
-}
-
-// Velocity solve of one collision constraint (pbd.cpp:646-711)
-template <class S>
-RP_HD void velocity_solve(const ContactT<S>& c, BodyT<S>& e1, BodyT<S>& e2, double h) {
-    V3T<S> n = c.n;
-    S lambda_n = c.lambda_n;
-    PosPrepT<S> p;
-    pos_prep(e1, e2, c.r1, c.r2, p);
-    V3T<S> v = sub(add(e1.v, cross(e1.w, p.r1)), add(e2.v, cross(e2.w, p.r2)));
-    S vn = dot(n, v);
-    V3T<S> vt = sub(v, scl(vn, n));
-    V3T<S> dv = v3<S>(S(0.0), S(0.0), S(0.0));
-    const S mu_d = (e1.mu_d + e2.mu_d) / 2.0f;
-    S fn = lambda_n / h;
-    S fact = RP_MIN(mu_d * fabs(fn), len(vt));
-    dv = add(dv, scl(-fact, nrm(vt)));
-    V3T<S> vtil = sub(add(e1.pv, cross(e1.pw, p.r1)), add(e2.pv, cross(e2.pw, p.r2)));
-    S vn_til = dot(n, vtil);
-    S e = e1.e * e2.e;
-    fact = -vn + RP_MIN(-e * vn_til, S(0.0));
-    dv = add(dv, scl(fact, n));
-    S w1 = e1.inv_mass + dot(cross(p.r1, n), m3_mulv(p.I1, cross(p.r1, n)));
-    S w2 = e2.inv_mass + dot(cross(p.r2, n), m3_mulv(p.I2, cross(p.r2, n)));
-    V3T<S> pimp = scl(1.0 / (w1 + w2), dv);
-    if (!e1.fixed) {
-        e1.v = add(e1.v, scl(e1.inv_mass, pimp));
-        e1.w = add(e1.w, m3_mulv(p.I1, cross(p.r1, pimp)));
-    }
-    if (!e2.fixed) {
-        e2.v = add(e2.v, inv3(scl(e2.inv_mass, pimp)));
-        e2.w = add(e2.w, inv3(m3_mulv(p.I2, cross(p.r2, pimp))));
-    }
 }
 
 // Integration of one body (pbd.cpp:537-577)
