@@ -1038,6 +1038,17 @@ static void plan_big(rp_world* w) {
     ++w->plan_gen;
 }
 
+// Live-pair slots of a record, and the first one of view k: those of the pair
+// capacity, or one per body where that is less. A recorded world has one
+// dynamic body per scene and every live pair holds one, so no scene, and no
+// view, has more live pairs than bodies.
+static int64_t record_slots(const rp_world* w) {
+    return std::max<int64_t>(1, std::min<int64_t>(w->im.pair_capacity, (int64_t)w->hw.body.size()));
+}
+static int64_t record_slot(const rp_world* w, int k) {
+    return w->im.pair_capacity <= (int64_t)w->hw.body.size() ? w->view_p0[k] : w->view[k].body_base;
+}
+
 static void sync_views(rp_world* w) {
     (void)hipStreamSynchronize(w->stream);
     for (int k = 1; k < w->nviews; ++k) (void)hipStreamSynchronize(w->view_stream[k]);
@@ -1057,7 +1068,7 @@ static hipError_t capture_part(rp_world* w, const FrameParams& fp, int k, FrameP
     v.big_classes = w->im.d.big_classes;
     v.big_rounds = std::max(least_rounds, w->im.d.big_rounds);
     Recorder rec = w->stage;
-    rec.p0 = w->view_p0[k];
+    rec.p0 = record_slot(w, k);
     hipStream_t st = w->view_stream[k];
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
@@ -1637,7 +1648,7 @@ static const size_t kAdjJacBytes = (size_t)512 << 20;
 
 static bool adjoint_prepare(rp_world* w, const FrameParams& fp, uint32_t frames, const std::vector<int32_t>& dyn) {
     const DevWorld& d = w->im.d;
-    size_t nb = (size_t)d.nb, ns = (size_t)d.ns, P = (size_t)std::max<int64_t>(1, w->im.pair_capacity);
+    size_t nb = (size_t)d.nb, ns = (size_t)d.ns, P = (size_t)record_slots(w);
     size_t per_step = nb * REC_STATE * sizeof(double) + P * (sizeof(int32_t) + MAXC * sizeof(AdjContact));
     size_t per_frame = fp.substeps * per_step + P * sizeof(int2) + 2 * ns * sizeof(int32_t);
     size_t limit = w->adj_record_bytes ? w->adj_record_bytes : kAdjRecordBytes, avail = 0, total = 0;
@@ -1705,7 +1716,7 @@ static uint32_t adjoint_record(rp_world* w, const FrameParams& fp, int k, uint32
         bool views = w->use_graphs && !w->timer.on;  // else one launch over the whole world
         for (int v = 0; e == hipSuccess && v < (views ? w->nviews : 1); ++v)
             e = launch_adjoint_pack(views ? w->view[v] : d, w->stage, w->rec, (int)f, views ? w->view_s0[v] : 0,
-                                    views ? w->view_p0[v] : 0, (int)fp.substeps, v == 0, w->stream);
+                                    views ? record_slot(w, v) : 0, (int)fp.substeps, v == 0, w->stream);
     }
     if (e != hipSuccess) {
         set_msg(std::string("adjoint: ") + hipGetErrorString(e));

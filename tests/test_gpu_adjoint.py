@@ -297,3 +297,47 @@ print("ok")
 def test_alternating_steps_and_recorded_runs_capture_once(tmp_path):
     """A loop that steps and records in turn keeps both frames' graphs."""
     _run_with_runtime(tmp_path, COUNTING_INSTANTIATE, ALTERNATING)
+
+
+@pytest.mark.parametrize("copies", [1, 66])
+def test_record_of_scenes_with_many_fixed_bodies(copies):
+    """Fixed bodies never pair with each other, so the record has a slot per
+    body and not per pair of bodies (4.5 GB a frame here for one scene), in one
+    view and in concurrent ones; bodies out of reach change no gradient."""
+    import ctypes
+
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the one the library runs on
+
+    def free_bytes():
+        n, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(n), ctypes.byref(total)) == 0
+        return n.value
+
+    def world(far):
+        w = scenes.World(name="thrown")
+        cube = w.shape(scenes.cube_corners())
+        for s in range(copies):
+            scenes._floor(w)
+            w.add_body(cube, (0.5, 0.4, 0.3), (0.0, -0.2 + 0.01 * s, 0.0), scenes.quaternion_new((0.0, 0.0, 1.0), 20.0 + s),
+                       mass=1.0, material=(0.6, 0.5, 0.0), linear_velocity=(2.0, -1.0, 0.3))
+            for k in range(far):
+                w.add_body(cube, (0.5, 0.5, 0.5), (10.0 + 2.0 * (k % 25), 20.0, 2.0 * (k // 25)),
+                           scenes.quaternion_new((0.0, 1.0, 0.0), 0.0), fixed=True)
+            w.end_scene()
+        return w
+
+    out = []
+    for far in (0, 550 if copies == 1 else 40):
+        w = world(far)
+        gw = pkg.World(w)
+        dl = np.zeros((w.num_bodies, 13))
+        dyn = 1 + (2 + far) * np.arange(copies)
+        dl[dyn] = np.random.default_rng(1).normal(size=(copies, 13))
+        before = free_bytes()
+        assert gw.adjoint_forward(20) == 0
+        gs, gp = gw.adjoint_backward(dl)
+        assert gw.adjoint_mismatches() == 0 and not gw.errors().any()
+        assert before - free_bytes() < 2 << 30
+        out.append((gs[dyn], gp[dyn], gw.state()["position"][dyn]))
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    assert np.abs(out[0][1]).max() > 0.0  # (friction and mass matter: it has landed)
