@@ -255,7 +255,10 @@ uint32_t rp_world_num_scenes(const rp_world* w);
  * Returns 0 or RP_ERR_RUNTIME. Blocks until the GPU is done. */
 uint32_t rp_world_step(rp_world* w, double dt, uint32_t frames, uint32_t num_substeps, uint32_t num_pos_iters,
                        int32_t enable_collisions, double gravity);
-/* Same, without waiting for completion (call rp_world_synchronize). */
+/* Same, without waiting for completion (call rp_world_synchronize). The queue
+ * is bounded: a call waits for earlier frames where more than 64 of its own, or
+ * 8 of a world with a large scene, would be in flight; with a large scene the
+ * first frame after a set state also waits until its solve order is known. */
 uint32_t rp_world_step_async(rp_world* w, double dt, uint32_t frames, uint32_t num_substeps, uint32_t num_pos_iters,
                              int32_t enable_collisions, double gravity);
 uint32_t rp_world_synchronize(rp_world* w);
@@ -383,15 +386,17 @@ int32_t rp_world_lds_limit(const rp_world* w);
 int32_t rp_world_set_views(rp_world* w, int32_t views);
 int32_t rp_world_views(const rp_world* w);
 
-/* Solve schedule: lanes serving one scene in the solve kernel (64, 32 or 16,
- * i.e. 1, 2 or 4 scenes per wave). Identical results. Returns 0 or -1. */
+/* Solve schedule: lanes serving one scene in the solve kernel: 32 or 16 (2 or
+ * 4 scenes per wave), or 64: whole waves, one per scene, or two or four per
+ * sweep where joints or scenes above 64 bodies gain by them and the world has
+ * few enough scenes. Identical results. Returns 0 or -1. */
 int32_t rp_world_set_solve_lanes(rp_world* w, int32_t lanes_per_scene);
 
 /* Large scenes (coloured solve): the first `classes` colour classes are
  * solved one launch each over the whole device, the remaining colours and
  * the serial class by one block with a barrier between classes (0..64; the
- * default is chosen from the class sizes of earlier frames). Items of one
- * colour are independent, so results are identical. Returns 0 or -1. */
+ * default is chosen from the class sizes of the frame or of those just before
+ * it). Items of one colour are independent, so results are identical. Returns 0 or -1. */
 int32_t rp_world_set_colour_launches(rp_world* w, int32_t classes);
 int32_t rp_world_solve_lanes(const rp_world* w);
 

@@ -303,8 +303,8 @@ class World:
 
     def set_colour_launches(self, classes: int):
         """Large scenes: colour classes solved one launch each before the
-        one-block tail (0..64; the default follows earlier frames' class
-        sizes; identical results)."""
+        one-block tail (0..64; the default follows the class sizes of the
+        frame or of those just before it; identical results)."""
         if self.lib.rp_world_set_colour_launches(self.h, classes) != 0:
             raise ValueError(f"colour launches must be 0..64, not {classes}")
 

@@ -403,9 +403,9 @@ __device__ __forceinline__ int pair_manifold(const DevWorld& w, int g, const Hul
 
 // kManifold: the contact manifold of a converged pair is built here too, on
 // the same staged hulls, and its contacts written (no manifold queue).
-// list / count: visit the pairs of a size-class list (LDS slices of `stage`
-// vertices per pair), or (list null) every live pair with slices of
-// stage_cap vertices.
+// list / count: visit the pairs of a size-class list, or (list null) every live
+// pair. LDS slices of `stage` vertices per pair: both hulls and what EPA and
+// clipping use beside them (stage_slice).
 template <int G, bool kManifold>
 __device__ __forceinline__ void gjk_epa_pairs(DevWorld& w, const int32_t* list, const int32_t* count, int stage) {
     extern __shared__ V3 rp_stage[];
@@ -701,10 +701,10 @@ static_assert(sizeof(Body) % sizeof(int4) == 0 && offsetof(Body, deact) % sizeof
 // of its own: they follow the position sweep P levels behind instead of waiting
 // for its end. Against one sweep after another on one wave (64 lanes) or four:
 // 10 frames of 500 chains of 6 links (4 iterations) 80.5 -> 65.3 ms, 4 frames
-// of 150 scenes of 4 to 256 bodies with chains 25.3 -> 23.1. Scenes of up to 64
-// bodies without joints keep one sweep after another on one wave: their floor
-// is in a pair with every body at level 0, so P is about their whole depth, and
-// the steps' bookkeeping cost 0.5 to 2 %.
+// of 150 scenes of 4 to 256 bodies with chains 25.3 -> 23.1. Scenes without
+// joints on one wave or less keep one sweep after another: their floor is in a
+// pair with every body at level 0, so P is about their whole depth, and the
+// steps' bookkeeping cost scenes of up to 64 bodies 0.5 to 2 %.
 template <bool kExt, int LPS, bool kLds>
 __global__ void __launch_bounds__(LPS > 64 ? 2 * LPS : 64) __attribute__((amdgpu_waves_per_eu(2)))
 k_solve(DevWorld w, double h, int iters, int collisions, int integrate_next, int cap) {
