@@ -218,9 +218,10 @@ def committed_traffic(kernel_class: str, schedule: dict):
 
 def adjoint_run(pkg, sc, n_scenes: int, frames: int, check_scenes: int = 256):
     """Differentiable workload: n_scenes cubes thrown onto tilted static boxes,
-    `frames` frames; the checkpointed forward pass, then the backward pass of
+    `frames` frames; the recorded forward pass, then the backward pass of
     L = sum |x_final - target|^2. Adjoint steps/s = scenes x frames x
-    substeps reversed per second of the backward pass (recomputation included)."""
+    substeps reversed per second of the backward pass (its re-evaluation of
+    every substep included)."""
     world, targets = sc.ramps(n_scenes)
     gw = pkg.World(world)
     init = gw.state()
@@ -681,7 +682,7 @@ def main():
             # peak, the same for its vector and matrix units; the kernel's FP64
             # work is VALU (no matrix-shaped work in the step)
             roofline = {"bound": "mfma", "bound_detail": "FP64 compute roof (78.6 TFLOP/s, vector = matrix "
-                        "peak); the kernel issues FP64 VALU, no MFMA; HBM under 8 % of 8 TB/s",
+                        "peak); the kernel issues FP64 VALU, no MFMA; HBM 9 % of 8 TB/s",
                         "kernel": names[dom],
                         "achieved": k["tflops"], "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                         "frac": k["tflops"] / FP64_PEAK_TFLOPS if k["tflops"] else None,
